@@ -395,9 +395,18 @@ __global__ __launch_bounds__(BS) void k_element(ElemArgs a) {
       a.evec[(size_t)e * LD + p] = f;
     }
   } else {
-    for (int k = threadIdx.x; k < EPB * NPE * NPE; k += BS) {
-      const int le = k / (NPE * NPE), rem = k % (NPE * NPE), p = rem / NPE, q = rem % NPE, e = e0 + le;
+    // The block of (q, p) is that of (p, q) transposed, and the elasticity
+    // matrix symmetric: one lane per pair p <= q writes both, so the blocks
+    // are symmetric to the bit (which the half storage of the assembled
+    // matrix needs) and the FP64 work, what bounds this kernel, halves.
+    constexpr int NPAIR = NPE * (NPE + 1) / 2;
+    for (int k = threadIdx.x; k < EPB * NPAIR; k += BS) {
+      const int le = k / NPAIR, rem = k % NPAIR, e = e0 + le;
       if (e >= a.nelem) continue;
+      int q = (int)((sqrtf(8.0f * rem + 1.0f) - 1.0f) * 0.5f);  // rem = q (q + 1) / 2 + p
+      if ((q + 1) * (q + 2) / 2 <= rem) ++q;
+      if (q * (q + 1) / 2 > rem) --q;
+      const int p = rem - q * (q + 1) / 2;
       double A[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
       for (int gp = 0; gp < NGP; gp++) {
         const double s = Wg[le][gp];
@@ -424,7 +433,11 @@ __global__ __launch_bounds__(BS) void k_element(ElemArgs a) {
 #pragma unroll
       for (int i = 0; i < 3; i++)
 #pragma unroll
-        for (int j = 0; j < 3; j++) out[(3 * p + i) * LD + 3 * q + j] = A[i][j];
+        for (int j = 0; j < 3; j++) {
+          const double v = p == q && j < i ? A[j][i] : A[i][j];
+          out[(3 * p + i) * LD + 3 * q + j] = v;
+          if (p != q) out[(3 * q + j) * LD + 3 * p + i] = v;
+        }
     }
     for (int k = threadIdx.x; k < EPB * LD; k += BS) {
       const int le = k / LD, i = k % LD, e = e0 + le;

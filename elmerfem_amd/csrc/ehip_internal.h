@@ -77,6 +77,29 @@ using KState32 = KStateT<float>;
 
 struct ehip_system_impl;
 
+// Half storage of a symmetric stencil matrix (spmv_sym_body).  The pattern's
+// offsets are one symmetric list for the whole matrix, k = 0 .. K - 1
+// ascending, entry `diag` being 0; the values of the offsets >= 0 lie one
+// array after another.  Entry k of row r = D node + a takes its D values
+// from val[k] + (k < diag ? D D node + a + D d : D r + d), d < D, and its x
+// from column D (node + col[k]) + d.
+constexpr int kSymMax = 31;
+struct SymTab {
+  int K, diag;
+  int val[kSymMax + 1];
+  int col[kSymMax + 1];
+};
+// One precision's values in that layout, of the values version `ver`:
+// good = that version is symmetric (else the copy is not used).
+// zero: per slice, the rows whose off-diagonal entries are all zero.
+template <typename T>
+struct SymCopy {
+  T *v = nullptr;
+  unsigned long long *zero = nullptr;
+  uint64_t ver = 0;
+  bool good = false;
+};
+
 }  // namespace ehip
 
 struct ehip_system {
@@ -153,6 +176,18 @@ struct ehip_system {
   double *sho64 = nullptr;
   float *sho32 = nullptr;
   uint64_t sho64_ver = 0, sho32_ver = 0;
+  // half storage for symmetric values of such a pattern (CG solves of
+  // systems over kSymMinBytes): the offsets, every row's present entries as
+  // a 32-bit mask, and the same as one 64-bit lane mask per (slice, entry)
+  bool sym_ok = false;
+  bool sym_on = false;                // the solve in progress may use it
+  ehip::SymTab sym_tab{};
+  int64_t sym_len = 0;                // values of a copy, padding included
+  unsigned *sym_mask = nullptr;       // n
+  unsigned long long *sym_pm = nullptr; // nslice * K
+  int *sym_flag = nullptr;            // set by a fill that met unequal values
+  ehip::SymCopy<double> sym64;
+  ehip::SymCopy<float> sym32;
   // workspace of the multi-system engine, kept across admissions (a
   // hipFree per retired request would synchronise the whole device)
   double *bw64 = nullptr;
@@ -260,6 +295,11 @@ const double *sell_values64(ehip_system *s);
 const float *sell_values32(ehip_system *s);
 const double *sho_values64(ehip_system *s);
 const float *sho_values32(ehip_system *s);
+// half-storage copies of the current values, or null when the system has no
+// such layout, the solve in progress does not ask for it, or the values are
+// not symmetric (a refresh waits for the stream)
+const double *sym_values64(ehip_system *s);
+const float *sym_values32(ehip_system *s);
 
 // SELL-64 launch shape: nonzeros per lane in flight (kSellU, or 9 when that
 // wastes fewer loads on the pattern's slice widths), and the grid (slice
@@ -298,6 +338,11 @@ inline int sho_nt_from(int nslice, int64_t bytes, int64_t n, int elem) {
   if (c >= bytes) return nslice;
   return (int)((double)nslice * (double)c / (double)bytes);
 }
+
+// Smallest FP64 values copy (bytes) that takes the half storage: below it
+// the SpMV is bound by launches, not by the matrix stream, and the check of
+// the values costs more than it gives.
+constexpr int64_t kSymMinBytes = 16ll << 20;
 
 inline int sell_grid(const ehip_system *s) {
   int g = (s->nslice + 3) / 4;

@@ -1357,7 +1357,8 @@ static void launch_epi_sellb(ehip_system *s, const T *sv, const T *xin, const Ep
 // kernels measured slower that way and keep sell_grid.
 template <typename T>
 static int epi_sell_grid(const ehip_system *s) {
-  return sizeof(T) == 4 && !s->sellb_d ? std::min(sell_grid(s), 1024) : sell_grid(s);
+  if (sizeof(T) != 4 || s->sellb_d) return sell_grid(s);
+  return std::min(sell_grid(s), s->sym_ok && s->sym_on ? 2048 : 1024);
 }
 
 template <int U, class Epi>
@@ -1403,6 +1404,41 @@ static void launch_epi_sho(ehip_system *s, const T *sv, const T *xin, const Epi 
   else launch_epi_sho_as<T, U, D, false>(s, sv, xin, e, st);
 }
 
+// Epilogues that run on the half storage too: those of the CG loops
+// (ehip_system::sym_on is set for these solves only).
+template <class Epi>
+struct EpiOnSym : std::false_type {};
+template <typename T> struct EpiOnSym<EpiInit<T>> : std::true_type {};
+template <typename T> struct EpiOnSym<EpiTrue<T>> : std::true_type {};
+template <typename T> struct EpiOnSym<EpiCgQ<T>> : std::true_type {};
+template <typename T> struct EpiOnSym<EpiCgResidual<T>> : std::true_type {};
+template <typename T> struct EpiOnSym<EpiCgFast1<T>> : std::true_type {};
+template <typename T> struct EpiOnSym<EpiCgFold<T>> : std::true_type {};
+template <> struct EpiOnSym<EpiRU> : std::true_type {};
+template <> struct EpiOnSym<EpiResid> : std::true_type {};
+
+template <typename T, int BS, int U, int D, class Epi>
+__global__ __launch_bounds__(BS) void k_spmv_epi_sym(int n, SymTab tab, const unsigned long long *__restrict__ pm,
+                                                     const unsigned long long *__restrict__ zero,
+                                                     const T *__restrict__ vals, const T *__restrict__ xin, int nslice,
+                                                     Epi epi, const KStateT<T> *st) {
+  if (st && solve_done(st)) return;
+  spmv_sym_body<T, T, BS, U, D>(n, tab, pm, zero, vals, xin, nslice, epi);
+}
+
+template <typename T, int D, class Epi>
+static void launch_epi_sym(ehip_system *s, const T *sv, const T *xin, const Epi &e, const KStateT<T> *st) {
+  const int g = epi_sell_grid<T>(s);
+  const unsigned long long *zero;
+  if constexpr (sizeof(T) == 4) zero = s->sym32.zero; else zero = s->sym64.zero;
+  if (s->prof_start)
+    hipExtLaunchKernelGGL((k_spmv_epi_sym<T, 256, 9, D, Epi>), dim3(g), dim3(256), 0, s->stream, s->prof_start,
+                          s->prof_stop, 0, s->n, s->sym_tab, s->sym_pm, zero, sv, xin, s->nslice, e, st);
+  else
+    launch_k((k_spmv_epi_sym<T, 256, 9, D, Epi>), dim3(g), dim3(256), s->stream, s->n, s->sym_tab, s->sym_pm, zero, sv,
+             xin, s->nslice, e, st);
+}
+
 // the active format of one precision: 0 CSR stream, 1 SELL-64, 2 SELL-64
 // with slice-shared offsets
 template <typename T>
@@ -1433,6 +1469,14 @@ static void launch_epi(ehip_system *s, const SpmvPlan &p, const T *vals, const T
   };
   if (active_fmt<T>(s) == 2) {
     const T *sv;
+    if constexpr (EpiOnSym<Epi>::value) {
+      if constexpr (F32) sv = sym_values32(s); else sv = sym_values64(s);
+      if (sv) {
+        if (s->sho_d == 3) launch_epi_sym<T, 3>(s, sv, xin, e, st);
+        else launch_epi_sym<T, 1>(s, sv, xin, e, st);
+        return;
+      }
+    }
     if constexpr (F32) sv = sho_values32(s); else sv = sho_values64(s);
     if (missing(sv)) return;
     if (s->sho_d == 3) launch_epi_sho<T, 9, 3>(s, sv, xin, e, st);
@@ -1780,6 +1824,7 @@ static void cg32_iterations(ehip_system *s, const Vecs<float> &v, int count, boo
 static uint64_t cg32_key(const ehip_system *s) {
   const uint64_t parts[] = {(uint64_t)(uintptr_t)s->work32, (uint64_t)(uintptr_t)s->vals32,
                             (uint64_t)(uintptr_t)s->sell32, (uint64_t)(uintptr_t)s->sho32,
+                            s->sym32.good ? (uint64_t)(uintptr_t)s->sym32.v : 0,
                             (uint64_t)(uintptr_t)s->partials32,
                             (uint64_t)(uintptr_t)s->st32, (uint64_t)(uintptr_t)s->plan32.chunk_row,
                             (uint64_t)s->fmt32, (uint64_t)s->plan32.block, (uint64_t)s->plan32.nb,
@@ -1875,7 +1920,7 @@ static int mixed_cg_ru(ehip_system *s, SolveCtx &c, double delta, int *inner_tot
   int batch = std::min(cap, 8);
   // the SELL copy of the FP32 values is refreshed here, outside any recording
   if (active_fmt<float>(s) == 1 && !sell_values32(s)) return EHIP_ENOMEM;
-  if (active_fmt<float>(s) == 2 && !sho_values32(s)) return EHIP_ENOMEM;
+  if (active_fmt<float>(s) == 2 && !sym_values32(s) && !sho_values32(s)) return EHIP_ENOMEM;
   while (!s->h_st->done) {
     if (c.prof || !graphs_enabled()) {
       cg32_iterations(s, v, batch, c.prof);  // sampled launches need their own events
@@ -2293,6 +2338,12 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   const int n = s->n;
   int rc;
   if ((rc = ensure_state(s))) return rc;
+  // half storage only where the method needs a symmetric matrix anyway
+  // ... of 3-DOF node blocks only in FP64: an entry below the diagonal takes
+  // its three values from three places there, and FP32 lost by it what the
+  // halved stream gave (63^3 Hex8: 37 us full, 42 us half; FP64 112 and 84)
+  s->sym_on = p->method == EHIP_CG && p->precond < EHIP_PRECOND_ILU0 &&
+              (s->sho_d == 1 || p->precision == EHIP_FP64);
   SolveClock clk(events, s->stream);
   EHIP_HIP_TRY(clk.create());
   ehip_report rep{};

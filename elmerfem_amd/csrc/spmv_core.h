@@ -16,6 +16,7 @@
 #pragma once
 #include <type_traits>
 #include <utility>
+#include "ehip_internal.h"
 #include "reduce.h"
 
 namespace ehip {
@@ -537,6 +538,86 @@ __device__ __forceinline__ void spmv_sho_body(int n, const int *__restrict__ off
     walk(std::true_type{}, nt_from, nslice);
   } else {
     walk(std::false_type{}, 0, nslice);
+  }
+  if constexpr (NV > 0) block_publish<A, NV>(acc, epi.partials, epi.stride);
+}
+
+// Half storage for symmetric values on a slice-shared-offset pattern whose
+// offsets are one symmetric list: only the values of offsets >= 0 are kept,
+// one array per offset, and the entry at offset -o of row r is row r - o's
+// value at offset +o.  A value is then read twice, by two rows o apart; o is
+// at most the bandwidth, and the workgroups of one XCD walk one contiguous
+// row range together, so the second read is served by that XCD's L2 and the
+// stream from the Infinity Cache or HBM halves.  What binds the SpMV here is
+// that stream (the caches deliver the second read and the x gathers several
+// times faster), so the loads are all cached, never non-temporal.
+// Entries are added in ascending offset order, the CRS order: FP64 adds only
+// the row's own entries (bit `lane` of pm[slice * K + k]), so its sums are
+// those of the other layouts to the bit; FP32 adds absent entries as +0.
+// A row whose off-diagonal entries are all zero (a Dirichlet row of a matrix
+// whose columns were not eliminated) is not symmetric to its neighbours;
+// zero[slice] names such rows and their products take +0, the value stored.
+template <typename V, typename A, int BS, int U, int D, class Epi>
+__device__ __forceinline__ void spmv_sym_body(int n, const SymTab &tab, const unsigned long long *__restrict__ pm,
+                                              const unsigned long long *__restrict__ zero,
+                                              const V *__restrict__ vals, const A *__restrict__ x, int nslice,
+                                              Epi &epi) {
+  constexpr int WPB = BS / 64;
+  constexpr bool kF32 = sizeof(V) == 4;
+  constexpr int NV = Epi::NV;
+  constexpr int NA = NV > 0 ? NV : 1;
+  A acc[NA];
+#pragma unroll
+  for (int k = 0; k < NA; ++k) acc[k] = (A)0;
+  epi.init();
+  if (epi_skipped(epi)) return;
+  const int lane = (int)threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int K = tab.K, diag = tab.diag;
+  const XcdWalk w((nslice + WPB - 1) / WPB);
+  for (int gidx = w.first; gidx < w.last; gidx += w.step) {
+    const int sl = gidx * WPB + wv;  // wave-uniform
+    if (sl >= nslice) continue;
+    const int r = sl * 64 + lane;  // >= n: a padding lane, its values are 0
+    const typename Epi::Pre pre = epi.load(min(r, n - 1));
+    const bool z = (zero[sl] >> lane) & 1ull;
+    const unsigned long long *__restrict__ m = pm + (int64_t)sl * K;
+    const int node = r / D;
+    const int up = D * r, low = D * D * node + (r - D * node);
+    A sum = (A)0;
+    for (int k0 = 0; k0 < K; k0 += U) {
+      V vv[U][D];
+      int cc[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int kk = min(k0 + u, K - 1);  // clamped into the list
+        const bool lower = kk < diag;
+        const int at = lower ? low : up, step = lower ? D : 1;
+        const V *__restrict__ v = vals + tab.val[kk];
+        cc[u] = min(max(D * (node + tab.col[kk]), 0), n - D);
+#pragma unroll
+        for (int d = 0; d < D; ++d) vv[u][d] = v[at + step * d];
+      }
+      A xv[U][D];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int d = 0; d < D; ++d) xv[u][d] = x[cc[u] + d];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u;
+        const bool on = k < K && (kF32 || ((m[min(k, K - 1)] >> lane) & 1ull));
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+#pragma clang fp contract(off)
+          const bool own = D == 1 ? k == diag : D * (node + tab.col[min(k, K - 1)]) + d == r;
+          const A vk = z && !own ? (A)0 : (A)vv[u][d];
+          const A tv = sum + vk * xv[u][d];
+          sum = on ? tv : sum;
+        }
+      }
+    }
+    if (r < n) epi.row(r, sum, pre, acc);
   }
   if constexpr (NV > 0) block_publish<A, NV>(acc, epi.partials, epi.stride);
 }
