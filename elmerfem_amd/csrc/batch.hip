@@ -1706,6 +1706,7 @@ static void lane_stop(ehip_batch *b) {
 }
 
 static void lane_worker(Lane *L) {
+  tl_shared_device = true;
   for (;;) {
     ehip_system *s = nullptr;
     {

@@ -4,6 +4,7 @@
 
 #include <cstdint>
 #include <cstdlib>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -196,6 +197,13 @@ struct ehip_system {
   size_t bw32_n = 0;
   int fmt64 = 0, fmt32 = 0;           // SpMV format per precision: 0 CSR stream, 1 SELL-64,
                                       // 2 SELL-64 with shared offsets
+  // largest distance of a column from its row, per layout (-1: no layout),
+  // and the buffers of the resident Krylov loops (resident.hip)
+  int sho_halo = -1, sell_halo = -1;
+  int sho_wmax = 0;                   // entries of the longest offset list
+  bool resident_on = false;           // the solve in progress may use them
+  void *res_buf = nullptr;
+  size_t res_bytes = 0;
   uint64_t vals_ver = 1, vals32_ver = 1, sell64_ver = 0, sell32_ver = 0;
   double *vals = nullptr, *rhs = nullptr, *x = nullptr;
   float *vals32 = nullptr;
@@ -400,6 +408,19 @@ void ilu_release(ehip_system *s);
 // ehip_solve's body.  events = false times the solve with host clock
 // readings instead of HIP events (for callers that create no runtime objects).
 int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, double *hist, bool events);
+
+// Resident Krylov sequences (resident.hip): whether the system and the LDS allow
+// one; its launches (the state's ticket[3] tells a grid that gave up, with
+// nothing changed); and the lock to hold from there until the state is read.
+template <typename T>
+struct Vecs;
+template <typename T>
+bool resident_fits(ehip_system *s, bool faithful);
+template <typename T>
+int resident_cg(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du);
+template <typename T>
+int resident_bicgstab(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du);
+std::mutex &resident_lock(const ehip_system *s);
 
 // SpMV launch sampling (ehip_params.profile_every)
 void prof_begin(ehip_system *s);

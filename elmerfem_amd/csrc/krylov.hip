@@ -26,6 +26,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "cg_steps.h"
 #include "ehip_internal.h"
 #include "launch.h"
 #include "linalg_kernels.h"
@@ -35,6 +36,7 @@ namespace ehip {
 
 thread_local GraphRec *tl_graph_rec = nullptr;
 thread_local hipError_t tl_launch_err = hipSuccess;
+thread_local bool tl_shared_device = false;
 
 // Whether the mixed form's FP32 CG runs its folded two-launch steps
 // (EHIP_CG_FOLD=0 turns them off: three launches per iteration).  Read at
@@ -316,33 +318,6 @@ namespace ehip {
 
 // ================================================================ Krylov kernels
 
-template <typename T>
-__device__ __forceinline__ bool solve_done(const KStateT<T> *st) {
-  // `done` only changes at the end of an earlier launch, so a plain load is
-  // coherent here; it is uniform, so it becomes one scalar load per wave
-  // instead of a same-address L2 request from every lane
-  return __builtin_amdgcn_readfirstlane(st->done) != 0;
-}
-
-// The unscaled relative residual ||b - A x|| / ||b|| from the sum of squares
-// of r_s / D on the scaled system (r_s = D0 (b - A x) / beta and D = D0 beta,
-// so r_s / D = (b - A x) / beta^2, and likewise b_s / D = b / beta^2).
-// Records it and tells whether it meets tol_u; true when the test is off.
-template <typename T>
-__device__ __forceinline__ bool unscaled_ok(KStateT<T> *st, T sum_u) {
-  if (!(st->tol_u > (T)0)) return true;
-  const T ru = sqrt(sum_u / st->bb_u);
-  st->res_u = ru;
-  return ru < st->tol_u;
-}
-
-#define EHIP_EPI_MEMBERS(T) \
-  Vecs<T> v;                \
-  KStateT<T> *st;           \
-  T *partials;              \
-  int stride;               \
-  unsigned *ticket;
-
 // r = b - A x ; z = r/dg ; partials r.z, r.r, b.b  (start of every solve)
 template <typename T>
 struct EpiInit {
@@ -493,51 +468,6 @@ __global__ __launch_bounds__(kVecBlock) void k_cg_fast2(int n, Vecs<T> v, KState
   }
   cg_vector_step<T, 2, Fold>(n, v, st, pq_part, pq_g, partials);
 }
-
-// The stopping tests on the recurrence residual after a CG vector step, in
-// the order HUTI applies them: converged, diverged, rho = 0, out of
-// iterations, and (mixed form) a reliable update due.
-struct CgCheck {
-  int done, info, rec_conv;
-};
-template <typename T>
-__device__ __forceinline__ CgCheck cg_check(T res, T rz, int it, const KStateT<T> *st) {
-  if (res < st->tol) return {1, 0, 1};
-  if (!(res == res) || (st->divtol > (T)0 && res > st->divtol)) return {1, 3, 0};
-  if (rz == (T)0) return {1, 20, 0};
-  if (it >= st->maxit) return {1, 2, 0};
-  if (res < st->ru) return {1, 0, 2};  // reliable update due
-  return {0, 0, 0};
-}
-template <typename T>
-__device__ __forceinline__ void cg_apply(const CgCheck &c, KStateT<T> *st) {
-  if (c.rec_conv) st->rec_conv = c.rec_conv;
-  if (c.info) st->info = c.info;
-  if (c.done) st->done = 1;
-}
-
-template <typename T>
-struct FinCgFast2 {
-  static constexpr int NV = 2;
-  KStateT<T> *st;
-  T *partials;
-  int stride;
-  double *hist;
-  __device__ void finish(T (&tot)[2]) {
-    if (threadIdx.x != 0) return;
-    const T rho_old = st->rho;
-    st->rho_new = rho_old;  // kept for a residual replacement, which recomputes beta
-    st->rho = tot[0];
-    st->beta = tot[0] / rho_old;
-    st->rr = tot[1];
-    const T res = sqrt(tot[1]) / st->rhsnorm;
-    st->res = res;
-    const int it = st->iter + 1;  // iterations done
-    st->iter = it;
-    if (hist && it - 1 < st->maxit) hist[it - 1] = (double)res;
-    cg_apply(cg_check(res, tot[0], it, st), st);
-  }
-};
 
 // ---- folded FP32 CG steps (the inner sequence of the mixed form): two
 // launches per iteration instead of three.  The SpMV step opens by summing
@@ -735,55 +665,6 @@ __global__ __launch_bounds__(kVecBlock) void k_cg_da(int n, Vecs<T> v, KStateT<T
   cg_vector_step<T, 1>(n, v, st, pq_part, pq_g, partials);
 }
 
-template <typename T>
-struct EpiCgResidual {
-  static constexpr int NV = 2;
-  EHIP_EPI_MEMBERS(T)
-  double *hist;
-  const T *rn_part;  // Kda's partials of rho_new = r.z
-  int rn_g;
-  T beta;
-  const T *du;  // the scaling's D, or null when the unscaled test is off
-  // rho_new summed from Kda's partials by every workgroup in the same order
-  // (workgroup 0 records it for the finalize), in place of a finalize launch
-  __device__ void init() {
-    T rn[1];
-    block_reduce_all<T, 1>(rn_part, 0, rn_g, rn);
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->rho_new = rn[0];
-    beta = rn[0] / st->rho;
-  }
-  struct Pre { T b, z, p, d; };
-  __device__ Pre load(int i) const { return Pre{v.b[i], v.z[i], v.p[i], du ? du[i] : (T)1}; }
-  __device__ void row(int i, T s, const Pre &pr, T (&acc)[2]) {
-    const T ti = s - pr.b;
-    acc[0] += ti * ti;
-    const T ui = ti / pr.d;
-    acc[1] += ui * ui;
-    v.p[i] = pr.z + beta * pr.p;
-  }
-  __device__ void finish(T (&tot)[2]) {
-    if (threadIdx.x != 0) return;
-    const T res = sqrt(tot[0]) / st->rhsnorm;
-    st->res = res;
-    const int it = st->iter;  // HUTI iter_count, 1-based
-    if (hist && it - 1 < st->maxit) hist[it - 1] = (double)res;
-    if (res < st->tol && unscaled_ok(st, tot[1])) {
-      st->info = 1;
-      st->done = 1;
-      return;
-    }
-    st->rho = st->rho_new;
-    st->iter = it + 1;
-    if (it + 1 > st->maxit) {
-      st->info = 2;
-      st->done = 1;
-    } else if (st->rho_new == (T)0) {
-      st->info = 20;
-      st->done = 1;
-    }
-  }
-};
-
 // ---- BiCGStab in huti_bicgstab.src order; per iteration k:
 //   B3 : v = A t1v ; alpha = rho / (rtld.v)
 //   B45: s = r - alpha v ; t2v = s/dg ; ||s|| (s-norm exit below HUTI_EPSILON)
@@ -807,36 +688,32 @@ struct EpiBiV {
   }
 };
 
+// Calls f(i) for this thread's rows of a vector kernel whose workgroups take
+// tiles of kVI * kVecBlock consecutive rows (as CgTile: the sums' grouping
+// that the resident loop of resident.hip repeats).
+template <class F>
+__device__ __forceinline__ void for_tiles(int n, F f) {
+  for (int base = blockIdx.x * kVecBlock * kVI; base < n; base += gridDim.x * kVecBlock * kVI)
+#pragma unroll
+    for (int k = 0; k < kVI; ++k) {
+      const int i = base + k * kVecBlock + (int)threadIdx.x;
+      if (i < n) f(i);
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(kVecBlock) void k_bi_s(int n, Vecs<T> v, KStateT<T> *st, T *partials) {
   if (solve_done(st)) return;
   const T alpha = st->alpha;
   T acc[1] = {(T)0};
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+  for_tiles(n, [&](int i) {
     const T si = v.r[i] - alpha * v.v[i];
     v.sv[i] = si;
     v.t2v[i] = si / v.dg[i];
     acc[0] += si * si;
-  }
+  });
   block_publish<T, 1>(acc, partials, gridDim.x);
 }
-
-template <typename T>
-struct FinSnorm {
-  static constexpr int NV = 1;
-  KStateT<T> *st;
-  T *partials;
-  int stride;
-  __device__ void finish(T (&tot)[1]) {
-    if (threadIdx.x != 0) return;
-    const T sn = sqrt(tot[0]);
-    st->snorm = sn;
-    if (sn < (T)1.17549435E-38f) {  // HUTI_EPSILON (huti_fdefs.h)
-      st->snorm_exit = 1;
-      st->info = 36;
-    }
-  }
-};
 
 template <typename T>
 struct EpiBiT {
@@ -879,116 +756,17 @@ __global__ __launch_bounds__(kVecBlock) void k_bi_xr(int n, Vecs<T> v, KStateT<T
   if (solve_done(st)) return;
   const T alpha = st->alpha, omega = st->omega;
   T acc[2] = {(T)0, (T)0};
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+  for_tiles(n, [&](int i) {
     v.x[i] = v.x[i] + alpha * v.t1v[i] + omega * v.t2v[i];
     const T ri = v.sv[i] - omega * v.t[i];
     v.r[i] = ri;
     acc[0] += v.rtld[i] * ri;
     acc[1] += ri * ri;
-  }
+  });
   (void)fast;
   (void)hist;
   block_publish<T, 2>(acc, partials, gridDim.x);
 }
-
-template <typename T>
-struct FinBiXr {
-  static constexpr int NV = 2;
-  KStateT<T> *st;
-  T *partials;
-  int stride;
-  int fast;
-  double *hist;
-  __device__ void finish(T (&tot)[2]) {
-    if (threadIdx.x != 0) return;
-    const T alpha = st->alpha, omega = st->omega;
-    st->rho_new = tot[0];
-    st->rr = tot[1];
-    if (fast) {
-      const T res = sqrt(tot[1]) / st->rhsnorm;
-      st->res = res;
-      const int it = st->iter;
-      if (hist && it - 1 < st->maxit) hist[it - 1] = (double)res;
-      if (res < st->tol) {
-        st->rec_conv = 1;
-        st->done = 1;
-        return;
-      }
-      if (!(res == res) || (st->divtol > (T)0 && res > st->divtol)) {
-        st->info = 3;
-        st->done = 1;
-        return;
-      }
-      if (omega == (T)0) {
-        st->info = 37;
-        st->done = 1;
-        return;
-      }
-      st->iter = it + 1;
-      if (it + 1 > st->maxit) {
-        st->info = 2;
-        st->done = 1;
-      } else if (tot[0] == (T)0) {
-        st->info = 35;
-        st->done = 1;
-      } else {
-        st->beta = (tot[0] * alpha) / (st->rho * omega);
-        st->rho = tot[0];
-      }
-    }
-  }
-};
-
-template <typename T>
-struct EpiBiResidual {
-  static constexpr int NV = 2;
-  EHIP_EPI_MEMBERS(T)
-  double *hist;
-  T beta, omega;
-  const T *du;  // the scaling's D, or null when the unscaled test is off
-  __device__ void init() {
-    omega = st->omega;
-    beta = (st->rho_new * st->alpha) / (st->rho * omega);
-  }
-  struct Pre { T b, r, p, v, dg, d; };
-  __device__ Pre load(int i) const { return Pre{v.b[i], v.r[i], v.p[i], v.v[i], v.dg[i], du ? du[i] : (T)1}; }
-  __device__ void row(int i, T s, const Pre &pr, T (&acc)[2]) {
-    const T ti = s - pr.b;
-    acc[0] += ti * ti;
-    const T ui = ti / pr.d;
-    acc[1] += ui * ui;
-    const T pi = pr.r + beta * (pr.p - omega * pr.v);
-    v.p[i] = pi;
-    v.t1v[i] = pi / pr.dg;
-  }
-  __device__ void finish(T (&tot)[2]) {
-    if (threadIdx.x != 0) return;
-    const T res = sqrt(tot[0]) / st->rhsnorm;
-    st->res = res;
-    const int it = st->iter;
-    if (hist && it - 1 < st->maxit) hist[it - 1] = (double)res;
-    if (res < st->tol && unscaled_ok(st, tot[1])) {
-      st->info = 1;
-      st->done = 1;
-      return;
-    }
-    if (st->omega == (T)0) {
-      st->info = 37;
-      st->done = 1;
-      return;
-    }
-    st->iter = it + 1;
-    if (it + 1 > st->maxit) {
-      st->info = 2;
-      st->done = 1;
-    } else if (st->rho_new == (T)0) {
-      st->info = 35;
-      st->done = 1;
-    } else {
-      st->rho = st->rho_new;
-    }
-  }
-};
 
 // fast BiCGStab p update: p = r + beta (p - omega v) ; t1v = p/dg
 template <typename T>
@@ -1355,6 +1133,9 @@ static void launch_epi_sellb(ehip_system *s, const T *sv, const T *xin, const Ep
 // after them reduces 4x fewer partials): the fused FP32 CG step on 128^3
 // Hex8 Poisson measured 73.5 against 75.2 us.  The FP64 and node-blocked
 // kernels measured slower that way and keep sell_grid.
+// With the half storage, whose step takes its second reads from the caches
+// and gains from more waves in flight, 2048 (microbenchmark of the step at
+// 128^3, 1024 / 2048 / 4096 workgroups: 36.7 / 33.2 / 31.7 us).
 template <typename T>
 static int epi_sell_grid(const ehip_system *s) {
   if (sizeof(T) != 4 || s->sellb_d) return sell_grid(s);
@@ -1575,6 +1356,21 @@ static Vecs<T> make_vecs(T *w, int n, int method, T *x, T *b) {
 }
 static int nvecs(int method) { return method == EHIP_CG ? 6 : 10; }
 
+// A Krylov sequence in one launch (resident.hip), until it stops; its state in
+// hst.  *resident = false: the grid gave up waiting (the device is shared
+// with something that kept part of it off the chip) and the vectors and the
+// state are as before, for the launched loop to go on from.
+template <typename T>
+static int run_resident(ehip_system *s, SolveCtx &c, const Vecs<T> &v, KStateT<T> *st, KStateT<T> *hst, bool faithful,
+                        double *hist, const T *du, int it0, bool *resident) {
+  std::lock_guard<std::mutex> lk(resident_lock(s));
+  int rc;
+  if ((rc = (c.method == EHIP_CG ? resident_cg<T> : resident_bicgstab<T>)(s, v, st, faithful, hist, du)) || (rc = read_state(s, st, hst))) return rc;
+  *resident = hst->ticket[3] == 0;
+  if (*resident) c.spmv += std::max(0, hst->iter - it0) * ((faithful ? 2 : 1) + (c.method == EHIP_CG ? 0 : 1));
+  return EHIP_OK;
+}
+
 // Krylov iterations on a scaled system in precision T.  For T = double the
 // vectors are s->x / s->rhs; for the FP32 inner solve of the mixed form they
 // are the caller's.  Returns with the final state in hst.
@@ -1601,10 +1397,15 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
     hipLaunchKernelGGL(k_init_state<T>, dim3(1), dim3(1), 0, s->stream, st, (T)c.tol, c.maxit, (T)c.divtol, iter0,
                        tol_u);
   }
+  bool resident = false;
   if (c.method == EHIP_CG) {
+    resident = s->resident_on && resident_fits<T>(s, c.mode == EHIP_FAITHFUL);
     if (c.mode == EHIP_FAITHFUL) {
       EHIP_HIP_TRY(hipMemcpyAsync(v.p, v.z, sizeof(T) * n, hipMemcpyDeviceToDevice, s->stream));
-      for (;;) {
+      if (resident) {
+        if ((rc = run_resident<T>(s, c, v, st, hst, true, c.hist, du, iter0, &resident))) return rc;
+      }
+      for (; !resident;) {
         for (int k = 0; k < c.check; ++k) {
           EpiCgQ<T> e1{v, st, part, pg, &st->ticket[0]};
           if (c.prof) prof_begin(s);
@@ -1621,8 +1422,9 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
       }
     } else {
       hipLaunchKernelGGL(k_zero2<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v.p, v.q);
-      for (;;) {
-        for (int k = 0; k < c.check; ++k) {
+      for (int it_seen = iter0;; it_seen = hst->iter) {
+        if (resident && (rc = run_resident<T>(s, c, v, st, hst, false, c.hist, du, it_seen, &resident))) return rc;
+        for (int k = 0; !resident && k < c.check; ++k) {
           EpiCgFast1<T> e1{v, st, part, pg, &st->ticket[0], (T)0};
           if (c.prof) prof_begin(s);
           launch_epi<T>(s, plan, vals, v.z, e1, st);
@@ -1632,7 +1434,7 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
           fin<T>(s, FinCgFast2<T>{st, part + kVecPartOff, gf, c.hist}, gf, st);
           c.spmv++;
         }
-        if ((rc = read_state(s, st, hst))) return rc;
+        if (!resident && (rc = read_state(s, st, hst))) return rc;
         if (!hst->done) continue;
         if (!hst->rec_conv || !init_residual) break;  // inner solves stop on the recurrence
         // recurrence converged: confirm with the true residual, restart from it otherwise
@@ -1644,10 +1446,14 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
       }
     }
   } else {
+    resident = s->resident_on && resident_fits<T>(s, c.mode == EHIP_FAITHFUL);
     hipLaunchKernelGGL(k_bi_start<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st, part);
     fin<T>(s, FinBiStart<T>{st, part, g}, g, st);
-    for (;;) {
-      for (int k = 0; k < c.check; ++k) {
+    for (int it_seen = iter0;; it_seen = hst->iter) {
+      if (resident &&
+          (rc = run_resident<T>(s, c, v, st, hst, c.mode == EHIP_FAITHFUL, c.hist, du, it_seen, &resident)))
+        return rc;
+      for (int k = 0; !resident && k < c.check; ++k) {
         EpiBiV<T> e3{v, st, part, pg, &st->ticket[0]};
         if (c.prof) prof_begin(s);
         launch_epi<T>(s, plan, vals, v.t1v, e3, st);
@@ -1671,7 +1477,7 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
           hipLaunchKernelGGL(k_bi_p<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st);
         }
       }
-      if ((rc = read_state(s, st, hst))) return rc;
+      if (!resident && (rc = read_state(s, st, hst))) return rc;
       if (!hst->done) continue;
       if (c.mode == EHIP_FAITHFUL || !hst->rec_conv || !init_residual) break;
       EpiTrue<T> et{v, st, part, pg, &st->ticket[0], du};
@@ -1921,14 +1727,20 @@ static int mixed_cg_ru(ehip_system *s, SolveCtx &c, double delta, int *inner_tot
   // the SELL copy of the FP32 values is refreshed here, outside any recording
   if (active_fmt<float>(s) == 1 && !sell_values32(s)) return EHIP_ENOMEM;
   if (active_fmt<float>(s) == 2 && !sym_values32(s) && !sho_values32(s)) return EHIP_ENOMEM;
+  bool resident = s->resident_on && resident_fits<float>(s, false);
   while (!s->h_st->done) {
-    if (c.prof || !graphs_enabled()) {
+    if (resident && (rc = run_resident<float>(s, c, v, st32, s->h_st32, false, nullptr, nullptr, it_prev, &resident)))
+      return rc;
+    if (resident) {
+    } else if (c.prof || !graphs_enabled()) {
       cg32_iterations(s, v, batch, c.prof);  // sampled launches need their own events
     } else if ((rc = cg32_iterations_graph(s, v, batch))) {
       return rc;
     }
-    c.spmv += batch;
-    if ((rc = read_state(s, st32, s->h_st32))) return rc;
+    if (!resident) {
+      c.spmv += batch;
+      if ((rc = read_state(s, st32, s->h_st32))) return rc;
+    }
     const KState32 h = *s->h_st32;
     if (h.iter > it_prev && h.res > 0.f) {
       const double lr = std::log((double)h.res);
@@ -2344,6 +2156,11 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   // halved stream gave (63^3 Hex8: 37 us full, 42 us half; FP64 112 and 84)
   s->sym_on = p->method == EHIP_CG && p->precond < EHIP_PRECOND_ILU0 &&
               (s->sho_d == 1 || p->precision == EHIP_FP64);
+  // one launch per sequence where the rows fit the chip (not for callers
+  // without runtime objects of their own, nor when launches are sampled)
+  s->resident_on = events && !tl_shared_device && p->profile_every <= 0 && p->precond < EHIP_PRECOND_ILU0;
+  if (s->resident_on && resident_fits<double>(s, p->mode == EHIP_FAITHFUL && p->precision == EHIP_FP64))
+    s->sym_on = false;  // that loop reads the full copy
   SolveClock clk(events, s->stream);
   EHIP_HIP_TRY(clk.create());
   ehip_report rep{};

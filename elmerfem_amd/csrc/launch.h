@@ -33,6 +33,11 @@ inline hipError_t take_launch_error() {
   return e;
 }
 
+// Set on threads whose solves run beside others on the device (a server's
+// concurrent lane): these keep the launched loops, which share the chip,
+// where a resident loop would hold it and make the others wait.
+extern thread_local bool tl_shared_device;
+
 // Whether iteration blocks may be replayed as graphs: off when EHIP_GRAPHS=0,
 // and off under rocprofv3 (ROCPROF_OUTPUT_PATH in the environment), where
 // the same kernels are launched one by one instead.

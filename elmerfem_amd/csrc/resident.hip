@@ -1,0 +1,820 @@
+// Resident Krylov loops: a whole CG sequence of a system of moderate size in
+// one launch.
+//
+// Below a quarter of a million rows an iteration of the launched loops
+// (krylov.hip) is bound by its two to four dependent launches of 4 to 8 us
+// each, not by the matrix: 27 us an iteration in HUTI's order on 17^3 Hex8
+// (5 832 rows), 21 us for the one-SpMV order on 47^3.  Here every row belongs
+// to one thread of a grid that stays on the chip until the sequence stops:
+// the thread's entries of x, r, z, p, q and the Jacobi diagonal stay in its
+// registers, the matrix in the L2 of its XCD, and the vector that the SpMV
+// gathers in the workgroup's LDS (its 1024 rows and a halo of the
+// bandwidth).  What is left of an iteration are its two exchanges between
+// workgroups: partial sums, and the halo's new entries with the second one.
+//
+// Exchanges.  A workgroup publishes its partial sums as 64-bit words that
+// carry the exchange's number beside 32 bits of the value, with agent-scope
+// stores; everyone polls the words of all workgroups and adds them up in the
+// launched loops' order.  Vector entries go out before that with
+// agent-scope stores, acknowledged before the partial sums are published,
+// and are read with agent-scope loads after everyone's have been seen: no
+// cache is written back or invalidated.  The words of one exchange are
+// written again two exchanges later, when every workgroup has published the
+// one between and so has read them.
+//
+// Bits.  Sums are grouped as the launched kernels group them -- the SpMV's
+// partials per 256 rows, the vector step's per 1024 rows with four rows to
+// a thread, the totals over 256 threads -- and the scalar updates and
+// stopping tests are the same functors (cg_steps.h), so a solve gives the
+// same bits either way.
+//
+// Waiting.  All workgroups of the grid (at most 256, one per CU) must be on
+// the chip at once.  One such launch at a time runs on a device (a host lock),
+// other kernels end by themselves, and every wait is bounded: a thread that
+// polls past kSpins gives up for the whole grid.  Results go to separate
+// buffers, which a commit launch copies only if nobody gave up, so the
+// launched loop then takes over from the unchanged vectors.
+#include <hip/hip_runtime.h>
+
+#include <mutex>
+
+#include "cg_steps.h"
+#include "ehip_internal.h"
+#include "launch.h"
+
+namespace ehip {
+
+namespace {
+
+constexpr int kResRows = 1024;    // rows (and threads) of a workgroup
+constexpr int kResGroups = 256;   // one per CU
+constexpr int kResLds = 156 * 1024;
+constexpr int kSpins = 1 << 20;
+typedef unsigned long long Word;
+
+__device__ __forceinline__ Word ld_word(const Word *p) {
+  return __hip_atomic_load(const_cast<Word *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_word(Word *p, Word v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double ld_agent(const double *p) {
+  return __hip_atomic_load(const_cast<double *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float ld_agent(const float *p) {
+  return __hip_atomic_load(const_cast<float *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void st_agent(T *p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// this wave's stores have reached the coherence point
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// A value as words: FP32 one, FP64 two.
+template <typename T>
+constexpr int kWords = sizeof(T) / 4;
+__device__ __forceinline__ void publish(Word *p, unsigned e, double v) {
+  const Word b = (Word)__double_as_longlong(v), hi = (Word)e << 32;
+  st_word(p, hi | (b & 0xffffffffull));
+  st_word(p + 1, hi | (b >> 32));
+}
+__device__ __forceinline__ void publish(Word *p, unsigned e, float v) {
+  st_word(p, ((Word)e << 32) | __float_as_uint(v));
+}
+__device__ __forceinline__ bool seen(const Word *p, unsigned e, double &v) {
+  const Word a = ld_word(p), b = ld_word(p + 1);
+  v = __longlong_as_double((long long)((a & 0xffffffffull) | (b << 32)));
+  return (unsigned)(a >> 32) == e && (unsigned)(b >> 32) == e;
+}
+__device__ __forceinline__ bool seen(const Word *p, unsigned e, float &v) {
+  const Word a = ld_word(p);
+  v = __uint_as_float((unsigned)a);
+  return (unsigned)(a >> 32) == e;
+}
+
+}  // namespace
+
+// The matrix in the layout the launched SpMV reads: slice-shared offsets
+// (SHO), or SELL-64 with 16-bit columns, FP64 values pair-packed.
+enum ResFmt { RES_SHO, RES_SELL };
+
+template <typename T>
+struct ResArgs {
+  int n, nslice, halo;
+  int ngroups;                  // 256-row groups with rows
+  int spmv_grid, vec_grid;      // workgroups of the launched kernels
+  const int *off, *tab;         // SHO: slice offsets and offset lists; SELL: slice offsets, slice bases
+  const unsigned *mask;         // SHO
+  const unsigned short *c16;    // SELL
+  const int *rows;              // SELL
+  const T *vals;
+  Vecs<T> v, out;               // the vectors, and where the results go
+  const KStateT<T> *st;
+  KStateT<T> *st_out;
+  Word *w1, *w2;                // words of the two exchanges
+  T *ex, *ez, *er, *ew;         // vector entries on their way to other workgroups
+  int *gave_up;
+  double *hist;
+  const T *du;
+};
+
+namespace {
+
+// launched workgroup of the SpMV that has 256-row group g (XcdWalk: at most
+// one group each, the grid being at least as large as their number)
+__device__ __forceinline__ int spmv_slot(int g, int ngroups) {
+  int xcd = (int)((long long)g * 8 / ngroups);
+  while ((long long)ngroups * (xcd + 1) / 8 <= g) ++xcd;
+  while ((long long)ngroups * xcd / 8 > g) --xcd;
+  return (g - (int)((long long)ngroups * xcd / 8)) * 8 + xcd;
+}
+__device__ __forceinline__ bool slot_used(int b, int ngroups) {
+  const int xcd = b & 7, lb = b >> 3;
+  return (int)((long long)ngroups * xcd / 8) + lb < (int)((long long)ngroups * (xcd + 1) / 8);
+}
+
+// A row's matrix entries.  SHO: the values in registers (at most KW of
+// them), the slice's offset list read with scalar loads.  SELL: read from
+// the L2 in every product.
+template <typename T, ResFmt F, int KW>
+struct ResRow {
+  T v[F == RES_SHO ? KW : 1];
+  unsigned m;                     // SHO: the row's own entries (FP32: all of the list's)
+  const int *__restrict__ t;
+  int wd, rl, p0, len;
+  __device__ __forceinline__ void load(const ResArgs<T> &a, int sl, int lane) {
+    constexpr bool kF32 = sizeof(T) == 4;
+    const int r = sl * 64 + lane;
+    rl = min(r, a.n - 1);
+    const bool live = sl < a.nslice;
+    p0 = live ? a.off[sl] : 0;
+    const int width = live ? a.off[sl + 1] - p0 : 0;
+    if constexpr (F == RES_SHO) {
+      wd = width >> 6;
+      t = a.tab + (p0 >> 6);
+      m = kF32 ? (wd >= 32 ? ~0u : (1u << wd) - 1u) : (r < a.n ? a.mask[rl] : 0u);
+#pragma unroll
+      for (int k = 0; k < KW; ++k) v[k] = k < wd ? a.vals[p0 + 64 * k + lane] : (T)0;
+    } else {
+      wd = kF32 ? width >> 6 : width >> 7;
+      len = r < a.n ? a.rows[rl + 1] - a.rows[rl] : 0;
+    }
+  }
+  // Sums of one or two vectors held in LDS windows starting at column wb, in
+  // the launched kernels' order (spmv_sho_body, spmv_sell2_body,
+  // spmv_sell_body).
+  template <int NX>
+  __device__ __forceinline__ void sums(const ResArgs<T> &a, int sl, int lane, int wb, const T *w0, const T *w1,
+                                       T (&s)[NX]) const {
+    constexpr bool kF32 = sizeof(T) == 4;
+#pragma unroll
+    for (int x = 0; x < NX; ++x) s[x] = (T)0;
+    auto add = [&](T e, int c, bool on) {
+#pragma clang fp contract(off)
+      const T t0 = s[0] + e * w0[c];
+      s[0] = on ? t0 : s[0];
+      if constexpr (NX > 1) {
+        const T t1 = s[1] + e * w1[c];
+        s[1] = on ? t1 : s[1];
+      }
+    };
+    if constexpr (F == RES_SHO) {
+#pragma unroll
+      for (int k = 0; k < KW; ++k)
+        if (k < wd) add(v[k], min(max(rl + t[k], 0), a.n - 1) - wb, (m >> k) & 1u);
+    } else if constexpr (!kF32) {
+      constexpr int U = 4;
+      const int b = sl < a.nslice ? a.tab[sl] - wb : 0;
+      for (int k0 = 0; k0 < wd; k0 += U) {
+        T v0[U], v1[U];
+        unsigned cc[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int idx = p0 + min(k0 + u, wd - 1) * 128 + 2 * lane;
+          v0[u] = a.vals[idx];
+          v1[u] = a.vals[idx + 1];
+          cc[u] = *reinterpret_cast<const unsigned *>(a.c16 + idx);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          add(v0[u], b + (int)(cc[u] & 0xffffu), 2 * (k0 + u) < len);
+          add(v1[u], b + (int)(cc[u] >> 16), 2 * (k0 + u) + 1 < len);
+        }
+      }
+    } else {
+      constexpr int U = 8;
+      const int b = sl < a.nslice ? a.tab[sl] - wb : 0;
+      for (int k0 = 0; k0 < wd; k0 += U) {
+        T vv[U];
+        int cc[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int idx = p0 + min(k0 + u, wd - 1) * 64 + lane;
+          vv[u] = a.vals[idx];
+          cc[u] = b + (int)a.c16[idx];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) add(vv[u], cc[u], k0 + u < wd);
+      }
+    }
+  }
+};
+
+// The workgroup's LDS beside the windows.
+template <typename T>
+struct ResShared {
+  KStateT<T> st;
+  // r and z of the vector step's partial sums (the first two), then
+  // everyone's partial sums
+  T part[3][kResRows];
+  T wave[16 * 3];
+  T tot[3][4];
+  int fail;
+};
+
+// Sum over a 256-row group's rows of val, as the launched SpMV's workgroup
+// publishes it (block_publish with 256 threads), for the workgroup's four groups.
+template <typename T, int NV>
+__device__ __forceinline__ void publish_groups(const ResArgs<T> &a, ResShared<T> &sh, Word *w, unsigned e,
+                                               const T (&val)[NV]) {
+  const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const T s = wave_sum(val[k]);
+    if (lane == 0) sh.wave[16 * k + wv] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < 4 * NV) {
+    const int g = blockIdx.x * 4 + ((int)threadIdx.x & 3), k = (int)threadIdx.x >> 2;
+    if (g < a.ngroups) {
+      T t = (T)0;
+      for (int i = 0; i < 4; ++i) t += sh.wave[16 * k + 4 * ((int)threadIdx.x & 3) + i];
+      publish(w + ((size_t)k * a.spmv_grid + spmv_slot(g, a.ngroups)) * kWords<T>, e, t);
+    }
+  }
+}
+
+// Partial sums of the vector step over this workgroup's 1024 rows
+// (block_publish after CgTile::step: four rows to a thread).
+template <typename T, int NV>
+__device__ __forceinline__ void publish_rows(const ResArgs<T> &a, ResShared<T> &sh, Word *w, unsigned e) {
+  const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  if (tid < 256) {
+    T acc[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) acc[k] = (T)0;
+#pragma unroll
+    for (int k = 0; k < kVI; ++k) {
+      const int i = k * kVecBlock + tid;
+      if ((int)blockIdx.x * kResRows + i < a.n) {
+        const T ri = sh.part[0][i], zi = sh.part[1][i];
+        acc[0] += ri * zi;
+        if constexpr (NV > 1) acc[1] += ri * ri;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const T s = wave_sum(acc[k]);
+      if (lane == 0) sh.wave[16 * k + wv] = s;
+    }
+  }
+  stores_done();  // the vector entries go before the partial sums
+  __syncthreads();
+  if (tid < NV) {
+    T t = (T)0;
+    for (int i = 0; i < 4; ++i) t += sh.wave[16 * tid + i];
+    publish(w + ((size_t)tid * a.vec_grid + blockIdx.x) * kWords<T>, e, t);
+  }
+}
+
+// Waits for everyone's partial sums, one workgroup's to a thread with all
+// its words in flight, and adds them in block_reduce_all's order (256
+// threads).  False: someone gave up.
+template <typename T, int NV, bool SPMV>
+__device__ __forceinline__ bool gather(const ResArgs<T> &a, ResShared<T> &sh, const Word *w, unsigned e, T (&tot)[NV]) {
+  const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int g = SPMV ? a.spmv_grid : a.vec_grid;  // at most 1024
+  T v[NV];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) v[k] = (T)0;
+  if (tid < g && (SPMV ? slot_used(tid, a.ngroups) : tid < (int)gridDim.x)) {
+    for (int spins = 0;; ++spins) {
+      bool all = true;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) all &= seen(w + ((size_t)k * g + tid) * kWords<T>, e, v[k]);
+      if (all) break;
+      if (spins > kSpins ||
+          ((spins & 63) == 63 && __hip_atomic_load(a.gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+        __hip_atomic_store(a.gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sh.fail = 1;
+        break;
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NV; ++k) sh.part[k][tid] = v[k];
+  __syncthreads();
+  if (tid < 256) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      T s = (T)0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s += sh.part[k][tid + 256 * u];
+      s = wave_sum(s);
+      if (lane == 0) sh.tot[k][wv] = s;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    T t = (T)0;
+    for (int i = 0; i < 4; ++i) t += sh.tot[k][i];
+    tot[k] = t;
+  }
+  return sh.fail == 0;
+}
+
+// Calls f(c, entries of e0 (and e1) at column c) for the workgroup's halo
+// columns, kHaloU columns of a thread in flight.
+constexpr int kHaloU = 6;
+template <typename T, int NE, class Fn>
+__device__ __forceinline__ void halo_columns(int wb, int nlow, int re, int nhalo, const T *e0, const T *e1, Fn f) {
+  for (int i0 = (int)threadIdx.x; i0 < nhalo; i0 += kHaloU * kResRows) {
+    T v[NE][kHaloU];
+#pragma unroll
+    for (int u = 0; u < kHaloU; ++u) {
+      const int i = min(i0 + u * kResRows, nhalo - 1);
+      const int c = i < nlow ? wb + i : re + (i - nlow);
+      v[0][u] = ld_agent(e0 + c);
+      if constexpr (NE > 1) v[1][u] = ld_agent(e1 + c);
+    }
+#pragma unroll
+    for (int u = 0; u < kHaloU; ++u) {
+      const int i = i0 + u * kResRows;
+      if (i < nhalo) f(i < nlow ? wb + i : re + (i - nlow), v[0][u], v[NE - 1][u]);
+    }
+  }
+}
+
+}  // namespace
+
+// One CG sequence.  FAITHFUL: HUTI's order with the true residual of every
+// iteration; its product A x and the next iteration's A p are taken in one
+// pass over the matrix.  Else the one-SpMV order (FinCgFast2's tests).
+template <typename T, ResFmt F, int KW, bool FAITHFUL>
+__global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
+  extern __shared__ __align__(16) char lds[];
+  __shared__ ResShared<T> sh;
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const int R0 = (int)blockIdx.x * kResRows, r = R0 + tid, rl = min(r, a.n - 1);
+  const bool ok = r < a.n;
+  const int sl = __builtin_amdgcn_readfirstlane(R0 / 64 + (tid >> 6));
+  const int wb = max(R0 - a.halo, 0), we = min(R0 + kResRows + a.halo, a.n), own = r - wb;
+  const int re = min(R0 + kResRows, a.n);  // the halo: [wb, R0) and [re, we)
+  const int nlow = R0 - wb, nhalo = nlow + (we - re);
+  T *win = reinterpret_cast<T *>(lds);     // z, or p with FAITHFUL
+  T *winx = win + (kResRows + 2 * a.halo); // x (FAITHFUL)
+  T x = a.v.x[rl], p = a.v.p[rl], q = a.v.q[rl], rr = a.v.r[rl], z = a.v.z[rl];
+  const T dg = a.v.dg[rl];
+  const T b = FAITHFUL ? a.v.b[rl] : (T)0, d = FAITHFUL && a.du ? a.du[rl] : (T)1;
+  ResRow<T, F, KW> row;
+  row.load(a, sl, lane);
+  if (tid == 0) {
+    sh.st = *a.st;
+    sh.fail = 0;
+  }
+  {
+    const T *src = FAITHFUL ? a.v.p : a.v.z;
+    for (int i = wb + tid; i < we; i += kResRows) win[i - wb] = src[i];
+  }
+  __syncthreads();
+  double *const hist = blockIdx.x == 0 ? a.hist : nullptr;
+  unsigned e = 1;
+  T sx[FAITHFUL ? 2 : 1];
+  bool lost = false;
+  if constexpr (FAITHFUL) {
+    T s[1];
+    row.template sums<1>(a, sl, lane, wb, win, win, s);
+    q = s[0];
+    T acc[3] = {(T)0, (T)0, (T)0};
+    if (ok) acc[0] += p * q;
+    publish_groups<T, 3>(a, sh, a.w1, e, acc);
+  }
+  if (!sh.st.done) for (bool first = true;; first = false) {
+    T pq;
+    if constexpr (FAITHFUL) {
+      T tot[3];
+      if (!gather<T, 3, true>(a, sh, a.w1, e, tot)) { lost = true; break; }
+      if (!first) {
+        T two[2] = {tot[1], tot[2]};
+        EpiCgResidual<T> f{a.v, &sh.st, nullptr, 0, nullptr, hist, nullptr, 0, (T)0, a.du};
+        f.finish(two);
+        __syncthreads();
+        if (sh.st.done) break;
+      }
+      pq = tot[0];
+    } else {
+      row.template sums<1>(a, sl, lane, wb, win, win, sx);
+      const T beta = sh.st.beta;
+      q = sx[0] + beta * q;
+      p = z + beta * p;
+      T acc[1] = {(T)0};
+      if (ok) acc[0] += p * q;
+      publish_groups<T, 1>(a, sh, a.w1, e, acc);
+      T tot[1];
+      if (!gather<T, 1, true>(a, sh, a.w1, e, tot)) { lost = true; break; }
+      pq = tot[0];
+    }
+    ++e;
+    const T alpha = sh.st.rho / pq;
+    x = x + alpha * p;
+    rr = rr - alpha * q;
+    z = rr / dg;
+    if (ok) {
+      st_agent(a.ez + r, z);
+      if constexpr (FAITHFUL) st_agent(a.ex + r, x);
+    }
+    sh.part[0][tid] = rr;
+    sh.part[1][tid] = z;
+    if constexpr (!FAITHFUL) win[own] = z;
+    __syncthreads();
+    if constexpr (FAITHFUL) {
+      publish_rows<T, 1>(a, sh, a.w2, e);
+      T rn[1];
+      if (!gather<T, 1, false>(a, sh, a.w2, e, rn)) { lost = true; break; }
+      const T beta = rn[0] / sh.st.rho;
+      p = z + beta * p;
+      halo_columns<T, 2>(wb, nlow, re, nhalo, a.ez, a.ex, [&](int c, T zc, T xc) {
+        win[c - wb] = zc + beta * win[c - wb];
+        winx[c - wb] = xc;
+      });
+      if (ok) {
+        win[own] = p;
+        winx[own] = x;
+      }
+      __syncthreads();
+      if (tid == 0) {
+        sh.st.pq = pq;
+        sh.st.alpha = alpha;
+        sh.st.rho_new = rn[0];
+      }
+      row.template sums<2>(a, sl, lane, wb, win, winx, sx);
+      q = sx[0];
+      T acc[3] = {(T)0, (T)0, (T)0};
+      if (ok) {
+        acc[0] += p * q;
+        const T ti = sx[1] - b;
+        acc[1] += ti * ti;
+        const T ui = ti / d;
+        acc[2] += ui * ui;
+      }
+      ++e;
+      publish_groups<T, 3>(a, sh, a.w1, e, acc);
+    } else {
+      publish_rows<T, 2>(a, sh, a.w2, e);
+      T tot[2];
+      if (!gather<T, 2, false>(a, sh, a.w2, e, tot)) { lost = true; break; }
+      if (tid == 0) {
+        sh.st.pq = pq;
+        sh.st.alpha = alpha;
+      }
+      FinCgFast2<T>{&sh.st, nullptr, 0, hist}.finish(tot);
+      halo_columns<T, 1>(wb, nlow, re, nhalo, a.ez, a.ez, [&](int c, T zc, T) { win[c - wb] = zc; });
+      __syncthreads();
+      if (sh.st.done) break;
+      ++e;
+    }
+  }
+  if (lost) return;  // nothing is committed
+  if (ok) {
+    a.out.x[r] = x;
+    a.out.r[r] = rr;
+    a.out.z[r] = z;
+    a.out.p[r] = p;
+    a.out.q[r] = q;
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    sh.st.fresh = 1;
+    *a.st_out = sh.st;
+  }
+}
+
+// One BiCGStab sequence in huti_bicgstab.src order, four exchanges an
+// iteration.  FAITHFUL: the true residual of every iteration, its product
+// A x taken in one pass with the next iteration's A t1v; else FinBiXr's tests
+// on the recurrence residual.  The halo's t1v = (r + beta w) / dg needs beta,
+// so r and w = p - omega v travel with the partial sums that give it.
+template <typename T, ResFmt F, int KW, bool FAITHFUL>
+__global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
+  extern __shared__ __align__(16) char lds[];
+  __shared__ ResShared<T> sh;
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const int R0 = (int)blockIdx.x * kResRows, r = R0 + tid, rl = min(r, a.n - 1);
+  const bool ok = r < a.n;
+  const int sl = __builtin_amdgcn_readfirstlane(R0 / 64 + (tid >> 6));
+  const int wb = max(R0 - a.halo, 0), we = min(R0 + kResRows + a.halo, a.n), own = r - wb;
+  const int re = min(R0 + kResRows, a.n);
+  const int nlow = R0 - wb, nhalo = nlow + (we - re);
+  T *win = reinterpret_cast<T *>(lds);      // t1v and t2v in turn
+  T *winx = win + (kResRows + 2 * a.halo);  // x (FAITHFUL)
+  T x = a.v.x[rl], p = a.v.p[rl], v = a.v.v[rl], rr = a.v.r[rl], t1 = a.v.t1v[rl];
+  const T dg = a.v.dg[rl], rt = a.v.rtld[rl];
+  const T b = FAITHFUL ? a.v.b[rl] : (T)0, d = FAITHFUL && a.du ? a.du[rl] : (T)1;
+  ResRow<T, F, KW> row;
+  row.load(a, sl, lane);
+  if (tid == 0) {
+    sh.st = *a.st;
+    sh.fail = 0;
+  }
+  for (int i = wb + tid; i < we; i += kResRows) win[i - wb] = a.v.t1v[i];
+  __syncthreads();
+  double *const hist = blockIdx.x == 0 ? a.hist : nullptr;
+  unsigned e = 0;
+  bool lost = false;
+  if (!sh.st.done) for (bool first = true;; first = false) {
+    ++e;
+    if (FAITHFUL && !first) {
+      T s[2];
+      row.template sums<2>(a, sl, lane, wb, win, winx, s);
+      v = s[0];
+      T acc[3] = {(T)0, (T)0, (T)0};
+      if (ok) {
+        acc[0] += rt * v;
+        const T ti = s[1] - b;
+        acc[1] += ti * ti;
+        const T ui = ti / d;
+        acc[2] += ui * ui;
+      }
+      publish_groups<T, 3>(a, sh, a.w1, e, acc);
+    } else {
+      T s[1];
+      row.template sums<1>(a, sl, lane, wb, win, win, s);
+      v = s[0];
+      T acc[3] = {(T)0, (T)0, (T)0};
+      if (ok) acc[0] += rt * v;
+      publish_groups<T, 3>(a, sh, a.w1, e, acc);
+    }
+    T rv[3];
+    if (!gather<T, 3, true>(a, sh, a.w1, e, rv)) { lost = true; break; }
+    if (FAITHFUL && !first) {
+      T two[2] = {rv[1], rv[2]};
+      EpiBiResidual<T> f{a.v, &sh.st, nullptr, 0, nullptr, hist, (T)0, (T)0, a.du};
+      f.finish(two);
+      __syncthreads();
+      if (sh.st.done) break;
+    }
+    const T alpha = sh.st.rho / rv[0];
+    const T s = rr - alpha * v;
+    const T t2 = s / dg;
+    if (ok) st_agent(a.ez + r, t2);
+    sh.part[0][tid] = s;
+    sh.part[1][tid] = s;
+    win[own] = t2;
+    __syncthreads();
+    ++e;
+    publish_rows<T, 1>(a, sh, a.w2, e);
+    T ss[1];
+    if (!gather<T, 1, false>(a, sh, a.w2, e, ss)) { lost = true; break; }
+    if (tid == 0) sh.st.alpha = alpha;
+    FinSnorm<T>{&sh.st, nullptr, 0}.finish(ss);
+    halo_columns<T, 1>(wb, nlow, re, nhalo, a.ez, a.ez, [&](int c, T tc, T) { win[c - wb] = tc; });
+    __syncthreads();
+    if (sh.st.snorm_exit) {
+      x = x + alpha * t1;
+      if (tid == 0) sh.st.done = 1;
+      break;
+    }
+    T tv;
+    {
+      T q[1];
+      row.template sums<1>(a, sl, lane, wb, win, win, q);
+      tv = q[0];
+    }
+    {
+      T acc[2] = {(T)0, (T)0};
+      if (ok) {
+        acc[0] += tv * s;
+        acc[1] += tv * tv;
+      }
+      ++e;
+      publish_groups<T, 2>(a, sh, a.w1, e, acc);
+    }
+    T tt[2];
+    if (!gather<T, 2, true>(a, sh, a.w1, e, tt)) { lost = true; break; }
+    const T omega = tt[0] / tt[1];
+    x = x + alpha * t1 + omega * t2;
+    rr = s - omega * tv;
+    const T w = p - omega * v;
+    if (ok) {
+      st_agent(a.er + r, rr);
+      st_agent(a.ew + r, w);
+      if constexpr (FAITHFUL) st_agent(a.ex + r, x);
+    }
+    sh.part[0][tid] = rr;
+    sh.part[1][tid] = rt;
+    __syncthreads();
+    ++e;
+    publish_rows<T, 2>(a, sh, a.w2, e);
+    T rn[2];
+    if (!gather<T, 2, false>(a, sh, a.w2, e, rn)) { lost = true; break; }
+    if (tid == 0) {
+      sh.st.ts = tt[0];
+      sh.st.tt = tt[1];
+      sh.st.omega = omega;
+    }
+    FinBiXr<T>{&sh.st, nullptr, 0, FAITHFUL ? 0 : 1, hist}.finish(rn);
+    __syncthreads();
+    if (!FAITHFUL && sh.st.done) break;
+    const T beta = FAITHFUL ? (sh.st.rho_new * alpha) / (sh.st.rho * omega) : sh.st.beta;
+    p = rr + beta * w;
+    t1 = p / dg;
+    halo_columns<T, 2>(wb, nlow, re, nhalo, a.er, a.ew,
+                       [&](int c, T rc, T wc) { win[c - wb] = (rc + beta * wc) / a.v.dg[c]; });
+    if constexpr (FAITHFUL)
+      halo_columns<T, 1>(wb, nlow, re, nhalo, a.ex, a.ex, [&](int c, T xc, T) { winx[c - wb] = xc; });
+    if (ok) {
+      win[own] = t1;
+      if constexpr (FAITHFUL) winx[own] = x;
+    }
+    __syncthreads();
+  }
+  if (lost) return;  // nothing is committed
+  if (ok) {
+    a.out.x[r] = x;
+    a.out.r[r] = rr;
+    a.out.p[r] = p;
+    a.out.v[r] = v;
+    a.out.t1v[r] = t1;
+  }
+  __syncthreads();
+  if (blockIdx.x == 0 && tid == 0) *a.st_out = sh.st;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_resident_commit(int n, Vecs<T> v, Vecs<T> out, KStateT<T> *st,
+                                                         const KStateT<T> *st_out, const int *gave_up) {
+  if (*gave_up) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->ticket[3] = 1;
+    return;
+  }
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    v.x[i] = out.x[i];
+    v.r[i] = out.r[i];
+    v.p[i] = out.p[i];
+    if (out.q) {  // CG
+      v.z[i] = out.z[i];
+      v.q[i] = out.q[i];
+    } else {
+      v.v[i] = out.v[i];
+      v.t1v[i] = out.t1v[i];
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) *st = *st_out;
+}
+
+__global__ void k_resident_clear(Word *w, int nw, int *gave_up, unsigned *mark) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nw; i += gridDim.x * blockDim.x) w[i] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    *gave_up = 0;
+    *mark = 0;
+  }
+}
+
+static std::mutex g_resident_mu[16];
+
+std::mutex &resident_lock(const ehip_system *s) { return g_resident_mu[s->dev & 15]; }
+
+// Words of the exchanges: three SpMV values of up to 1024 groups, two
+// vector values of up to 1024 tiles, two words each.
+constexpr int kW1 = 3 * 1024 * 2, kW2 = 2 * 1024 * 2;
+
+// Rows per workgroup times CUs bound n; two windows of 1024 rows and the
+// halo on both sides must fit the LDS (one in the one-SpMV order).
+template <typename T>
+bool resident_fits(ehip_system *s, bool faithful) {
+  const int fmt = sizeof(T) == 4 ? s->fmt32 : s->fmt64;
+  const int halo = fmt == 2 ? s->sho_halo : s->sell_halo;
+  if (s->n > kResRows * kResGroups || halo < 0 || s->n < 1) return false;
+  if (fmt == 2) {
+    if (!s->sho_ok || s->sho_d != 1) return false;
+  } else if (fmt == 1) {
+    if (!s->sell_ok || s->sellb_d || s->sell_row || !s->sell_c16) return false;
+    if (sizeof(T) == 8 && !s->sell2_ok) return false;
+  } else {
+    return false;
+  }
+  const int64_t win = (kResRows + 2 * (int64_t)halo) * (int64_t)sizeof(T) * (faithful ? 2 : 1);
+  return win + (int64_t)sizeof(ResShared<T>) + 64 <= kResLds;
+}
+
+// Enqueues the sequence and its commit; the caller holds resident_lock from
+// here until it has read the state back, whose ticket[3] tells that the
+// grid gave up and nothing changed.
+template <typename T, bool CG>
+static int resident_run(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du) {
+  const int n = s->n;
+  int rc;
+  const size_t vec = ((size_t)n + 63) / 64 * 64;
+  const size_t need = (sizeof(Word) * (kW1 + kW2) + sizeof(KState) + 256) + 9 * vec * sizeof(double);
+  if (s->res_bytes < need) {
+    if (s->res_buf) dfree(s, s->res_buf, s->res_bytes);
+    s->res_buf = nullptr;
+    s->res_bytes = 0;
+    if ((rc = dmalloc(s, &s->res_buf, need))) return rc;
+    s->res_bytes = need;
+  }
+  char *p = (char *)s->res_buf;
+  ResArgs<T> a{};
+  a.w1 = (Word *)p;
+  a.w2 = a.w1 + kW1;
+  p += sizeof(Word) * (kW1 + kW2);
+  a.st_out = (KStateT<T> *)p;
+  p += (sizeof(KState) + 63) / 64 * 64;
+  a.gave_up = (int *)p;
+  p += 64;
+  T *w = (T *)p;
+  a.ex = w;
+  a.ez = w + vec;
+  a.er = w + 2 * vec;
+  a.ew = w + 3 * vec;
+  a.out.x = w + 4 * vec;
+  a.out.r = w + 5 * vec;
+  a.out.p = w + 6 * vec;
+  (CG ? a.out.z : a.out.v) = w + 7 * vec;
+  (CG ? a.out.q : a.out.t1v) = w + 8 * vec;
+  a.v = v;
+  a.st = st;
+  a.n = n;
+  a.nslice = s->nslice;
+  a.ngroups = (s->nslice + 3) / 4;
+  a.spmv_grid = sell_grid(s);
+  a.vec_grid = fused_grid(n);
+  a.hist = hist;
+  a.du = du;
+  const int fmt = sizeof(T) == 4 ? s->fmt32 : s->fmt64;
+  a.halo = fmt == 2 ? s->sho_halo : s->sell_halo;
+  if (fmt == 2) {
+    if constexpr (sizeof(T) == 4) a.vals = sho_values32(s); else a.vals = sho_values64(s);
+    a.off = s->sho_off;
+    a.tab = s->sho_tab;
+    a.mask = s->sho_mask;
+  } else {
+    if constexpr (sizeof(T) == 4) {
+      a.vals = sell_values32(s);
+      a.off = s->sell_off;
+      a.c16 = s->sell_c16;
+    } else {
+      a.vals = sell_values64(s);
+      a.off = s->sell2_off;
+      a.c16 = s->sell2_c16;
+    }
+    a.rows = s->rows;
+    a.tab = s->sell_base;
+  }
+  if (!a.vals) return EHIP_ENOMEM;
+  const int g = (n + kResRows - 1) / kResRows;
+  const size_t lds = (size_t)(kResRows + 2 * a.halo) * sizeof(T) * (faithful ? 2 : 1);
+  hipLaunchKernelGGL(k_resident_clear, dim3(16), dim3(256), 0, s->stream, a.w1, kW1 + kW2, a.gave_up, &st->ticket[3]);
+#define EHIP_RES(F, KW)                                                                                            \
+  if constexpr (CG) {                                                                                              \
+    if (faithful) hipLaunchKernelGGL((k_resident_cg<T, F, KW, true>), dim3(g), dim3(kResRows), lds, s->stream, a); \
+    else hipLaunchKernelGGL((k_resident_cg<T, F, KW, false>), dim3(g), dim3(kResRows), lds, s->stream, a);         \
+  } else {                                                                                                         \
+    if (faithful) hipLaunchKernelGGL((k_resident_bi<T, F, KW, true>), dim3(g), dim3(kResRows), lds, s->stream, a); \
+    else hipLaunchKernelGGL((k_resident_bi<T, F, KW, false>), dim3(g), dim3(kResRows), lds, s->stream, a);         \
+  }
+  // the widest slice's entries in registers: 9 (Quad4), 15 (Tet4), 27 (Hex8)
+  if (fmt != 2) { EHIP_RES(RES_SELL, 1); }
+  else if (s->sho_wmax <= 9) { EHIP_RES(RES_SHO, 9); }
+  else if (s->sho_wmax <= 15) { EHIP_RES(RES_SHO, 15); }
+  else if (s->sho_wmax <= 27) { EHIP_RES(RES_SHO, 27); }
+  else { EHIP_RES(RES_SHO, 32); }
+#undef EHIP_RES
+  EHIP_HIP_TRY(hipGetLastError());
+  hipLaunchKernelGGL(k_resident_commit<T>, dim3(vec_grid(n)), dim3(256), 0, s->stream, n, v, a.out, st,
+                     (const KStateT<T> *)a.st_out, (const int *)a.gave_up);
+  EHIP_HIP_TRY(hipGetLastError());
+  return EHIP_OK;
+}
+
+template <typename T>
+int resident_cg(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du) {
+  return resident_run<T, true>(s, v, st, faithful, hist, du);
+}
+template <typename T>
+int resident_bicgstab(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du) {
+  return resident_run<T, false>(s, v, st, faithful, hist, du);
+}
+
+template bool resident_fits<double>(ehip_system *, bool);
+template bool resident_fits<float>(ehip_system *, bool);
+template int resident_cg<double>(ehip_system *, const Vecs<double> &, KStateT<double> *, bool, double *,
+                                 const double *);
+template int resident_cg<float>(ehip_system *, const Vecs<float> &, KStateT<float> *, bool, double *, const float *);
+template int resident_bicgstab<double>(ehip_system *, const Vecs<double> &, KStateT<double> *, bool, double *,
+                                       const double *);
+template int resident_bicgstab<float>(ehip_system *, const Vecs<float> &, KStateT<float> *, bool, double *,
+                                      const float *);
+
+}  // namespace ehip

@@ -480,6 +480,9 @@ static int build_sho(ehip_system *s, const std::vector<int> &c0, int64_t sell_to
   s->sho_d = D;
   s->sho_nnz = tot;
   s->nslice = S;
+  s->sho_halo = 0;
+  for (int v : ctab) s->sho_halo = std::max(s->sho_halo, std::abs(v));
+  s->sho_wmax = *std::max_element(len.begin(), len.end());
   s->sho_ok = true;
   s->fmt64 = s->fmt32 = 2;
   return build_sym(s, ctab);
@@ -541,6 +544,7 @@ static int build_sell(ehip_system *s, const std::vector<int> &c0) {
   std::vector<int> col((size_t)tot, 0);
   std::vector<int> base((size_t)S, 0);
   bool c16 = true;
+  int halo = 0;
   for (int sl = 0; sl < S; ++sl) {
     const int wd = (off[sl + 1] - off[sl]) / 64;
     int lo = INT32_MAX, hi = INT32_MIN;
@@ -559,9 +563,11 @@ static int build_sell(ehip_system *s, const std::vector<int> &c0) {
       }
     }
     base[sl] = lo;
+    halo = std::max({halo, sl * 64 + 63 - lo, hi - sl * 64});
     if ((int64_t)hi - lo > 65535) c16 = false;
     if (blk && hi / D - lo / D > 65535) blk = false;
   }
+  if (!mapped) s->sell_halo = halo;
   int rc;
   if (mapped) {
     std::vector<int> rm((size_t)S * 64, n);
@@ -1202,7 +1208,7 @@ int ehip_system_free(ehip_system *s) {
                   s->sell2_c16,  s->sell_row,    s->sellb_c16, s->sellb_base, s->bw64,
                   s->bw32,       s->sho_off,     s->sho_tab,   s->sho_mask,   s->sho64,
                   s->sho32,      s->map_base,    s->sym_mask,  s->sym_pm,     s->sym_flag,
-                  s->sym64.v,    s->sym64.zero,  s->sym32.v,   s->sym32.zero};
+                  s->sym64.v,    s->sym64.zero,  s->sym32.v,   s->sym32.zero, s->res_buf};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   for (hipEvent_t e : s->prof_ev)
