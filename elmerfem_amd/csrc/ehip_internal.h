@@ -272,6 +272,7 @@ struct ehip_system {
   // recorded sweeps of up to two (source, destination) vector pairs
   int ilu_order = -1;
   int64_t ilu_nnz = 0;
+  int ilu_maxrow = 0;                  // entries of the longest row
   int *ilu_rows = nullptr, *ilu_cols = nullptr, *ilu_diag = nullptr, *ilu_amap = nullptr;
   double *ilu = nullptr;
   int *ilu_lord = nullptr, *ilu_uord = nullptr;

@@ -69,6 +69,106 @@ __global__ __launch_bounds__(kIluBlock) void k_ilu_rows(const int *__restrict__ 
   }
 }
 
+// The same level with one wave per row of at most 64 NC entries: lane t holds
+// entries t, t + 64, ... of row i, and each elimination step broadcasts row
+// k's upper entries to the lanes, so an entry takes its subtractions in the
+// same order (the same bits).  One lane per row walked both rows entry by
+// entry, a dependent memory latency each: 158 us a level at 64^3 Hex8,
+// against kAhead rows k in flight here, their bounds loaded for all of them
+// at once: 12 us (the launch included).
+constexpr int kAhead = 4;
+template <int NC>
+__global__ __launch_bounds__(kIluBlock) void k_ilu_rows_wave(const int *__restrict__ rows, const int *__restrict__ cols,
+                                                           const int *__restrict__ diag, double *ilu,
+                                                           const int *__restrict__ order, int begin, int end) {
+#pragma clang fp contract(off)
+  const int lane = (int)threadIdx.x & 63;
+  const int t = __builtin_amdgcn_readfirstlane(begin + (int)blockIdx.x * (kIluBlock / 64) + ((int)threadIdx.x >> 6));
+  if (t >= end) return;
+  const int i = order[t];
+  const int r0 = rows[i], len = rows[i + 1] - r0, nlow = diag[i] - r0;
+  int c[NC];
+  double v[NC];
+#pragma unroll
+  for (int h = 0; h < NC; ++h) {
+    const int e = lane + 64 * h;
+    c[h] = e < len ? cols[r0 + e] : -1;  // -1 names no column
+    v[h] = e < len ? ilu[r0 + e] : 0.0;
+  }
+  // bounds of the rows k that the lower entries name
+  int kd[NC], ke[NC];
+#pragma unroll
+  for (int h = 0; h < NC; ++h) {
+    const bool low = lane + 64 * h < nlow;
+    kd[h] = low ? diag[c[h]] : 0;
+    ke[h] = low ? rows[c[h] + 1] : 0;
+  }
+  auto pick_i = [&](const int (&x)[NC], int m) {
+    int y = 0;
+#pragma unroll
+    for (int h = 0; h < NC; ++h) {
+      const int z = __shfl(x[h], m & 63);
+      y = (m >> 6) == h ? z : y;
+    }
+    return __builtin_amdgcn_readfirstlane(y);
+  };
+  for (int m0 = 0; m0 < nlow; m0 += kAhead) {
+    // rows k of the next steps: their diagonal (entry 0) and upper entries
+    int uc[kAhead][NC], ul[kAhead];
+    double uv[kAhead][NC];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      const int m = min(m0 + q, nlow - 1);
+      const int d = pick_i(kd, m), l = pick_i(ke, m) - d;
+      ul[q] = l;
+#pragma unroll
+      for (int h = 0; h < NC; ++h) {
+        const int j = d + min(lane + 64 * h, l - 1);  // clamped into the row
+        uc[q][h] = cols[j];
+        uv[q][h] = ilu[j];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      const int m = m0 + q;
+      if (m >= nlow) break;
+      double sk = 0.0;
+#pragma unroll
+      for (int h = 0; h < NC; ++h) {
+        const double z = __shfl(v[h], m & 63);
+        sk = (m >> 6) == h ? z : sk;
+      }
+      if (sk == 0.0) continue;  // the same in every lane
+      const double ukk = __shfl(uv[q][0], 0);
+      if (fabs(ukk) > kAeps) {
+        sk = sk / ukk;
+#pragma unroll
+        for (int h = 0; h < NC; ++h)
+          if (lane + 64 * h == m) v[h] = sk;
+      }
+      for (int l = 1; l < ul[q]; ++l) {
+        int j = 0;
+        double u = 0.0;
+#pragma unroll
+        for (int h = 0; h < NC; ++h) {
+          const int zj = __shfl(uc[q][h], l & 63);
+          const double zu = __shfl(uv[q][h], l & 63);
+          j = (l >> 6) == h ? zj : j;
+          u = (l >> 6) == h ? zu : u;
+        }
+#pragma unroll
+        for (int h = 0; h < NC; ++h) {
+          const double w = v[h] - sk * u;
+          v[h] = c[h] == j ? w : v[h];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < NC; ++h)
+    if (lane + 64 * h < len) ilu[r0 + lane + 64 * h] = v[h];
+}
+
 // The LU solve's prescaled diagonal: 1/U(i,i), or 1 when |U(i,i)| < AEPS.
 __global__ void k_ilu_invdiag(int n, const int *__restrict__ diag, double *ilu) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
@@ -167,15 +267,19 @@ __global__ void k_lu_pending(int n, double *y, double *z, int *sync) {
 
 // One row of a sweep.  FWD: dst(i) = src(i) - sum over the lower part of
 // L(i,j) dst(j); else dst(i) = U(i,i)^-1 (src(i) - sum over the upper part
-// of U(i,j) dst(j)).  The lane first polls only the part's nearest entry
-// (column i - 1 or i + 1 as a rule, the dependency finished last), then
-// loads kLuU entries at a time; all of it in one loop, publishing the row
+// of U(i,j) dst(j)).  The lane first polls only the part's gate, an entry
+// of the last level but one or more before the row's own; from then on it
+// polls every entry that is still pending, so the value that turns ready
+// last arrives with the poll that finds it ready.  (Polling the entry of the
+// last level alone and loading the others after it cost a memory trip more
+// for every level of the critical path: 64^3 Hex8 ILU(0), 449 levels, 1.52 ms
+// a sweep then, 1.30 ms so.)  All of it is in one loop, the row published
 // inside it.  The loop ends for the whole wave at once (when every lane is
 // done): with a per-lane exit the compiler may move the publishing store
 // after the loop, where a lane publishes only once every lane of its wave is
 // done -- and a lane waiting for another lane of its wave would never be.
 template <bool FWD>
-__device__ __forceinline__ void sweep_row(int i, const int *__restrict__ rows, const int *__restrict__ cols,
+__device__ __forceinline__ void sweep_row(int i, int gate, const int *__restrict__ rows, const int *__restrict__ cols,
                                           const int *__restrict__ diag, const double *__restrict__ ilu,
                                           const double *__restrict__ src, double *dst, int *sync) {
 #pragma clang fp contract(off)
@@ -183,36 +287,37 @@ __device__ __forceinline__ void sweep_row(int i, const int *__restrict__ rows, c
   const int len = (FWD ? diag[i] : rows[i + 1]) - j0;
   double s = src[i];
   int k0 = 0, spins = 0;
-  bool near = len == 0, done = false;
+  bool open = gate < 0, done = false;
   // the part's factors and columns do not change during the sweep: the
-  // current chunk's are loaded before the wait, so a dependency that turns
-  // ready costs one more trip (its values), not two
+  // current chunk's are loaded before the wait
   double a[kLuU];
   int c[kLuU];
+  unsigned long long xb[kLuU];
+  unsigned pend = 0;  // entries of the chunk not seen ready yet
   auto load_chunk = [&](int k) {
 #pragma unroll
     for (int u = 0; u < kLuU; ++u) {
-      const int j = j0 + min(k + u, len - 1);  // clamped entries are dependencies too
+      const int j = j0 + min(k + u, len - 1);
       a[u] = ilu[j];
       c[u] = cols[j];
+      xb[u] = 0;
     }
+    pend = (1u << min(len - k, kLuU)) - 1u;
   };
-  int cn = 0;
-  if (len > 0) {
-    load_chunk(0);
-    cn = cols[FWD ? j0 + len - 1 : j0];
-  }
+  if (len > 0) load_chunk(0);
   for (;;) {
     if (__all(done)) break;  // wave-uniform exit
     if (done) continue;
     bool ready = true;
-    if (!near) ready = near = ld_agent(dst + cn) != kPending;
-    if (near && k0 < len) {
-      unsigned long long xb[kLuU];
+    if (!open) ready = open = ld_agent(dst + gate) != kPending;
+    if (open && k0 < len) {
 #pragma unroll
-      for (int u = 0; u < kLuU; ++u) xb[u] = ld_agent(dst + c[u]);
+      for (int u = 0; u < kLuU; ++u)
+        if ((pend >> u) & 1u) xb[u] = ld_agent(dst + c[u]);
 #pragma unroll
-      for (int u = 0; u < kLuU; ++u) ready = ready && xb[u] != kPending;
+      for (int u = 0; u < kLuU; ++u)
+        if (xb[u] != kPending) pend &= ~(1u << u);
+      ready = pend == 0;
       if (ready) {
 #pragma unroll
         for (int u = 0; u < kLuU; ++u) {
@@ -230,7 +335,7 @@ __device__ __forceinline__ void sweep_row(int i, const int *__restrict__ rows, c
       else
         __builtin_amdgcn_s_sleep(1);
     }
-    if ((near && k0 >= len) || fail) {
+    if ((open && k0 >= len) || fail) {
       if (fail) {
         __hip_atomic_store(&sync[2], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s = __longlong_as_double(0x7ff8000000000000ll);
@@ -244,7 +349,8 @@ __device__ __forceinline__ void sweep_row(int i, const int *__restrict__ rows, c
   }
 }
 
-// A sweep over all rows in level order (`order`): each workgroup takes the
+// A sweep over all rows in level order (`order`, then their gates in the
+// same order): each workgroup takes the
 // next kIluBlock rows by ticket until none is left, so the grid bounds the
 // rows in flight.
 template <bool FWD>
@@ -260,7 +366,7 @@ __global__ __launch_bounds__(kIluBlock) void k_lu_sweep(const int *__restrict__ 
     const int t0 = ticket * kIluBlock;
     if (t0 >= n) return;
     const int t = t0 + (int)threadIdx.x;
-    if (t < n) sweep_row<FWD>(order[t], rows, cols, diag, ilu, src, dst, sync);
+    if (t < n) sweep_row<FWD>(order[t], order[n + t], rows, cols, diag, ilu, src, dst, sync);
   }
 }
 
@@ -305,7 +411,9 @@ void fill_round(int n, const std::vector<int> &R, const std::vector<int> &K, con
 
 // Rows grouped by dependency level (forward: over the lower part in row
 // order; backward: over the upper part in reverse row order), ascending row
-// index inside a level.
+// index inside a level; after the n rows of `order`, each one's gate in the
+// sweep: of the entries whose level is at least two below the row's, one of
+// the highest level (-1: none).
 void levels(int n, const std::vector<int> &R, const std::vector<int> &K, const std::vector<int> &D, bool lower,
             std::vector<int> &order, std::vector<int> &off) {
   std::vector<int> lev((size_t)n, 0);
@@ -328,9 +436,21 @@ void levels(int n, const std::vector<int> &R, const std::vector<int> &K, const s
   off.assign((size_t)top + 2, 0);
   for (int i = 0; i < n; ++i) off[lev[i] + 1]++;
   for (int l = 0; l <= top; ++l) off[l + 1] += off[l];
-  order.assign((size_t)n, 0);
+  order.assign(2 * (size_t)n, 0);
   std::vector<int> pos(off.begin(), off.end() - 1);
-  for (int i = 0; i < n; ++i) order[pos[lev[i]]++] = i;
+  for (int i = 0; i < n; ++i) {
+    const int t = pos[lev[i]]++;
+    order[t] = i;
+    int gate = -1, best = -1;
+    for (int j = lower ? R[i] : D[i] + 1; j < (lower ? D[i] : R[i + 1]); ++j) {
+      const int l = lev[K[j]];
+      if (l <= lev[i] - 2 && l > best) {
+        best = l;
+        gate = K[j];
+      }
+    }
+    order[(size_t)n + t] = gate;
+  }
 }
 
 }  // namespace
@@ -343,8 +463,8 @@ void ilu_release(ehip_system *s) {
     dfree(s, s->ilu_amap, sizeof(int) * (size_t)s->nnz);
   }
   dfree(s, s->ilu, sizeof(double) * (size_t)s->ilu_nnz);
-  dfree(s, s->ilu_lord, sizeof(int) * (size_t)s->n);
-  dfree(s, s->ilu_uord, sizeof(int) * (size_t)s->n);
+  dfree(s, s->ilu_lord, sizeof(int) * 2 * (size_t)s->n);
+  dfree(s, s->ilu_uord, sizeof(int) * 2 * (size_t)s->n);
   dfree(s, s->ilu_y, sizeof(double) * (size_t)s->n);
   dfree(s, s->ilu_sync, sizeof(int) * 4);
   s->ilu_y = nullptr;
@@ -388,13 +508,13 @@ int ilu_setup(ehip_system *s, int order) {
   int rc;
   s->ilu_nnz = (int64_t)K.size();
   if ((rc = dmalloc(s, (void **)&s->ilu, sizeof(double) * (size_t)s->ilu_nnz)) ||
-      (rc = dmalloc(s, (void **)&s->ilu_lord, sizeof(int) * (size_t)n)) ||
-      (rc = dmalloc(s, (void **)&s->ilu_uord, sizeof(int) * (size_t)n)) ||
+      (rc = dmalloc(s, (void **)&s->ilu_lord, sizeof(int) * 2 * (size_t)n)) ||
+      (rc = dmalloc(s, (void **)&s->ilu_uord, sizeof(int) * 2 * (size_t)n)) ||
       (rc = dmalloc(s, (void **)&s->ilu_y, sizeof(double) * (size_t)n)) ||
       (rc = dmalloc(s, (void **)&s->ilu_sync, sizeof(int) * 4)))
     return rc;
-  EHIP_HIP_TRY(hipMemcpy(s->ilu_lord, lord.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  EHIP_HIP_TRY(hipMemcpy(s->ilu_uord, uord.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+  EHIP_HIP_TRY(hipMemcpy(s->ilu_lord, lord.data(), sizeof(int) * 2 * (size_t)n, hipMemcpyHostToDevice));
+  EHIP_HIP_TRY(hipMemcpy(s->ilu_uord, uord.data(), sizeof(int) * 2 * (size_t)n, hipMemcpyHostToDevice));
   EHIP_HIP_TRY(hipMemset(s->ilu_sync, 0, sizeof(int) * 4));
   if (order > 0) {
     // the matrix's nonzeros inside the ILU rows (a subset of them, both sorted)
@@ -420,6 +540,8 @@ int ilu_setup(ehip_system *s, int order) {
     s->ilu_cols = s->cols;
     s->ilu_diag = s->diag;
   }
+  s->ilu_maxrow = 0;
+  for (int i = 0; i < n; ++i) s->ilu_maxrow = std::max(s->ilu_maxrow, R[i + 1] - R[i]);
   s->ilu_loff = std::move(loff);
   s->ilu_uoff = std::move(uoff);
   s->ilu_order = order;
@@ -440,9 +562,18 @@ int ilu_factor(ehip_system *s) {
   const std::vector<int> &off = s->ilu_loff;
   for (size_t l = 0; l + 1 < off.size(); ++l) {
     const int cnt = off[l + 1] - off[l];
-    if (cnt > 0)
-      hipLaunchKernelGGL(k_ilu_rows, dim3(level_grid(cnt)), dim3(kIluBlock), 0, s->stream, s->ilu_rows, s->ilu_cols,
-                         s->ilu_diag, s->ilu, s->ilu_lord, off[l], off[l + 1]);
+    if (cnt <= 0) continue;
+    // one wave per row, its entries in registers; longer rows one lane per row
+    const dim3 gw((cnt + kIluBlock / 64 - 1) / (kIluBlock / 64)), bs(kIluBlock);
+    if (s->ilu_maxrow <= 64)
+      hipLaunchKernelGGL(k_ilu_rows_wave<1>, gw, bs, 0, s->stream, s->ilu_rows, s->ilu_cols, s->ilu_diag, s->ilu,
+                         s->ilu_lord, off[l], off[l + 1]);
+    else if (s->ilu_maxrow <= 192)
+      hipLaunchKernelGGL(k_ilu_rows_wave<3>, gw, bs, 0, s->stream, s->ilu_rows, s->ilu_cols, s->ilu_diag, s->ilu,
+                         s->ilu_lord, off[l], off[l + 1]);
+    else
+      hipLaunchKernelGGL(k_ilu_rows, dim3(level_grid(cnt)), bs, 0, s->stream, s->ilu_rows, s->ilu_cols, s->ilu_diag,
+                         s->ilu, s->ilu_lord, off[l], off[l + 1]);
   }
   hipLaunchKernelGGL(k_ilu_invdiag, dim3(std::min(2048, (n + 255) / 256)), dim3(256), 0, s->stream, n, s->ilu_diag,
                      s->ilu);
