@@ -10,7 +10,12 @@
 // registers, the matrix in the L2 of its XCD, and the vector that the SpMV
 // gathers in the workgroup's LDS (its 1024 rows and a halo of the
 // bandwidth).  What is left of an iteration are its two exchanges between
-// workgroups: partial sums, and the halo's new entries with the second one.
+// workgroups (four in BiCGStab): partial sums, and the halo's new entries with
+// the second one.  Per iteration, launched and resident: 17^3 Hex8 in HUTI's
+// order 27 and 10 us, 55^3 Tet4 (SELL-64) one-SpMV order 20 and 17 us, 301^2
+// Quad4 BiCGStab in HUTI's order 50 and 23 us.  Of the 10 us, measured by the
+// kernel's own clock, some 5 are the exchanges' trips to the memory the XCDs
+// share, the rest the row sums and the reductions inside the workgroup.
 //
 // Exchanges.  A workgroup publishes its partial sums as 64-bit words that
 // carry the exchange's number beside 32 bits of the value, with agent-scope
@@ -95,6 +100,36 @@ __device__ __forceinline__ bool seen(const Word *p, unsigned e, float &v) {
 
 }  // namespace
 
+namespace {
+
+// wave_sum (reduce.h) with the last four steps as rotations inside rows of
+// 16 lanes instead of cross-lane LDS operations: after the steps of 32 and
+// 16 lanes the sums repeat every 16, 8, ... lanes, so adding the lane 8, 4,
+// 2, 1 further on adds the same two numbers (the same bits).
+template <int CTRL>
+__device__ __forceinline__ float rotated(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double rotated(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((Word)hi << 32) | lo));
+}
+template <typename T>
+__device__ __forceinline__ T row_wave_sum(T v) {
+  v += __shfl_xor(v, 32, kWave);
+  v += __shfl_xor(v, 16, kWave);
+  v += rotated<0x128>(v);  // row_ror:8
+  v += rotated<0x124>(v);
+  v += rotated<0x122>(v);
+  v += rotated<0x121>(v);
+  return v;
+}
+
+}  // namespace
+
 // The matrix in the layout the launched SpMV reads: slice-shared offsets
 // (SHO), or SELL-64 with 16-bit columns, FP64 values pair-packed.
 enum ResFmt { RES_SHO, RES_SELL };
@@ -129,30 +164,35 @@ __device__ __forceinline__ int spmv_slot(int g, int ngroups) {
   while ((long long)ngroups * xcd / 8 > g) --xcd;
   return (g - (int)((long long)ngroups * xcd / 8)) * 8 + xcd;
 }
+// The slot of the group that this thread publishes, -1 where it has no rows;
+// found once, as it takes a division.
+__device__ __forceinline__ int group_slot(int ngroups) {
+  const int g = (int)blockIdx.x * 4 + ((int)threadIdx.x & 3);
+  return g < ngroups ? spmv_slot(g, ngroups) : -1;
+}
 __device__ __forceinline__ bool slot_used(int b, int ngroups) {
   const int xcd = b & 7, lb = b >> 3;
   return (int)((long long)ngroups * xcd / 8) + lb < (int)((long long)ngroups * (xcd + 1) / 8);
 }
 
 // A row's matrix entries.  SHO: the values in registers (at most KW of
-// them), the slice's offset list read with scalar loads.  SELL: read from
-// the L2 in every product.
+// them), the slice's offset list in scalar loads of many offsets each (one
+// by one, each cost its latency: 5.7 us of a 15 us iteration at 17^3 Hex8).
+// SELL: read from the L2 in every product.
 template <typename T, ResFmt F, int KW>
 struct ResRow {
   T v[F == RES_SHO ? KW : 1];
-  unsigned m;                     // SHO: the row's own entries (FP32: all of the list's)
-  const int *__restrict__ t;
-  int wd, rl, p0, len;
+  unsigned m;  // SHO: the row's own entries (FP32: all of the list's)
+  int wd, p0, len;
   __device__ __forceinline__ void load(const ResArgs<T> &a, int sl, int lane) {
     constexpr bool kF32 = sizeof(T) == 4;
     const int r = sl * 64 + lane;
-    rl = min(r, a.n - 1);
+    const int rl = min(r, a.n - 1);
     const bool live = sl < a.nslice;
     p0 = live ? a.off[sl] : 0;
     const int width = live ? a.off[sl + 1] - p0 : 0;
     if constexpr (F == RES_SHO) {
       wd = width >> 6;
-      t = a.tab + (p0 >> 6);
       m = kF32 ? (wd >= 32 ? ~0u : (1u << wd) - 1u) : (r < a.n ? a.mask[rl] : 0u);
 #pragma unroll
       for (int k = 0; k < KW; ++k) v[k] = k < wd ? a.vals[p0 + 64 * k + lane] : (T)0;
@@ -180,9 +220,12 @@ struct ResRow {
       }
     };
     if constexpr (F == RES_SHO) {
+      // KW offsets in a few wide scalar loads: past the slice's list they are
+      // the next slices' (or the padding's), inside the window all the same
+      const int *__restrict__ t = a.tab + (p0 >> 6);
+      const int own = (int)threadIdx.x + a.halo;
 #pragma unroll
-      for (int k = 0; k < KW; ++k)
-        if (k < wd) add(v[k], min(max(rl + t[k], 0), a.n - 1) - wb, (m >> k) & 1u);
+      for (int k = 0; k < KW; ++k) add(v[k], own + t[k], (m >> k) & 1u);
     } else if constexpr (!kF32) {
       constexpr int U = 4;
       const int b = sl < a.nslice ? a.tab[sl] - wb : 0;
@@ -234,23 +277,24 @@ struct ResShared {
 };
 
 // Sum over a 256-row group's rows of val, as the launched SpMV's workgroup
-// publishes it (block_publish with 256 threads), for the workgroup's four groups.
+// publishes it (block_publish with 256 threads), for the workgroup's four
+// groups; slot: this thread's (group_slot).
 template <typename T, int NV>
-__device__ __forceinline__ void publish_groups(const ResArgs<T> &a, ResShared<T> &sh, Word *w, unsigned e,
+__device__ __forceinline__ void publish_groups(const ResArgs<T> &a, ResShared<T> &sh, Word *w, unsigned e, int slot,
                                                const T (&val)[NV]) {
   const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const T s = wave_sum(val[k]);
+    const T s = row_wave_sum(val[k]);
     if (lane == 0) sh.wave[16 * k + wv] = s;
   }
   __syncthreads();
   if (threadIdx.x < 4 * NV) {
-    const int g = blockIdx.x * 4 + ((int)threadIdx.x & 3), k = (int)threadIdx.x >> 2;
-    if (g < a.ngroups) {
+    const int k = (int)threadIdx.x >> 2;
+    if (slot >= 0) {
       T t = (T)0;
       for (int i = 0; i < 4; ++i) t += sh.wave[16 * k + 4 * ((int)threadIdx.x & 3) + i];
-      publish(w + ((size_t)k * a.spmv_grid + spmv_slot(g, a.ngroups)) * kWords<T>, e, t);
+      publish(w + ((size_t)k * a.spmv_grid + slot) * kWords<T>, e, t);
     }
   }
 }
@@ -275,7 +319,7 @@ __device__ __forceinline__ void publish_rows(const ResArgs<T> &a, ResShared<T> &
     }
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const T s = wave_sum(acc[k]);
+      const T s = row_wave_sum(acc[k]);
       if (lane == 0) sh.wave[16 * k + wv] = s;
     }
   }
@@ -292,13 +336,14 @@ __device__ __forceinline__ void publish_rows(const ResArgs<T> &a, ResShared<T> &
 // its words in flight, and adds them in block_reduce_all's order (256
 // threads).  False: someone gave up.
 template <typename T, int NV, bool SPMV>
-__device__ __forceinline__ bool gather(const ResArgs<T> &a, ResShared<T> &sh, const Word *w, unsigned e, T (&tot)[NV]) {
+__device__ __forceinline__ bool gather(const ResArgs<T> &a, ResShared<T> &sh, const Word *w, unsigned e, bool used,
+                                       T (&tot)[NV]) {
   const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int g = SPMV ? a.spmv_grid : a.vec_grid;  // at most 1024
   T v[NV];
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = (T)0;
-  if (tid < g && (SPMV ? slot_used(tid, a.ngroups) : tid < (int)gridDim.x)) {
+  if (SPMV ? used : tid < (int)gridDim.x) {
     for (int spins = 0;; ++spins) {
       bool all = true;
 #pragma unroll
@@ -321,7 +366,7 @@ __device__ __forceinline__ bool gather(const ResArgs<T> &a, ResShared<T> &sh, co
       T s = (T)0;
 #pragma unroll
       for (int u = 0; u < 4; ++u) s += sh.part[k][tid + 256 * u];
-      s = wave_sum(s);
+      s = row_wave_sum(s);
       if (lane == 0) sh.tot[k][wv] = s;
     }
   }
@@ -339,20 +384,20 @@ __device__ __forceinline__ bool gather(const ResArgs<T> &a, ResShared<T> &sh, co
 // columns, kHaloU columns of a thread in flight.
 constexpr int kHaloU = 6;
 template <typename T, int NE, class Fn>
-__device__ __forceinline__ void halo_columns(int wb, int nlow, int re, int nhalo, const T *e0, const T *e1, Fn f) {
+__device__ __forceinline__ void halo_columns(int lo, int nlow, int re, int nhalo, const T *e0, const T *e1, Fn f) {
   for (int i0 = (int)threadIdx.x; i0 < nhalo; i0 += kHaloU * kResRows) {
     T v[NE][kHaloU];
 #pragma unroll
     for (int u = 0; u < kHaloU; ++u) {
       const int i = min(i0 + u * kResRows, nhalo - 1);
-      const int c = i < nlow ? wb + i : re + (i - nlow);
+      const int c = i < nlow ? lo + i : re + (i - nlow);
       v[0][u] = ld_agent(e0 + c);
       if constexpr (NE > 1) v[1][u] = ld_agent(e1 + c);
     }
 #pragma unroll
     for (int u = 0; u < kHaloU; ++u) {
       const int i = i0 + u * kResRows;
-      if (i < nhalo) f(i < nlow ? wb + i : re + (i - nlow), v[0][u], v[NE - 1][u]);
+      if (i < nhalo) f(i < nlow ? lo + i : re + (i - nlow), v[0][u], v[NE - 1][u]);
     }
   }
 }
@@ -370,9 +415,10 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
   const int R0 = (int)blockIdx.x * kResRows, r = R0 + tid, rl = min(r, a.n - 1);
   const bool ok = r < a.n;
   const int sl = __builtin_amdgcn_readfirstlane(R0 / 64 + (tid >> 6));
-  const int wb = max(R0 - a.halo, 0), we = min(R0 + kResRows + a.halo, a.n), own = r - wb;
-  const int re = min(R0 + kResRows, a.n);  // the halo: [wb, R0) and [re, we)
-  const int nlow = R0 - wb, nhalo = nlow + (we - re);
+  const int wb = R0 - a.halo, own = tid + a.halo;  // the window's first column, this row's place
+  const int lo = max(wb, 0), re = min(R0 + kResRows, a.n);  // the halo: [lo, R0) and [re, we)
+  const int we = min(R0 + kResRows + a.halo, a.n);
+  const int nlow = R0 - lo, nhalo = nlow + (we - re);
   T *win = reinterpret_cast<T *>(lds);     // z, or p with FAITHFUL
   T *winx = win + (kResRows + 2 * a.halo); // x (FAITHFUL)
   T x = a.v.x[rl], p = a.v.p[rl], q = a.v.q[rl], rr = a.v.r[rl], z = a.v.z[rl];
@@ -386,10 +432,16 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
   }
   {
     const T *src = FAITHFUL ? a.v.p : a.v.z;
-    for (int i = wb + tid; i < we; i += kResRows) win[i - wb] = src[i];
+    for (int i = tid; i < kResRows + 2 * a.halo; i += kResRows) {
+      const int c = wb + i;
+      win[i] = c >= 0 && c < a.n ? src[c] : (T)0;
+      if constexpr (FAITHFUL) winx[i] = (T)0;
+    }
   }
   __syncthreads();
   double *const hist = blockIdx.x == 0 ? a.hist : nullptr;
+  const int slot = group_slot(a.ngroups);
+  const bool used = tid < a.spmv_grid && slot_used(tid, a.ngroups);
   unsigned e = 1;
   T sx[FAITHFUL ? 2 : 1];
   bool lost = false;
@@ -399,13 +451,13 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
     q = s[0];
     T acc[3] = {(T)0, (T)0, (T)0};
     if (ok) acc[0] += p * q;
-    publish_groups<T, 3>(a, sh, a.w1, e, acc);
+    publish_groups<T, 3>(a, sh, a.w1, e, slot, acc);
   }
   if (!sh.st.done) for (bool first = true;; first = false) {
     T pq;
     if constexpr (FAITHFUL) {
       T tot[3];
-      if (!gather<T, 3, true>(a, sh, a.w1, e, tot)) { lost = true; break; }
+      if (!gather<T, 3, true>(a, sh, a.w1, e, used, tot)) { lost = true; break; }
       if (!first) {
         T two[2] = {tot[1], tot[2]};
         EpiCgResidual<T> f{a.v, &sh.st, nullptr, 0, nullptr, hist, nullptr, 0, (T)0, a.du};
@@ -421,9 +473,9 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
       p = z + beta * p;
       T acc[1] = {(T)0};
       if (ok) acc[0] += p * q;
-      publish_groups<T, 1>(a, sh, a.w1, e, acc);
+      publish_groups<T, 1>(a, sh, a.w1, e, slot, acc);
       T tot[1];
-      if (!gather<T, 1, true>(a, sh, a.w1, e, tot)) { lost = true; break; }
+      if (!gather<T, 1, true>(a, sh, a.w1, e, used, tot)) { lost = true; break; }
       pq = tot[0];
     }
     ++e;
@@ -437,15 +489,15 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
     }
     sh.part[0][tid] = rr;
     sh.part[1][tid] = z;
-    if constexpr (!FAITHFUL) win[own] = z;
+    if (!FAITHFUL && ok) win[own] = z;
     __syncthreads();
     if constexpr (FAITHFUL) {
       publish_rows<T, 1>(a, sh, a.w2, e);
       T rn[1];
-      if (!gather<T, 1, false>(a, sh, a.w2, e, rn)) { lost = true; break; }
+      if (!gather<T, 1, false>(a, sh, a.w2, e, used, rn)) { lost = true; break; }
       const T beta = rn[0] / sh.st.rho;
       p = z + beta * p;
-      halo_columns<T, 2>(wb, nlow, re, nhalo, a.ez, a.ex, [&](int c, T zc, T xc) {
+      halo_columns<T, 2>(lo, nlow, re, nhalo, a.ez, a.ex, [&](int c, T zc, T xc) {
         win[c - wb] = zc + beta * win[c - wb];
         winx[c - wb] = xc;
       });
@@ -470,17 +522,17 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
         acc[2] += ui * ui;
       }
       ++e;
-      publish_groups<T, 3>(a, sh, a.w1, e, acc);
+      publish_groups<T, 3>(a, sh, a.w1, e, slot, acc);
     } else {
       publish_rows<T, 2>(a, sh, a.w2, e);
       T tot[2];
-      if (!gather<T, 2, false>(a, sh, a.w2, e, tot)) { lost = true; break; }
+      if (!gather<T, 2, false>(a, sh, a.w2, e, used, tot)) { lost = true; break; }
       if (tid == 0) {
         sh.st.pq = pq;
         sh.st.alpha = alpha;
       }
       FinCgFast2<T>{&sh.st, nullptr, 0, hist}.finish(tot);
-      halo_columns<T, 1>(wb, nlow, re, nhalo, a.ez, a.ez, [&](int c, T zc, T) { win[c - wb] = zc; });
+      halo_columns<T, 1>(lo, nlow, re, nhalo, a.ez, a.ez, [&](int c, T zc, T) { win[c - wb] = zc; });
       __syncthreads();
       if (sh.st.done) break;
       ++e;
@@ -513,9 +565,10 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
   const int R0 = (int)blockIdx.x * kResRows, r = R0 + tid, rl = min(r, a.n - 1);
   const bool ok = r < a.n;
   const int sl = __builtin_amdgcn_readfirstlane(R0 / 64 + (tid >> 6));
-  const int wb = max(R0 - a.halo, 0), we = min(R0 + kResRows + a.halo, a.n), own = r - wb;
-  const int re = min(R0 + kResRows, a.n);
-  const int nlow = R0 - wb, nhalo = nlow + (we - re);
+  const int wb = R0 - a.halo, own = tid + a.halo;
+  const int lo = max(wb, 0), re = min(R0 + kResRows, a.n);
+  const int we = min(R0 + kResRows + a.halo, a.n);
+  const int nlow = R0 - lo, nhalo = nlow + (we - re);
   T *win = reinterpret_cast<T *>(lds);      // t1v and t2v in turn
   T *winx = win + (kResRows + 2 * a.halo);  // x (FAITHFUL)
   T x = a.v.x[rl], p = a.v.p[rl], v = a.v.v[rl], rr = a.v.r[rl], t1 = a.v.t1v[rl];
@@ -527,9 +580,15 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
     sh.st = *a.st;
     sh.fail = 0;
   }
-  for (int i = wb + tid; i < we; i += kResRows) win[i - wb] = a.v.t1v[i];
+  for (int i = tid; i < kResRows + 2 * a.halo; i += kResRows) {
+    const int c = wb + i;
+    win[i] = c >= 0 && c < a.n ? a.v.t1v[c] : (T)0;
+    if constexpr (FAITHFUL) winx[i] = (T)0;
+  }
   __syncthreads();
   double *const hist = blockIdx.x == 0 ? a.hist : nullptr;
+  const int slot = group_slot(a.ngroups);
+  const bool used = tid < a.spmv_grid && slot_used(tid, a.ngroups);
   unsigned e = 0;
   bool lost = false;
   if (!sh.st.done) for (bool first = true;; first = false) {
@@ -546,17 +605,17 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
         const T ui = ti / d;
         acc[2] += ui * ui;
       }
-      publish_groups<T, 3>(a, sh, a.w1, e, acc);
+      publish_groups<T, 3>(a, sh, a.w1, e, slot, acc);
     } else {
       T s[1];
       row.template sums<1>(a, sl, lane, wb, win, win, s);
       v = s[0];
       T acc[3] = {(T)0, (T)0, (T)0};
       if (ok) acc[0] += rt * v;
-      publish_groups<T, 3>(a, sh, a.w1, e, acc);
+      publish_groups<T, 3>(a, sh, a.w1, e, slot, acc);
     }
     T rv[3];
-    if (!gather<T, 3, true>(a, sh, a.w1, e, rv)) { lost = true; break; }
+    if (!gather<T, 3, true>(a, sh, a.w1, e, used, rv)) { lost = true; break; }
     if (FAITHFUL && !first) {
       T two[2] = {rv[1], rv[2]};
       EpiBiResidual<T> f{a.v, &sh.st, nullptr, 0, nullptr, hist, (T)0, (T)0, a.du};
@@ -570,15 +629,15 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
     if (ok) st_agent(a.ez + r, t2);
     sh.part[0][tid] = s;
     sh.part[1][tid] = s;
-    win[own] = t2;
+    if (ok) win[own] = t2;
     __syncthreads();
     ++e;
     publish_rows<T, 1>(a, sh, a.w2, e);
     T ss[1];
-    if (!gather<T, 1, false>(a, sh, a.w2, e, ss)) { lost = true; break; }
+    if (!gather<T, 1, false>(a, sh, a.w2, e, used, ss)) { lost = true; break; }
     if (tid == 0) sh.st.alpha = alpha;
     FinSnorm<T>{&sh.st, nullptr, 0}.finish(ss);
-    halo_columns<T, 1>(wb, nlow, re, nhalo, a.ez, a.ez, [&](int c, T tc, T) { win[c - wb] = tc; });
+    halo_columns<T, 1>(lo, nlow, re, nhalo, a.ez, a.ez, [&](int c, T tc, T) { win[c - wb] = tc; });
     __syncthreads();
     if (sh.st.snorm_exit) {
       x = x + alpha * t1;
@@ -598,10 +657,10 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
         acc[1] += tv * tv;
       }
       ++e;
-      publish_groups<T, 2>(a, sh, a.w1, e, acc);
+      publish_groups<T, 2>(a, sh, a.w1, e, slot, acc);
     }
     T tt[2];
-    if (!gather<T, 2, true>(a, sh, a.w1, e, tt)) { lost = true; break; }
+    if (!gather<T, 2, true>(a, sh, a.w1, e, used, tt)) { lost = true; break; }
     const T omega = tt[0] / tt[1];
     x = x + alpha * t1 + omega * t2;
     rr = s - omega * tv;
@@ -617,7 +676,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
     ++e;
     publish_rows<T, 2>(a, sh, a.w2, e);
     T rn[2];
-    if (!gather<T, 2, false>(a, sh, a.w2, e, rn)) { lost = true; break; }
+    if (!gather<T, 2, false>(a, sh, a.w2, e, used, rn)) { lost = true; break; }
     if (tid == 0) {
       sh.st.ts = tt[0];
       sh.st.tt = tt[1];
@@ -629,10 +688,10 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
     const T beta = FAITHFUL ? (sh.st.rho_new * alpha) / (sh.st.rho * omega) : sh.st.beta;
     p = rr + beta * w;
     t1 = p / dg;
-    halo_columns<T, 2>(wb, nlow, re, nhalo, a.er, a.ew,
+    halo_columns<T, 2>(lo, nlow, re, nhalo, a.er, a.ew,
                        [&](int c, T rc, T wc) { win[c - wb] = (rc + beta * wc) / a.v.dg[c]; });
     if constexpr (FAITHFUL)
-      halo_columns<T, 1>(wb, nlow, re, nhalo, a.ex, a.ex, [&](int c, T xc, T) { winx[c - wb] = xc; });
+      halo_columns<T, 1>(lo, nlow, re, nhalo, a.ex, a.ex, [&](int c, T xc, T) { winx[c - wb] = xc; });
     if (ok) {
       win[own] = t1;
       if constexpr (FAITHFUL) winx[own] = x;

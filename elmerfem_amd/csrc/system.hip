@@ -467,6 +467,7 @@ static int build_sho(ehip_system *s, const std::vector<int> &c0, int64_t sell_to
   for (int sl = 0; sl < S; ++sl)
     std::copy(tab.begin() + (size_t)sl * kMax, tab.begin() + (size_t)sl * kMax + len[sl],
               ctab.begin() + off[sl] / (64 * D));
+  ctab.resize(ctab.size() + kMax, 0);  // readers take a fixed number of offsets from any slice's first
   int rc;
   if ((rc = dmalloc(s, (void **)&s->sho_off, sizeof(int) * off.size())) ||
       (rc = dmalloc(s, (void **)&s->sho_tab, sizeof(int) * ctab.size())) ||
