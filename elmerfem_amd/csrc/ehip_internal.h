@@ -349,8 +349,8 @@ inline int sho_nt_from(int nslice, int64_t bytes, int64_t n, int elem) {
 }
 
 // Smallest FP64 values copy (bytes) that takes the half storage: below it
-// the SpMV is bound by launches, not by the matrix stream, and the check of
-// the values costs more than it gives.
+// the copy fits the L2s (8 x 4 MB with the vectors), so halving its stream
+// gains nothing, and the system is small enough for the resident loops.
 constexpr int64_t kSymMinBytes = 16ll << 20;
 
 inline int sell_grid(const ehip_system *s) {

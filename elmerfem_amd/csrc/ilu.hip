@@ -74,8 +74,9 @@ __global__ __launch_bounds__(kIluBlock) void k_ilu_rows(const int *__restrict__ 
 // k's upper entries to the lanes, so an entry takes its subtractions in the
 // same order (the same bits).  One lane per row walked both rows entry by
 // entry, a dependent memory latency each: 158 us a level at 64^3 Hex8,
-// against kAhead rows k in flight here, their bounds loaded for all of them
-// at once: 12 us (the launch included).
+// against 21 us with kAhead rows k in flight, their bounds loaded for all of
+// them at once.  Rows of 65 to 192 entries (ILU(1)) take three entries to a
+// lane; beyond that the registers would not hold row and rows ahead.
 constexpr int kAhead = 4;
 template <int NC>
 __global__ __launch_bounds__(kIluBlock) void k_ilu_rows_wave(const int *__restrict__ rows, const int *__restrict__ cols,
@@ -272,8 +273,8 @@ __global__ void k_lu_pending(int n, double *y, double *z, int *sync) {
 // polls every entry that is still pending, so the value that turns ready
 // last arrives with the poll that finds it ready.  (Polling the entry of the
 // last level alone and loading the others after it cost a memory trip more
-// for every level of the critical path: 64^3 Hex8 ILU(0), 449 levels, 1.52 ms
-// a sweep then, 1.30 ms so.)  All of it is in one loop, the row published
+// for every level of the critical path: 64^3 Hex8 ILU(0), 449 levels, 1.45 ms
+// forward and 1.60 ms backward then, 1.31 and 1.52 ms so.)  All of it is in one loop, the row published
 // inside it.  The loop ends for the whole wave at once (when every lane is
 // done): with a per-lane exit the compiler may move the publishing store
 // after the loop, where a lane publishes only once every lane of its wave is

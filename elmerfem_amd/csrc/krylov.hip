@@ -688,30 +688,17 @@ struct EpiBiV {
   }
 };
 
-// Calls f(i) for this thread's rows of a vector kernel whose workgroups take
-// tiles of kVI * kVecBlock consecutive rows (as CgTile: the sums' grouping
-// that the resident loop of resident.hip repeats).
-template <class F>
-__device__ __forceinline__ void for_tiles(int n, F f) {
-  for (int base = blockIdx.x * kVecBlock * kVI; base < n; base += gridDim.x * kVecBlock * kVI)
-#pragma unroll
-    for (int k = 0; k < kVI; ++k) {
-      const int i = base + k * kVecBlock + (int)threadIdx.x;
-      if (i < n) f(i);
-    }
-}
-
 template <typename T>
 __global__ __launch_bounds__(kVecBlock) void k_bi_s(int n, Vecs<T> v, KStateT<T> *st, T *partials) {
   if (solve_done(st)) return;
   const T alpha = st->alpha;
   T acc[1] = {(T)0};
-  for_tiles(n, [&](int i) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const T si = v.r[i] - alpha * v.v[i];
     v.sv[i] = si;
     v.t2v[i] = si / v.dg[i];
     acc[0] += si * si;
-  });
+  }
   block_publish<T, 1>(acc, partials, gridDim.x);
 }
 
@@ -756,13 +743,13 @@ __global__ __launch_bounds__(kVecBlock) void k_bi_xr(int n, Vecs<T> v, KStateT<T
   if (solve_done(st)) return;
   const T alpha = st->alpha, omega = st->omega;
   T acc[2] = {(T)0, (T)0};
-  for_tiles(n, [&](int i) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     v.x[i] = v.x[i] + alpha * v.t1v[i] + omega * v.t2v[i];
     const T ri = v.sv[i] - omega * v.t[i];
     v.r[i] = ri;
     acc[0] += v.rtld[i] * ri;
     acc[1] += ri * ri;
-  });
+  }
   (void)fast;
   (void)hist;
   block_publish<T, 2>(acc, partials, gridDim.x);
@@ -1447,6 +1434,7 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
     }
   } else {
     resident = s->resident_on && resident_fits<T>(s, c.mode == EHIP_FAITHFUL);
+    const int gb = bi_grid(n);
     hipLaunchKernelGGL(k_bi_start<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st, part);
     fin<T>(s, FinBiStart<T>{st, part, g}, g, st);
     for (int it_seen = iter0;; it_seen = hst->iter) {
@@ -1459,15 +1447,15 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
         launch_epi<T>(s, plan, vals, v.t1v, e3, st);
         if (c.prof) prof_end(s);
         fin<T>(s, e3, epi_grid<T>(s, plan), st);
-        hipLaunchKernelGGL(k_bi_s<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st, part);
-        fin<T>(s, FinSnorm<T>{st, part, g}, g, st);
+        hipLaunchKernelGGL(k_bi_s<T>, dim3(gb), dim3(kVecBlock), 0, s->stream, n, v, st, part);
+        fin<T>(s, FinSnorm<T>{st, part, gb}, gb, st);
         hipLaunchKernelGGL(k_bi_snorm_exit<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st);
         hipLaunchKernelGGL(k_bi_snorm_mark<T>, dim3(1), dim3(1), 0, s->stream, st);
         EpiBiT<T> e6{v, st, part, pg, &st->ticket[0], 1};
         launch_epi_fin<T>(s, plan, vals, v.t2v, e6, st);
-        hipLaunchKernelGGL(k_bi_xr<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st, part,
+        hipLaunchKernelGGL(k_bi_xr<T>, dim3(gb), dim3(kVecBlock), 0, s->stream, n, v, st, part,
                            c.mode == EHIP_FAST ? 1 : 0, c.hist);
-        fin<T>(s, FinBiXr<T>{st, part, g, c.mode == EHIP_FAST ? 1 : 0, c.hist}, g, st);
+        fin<T>(s, FinBiXr<T>{st, part, gb, c.mode == EHIP_FAST ? 1 : 0, c.hist}, gb, st);
         c.spmv += 2;
         if (c.mode == EHIP_FAITHFUL) {
           EpiBiResidual<T> e8{v, st, part, pg, &st->ticket[2], c.hist, (T)0, (T)0, du};
@@ -2150,10 +2138,10 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   const int n = s->n;
   int rc;
   if ((rc = ensure_state(s))) return rc;
-  // half storage only where the method needs a symmetric matrix anyway
-  // ... of 3-DOF node blocks only in FP64: an entry below the diagonal takes
-  // its three values from three places there, and FP32 lost by it what the
-  // halved stream gave (63^3 Hex8: 37 us full, 42 us half; FP64 112 and 84)
+  // half storage only where the method needs a symmetric matrix anyway, and
+  // of 3-DOF node blocks only in FP64: an entry below the diagonal takes its
+  // three values from three places there, and FP32 lost by that more than
+  // the halved stream gave (63^3 Hex8: 37 us full, 42 us half; FP64 112, 84)
   s->sym_on = p->method == EHIP_CG && p->precond < EHIP_PRECOND_ILU0 &&
               (s->sho_d == 1 || p->precision == EHIP_FP64);
   // one launch per sequence where the rows fit the chip (not for callers

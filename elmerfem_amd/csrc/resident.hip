@@ -28,8 +28,8 @@
 // one between and so has read them.
 //
 // Bits.  Sums are grouped as the launched kernels group them -- the SpMV's
-// partials per 256 rows, the vector step's per 1024 rows with four rows to
-// a thread, the totals over 256 threads -- and the scalar updates and
+// partials per 256 rows, CG's vector step's per 1024 rows with four rows to
+// a thread, BiCGStab's per 256 rows, the totals over 256 threads -- and the scalar updates and
 // stopping tests are the same functors (cg_steps.h), so a solve gives the
 // same bits either way.
 //
@@ -227,7 +227,7 @@ struct ResRow {
 #pragma unroll
       for (int k = 0; k < KW; ++k) add(v[k], own + t[k], (m >> k) & 1u);
     } else if constexpr (!kF32) {
-      constexpr int U = 4;
+      constexpr int U = 8;
       const int b = sl < a.nslice ? a.tab[sl] - wb : 0;
       for (int k0 = 0; k0 < wd; k0 += U) {
         T v0[U], v1[U];
@@ -278,9 +278,9 @@ struct ResShared {
 
 // Sum over a 256-row group's rows of val, as the launched SpMV's workgroup
 // publishes it (block_publish with 256 threads), for the workgroup's four
-// groups; slot: this thread's (group_slot).
+// groups; slot: this thread's, of `stride` to a value.
 template <typename T, int NV>
-__device__ __forceinline__ void publish_groups(const ResArgs<T> &a, ResShared<T> &sh, Word *w, unsigned e, int slot,
+__device__ __forceinline__ void publish_groups(int stride, ResShared<T> &sh, Word *w, unsigned e, int slot,
                                                const T (&val)[NV]) {
   const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
 #pragma unroll
@@ -288,13 +288,14 @@ __device__ __forceinline__ void publish_groups(const ResArgs<T> &a, ResShared<T>
     const T s = row_wave_sum(val[k]);
     if (lane == 0) sh.wave[16 * k + wv] = s;
   }
+  stores_done();  // the vector entries go before the partial sums
   __syncthreads();
   if (threadIdx.x < 4 * NV) {
     const int k = (int)threadIdx.x >> 2;
     if (slot >= 0) {
       T t = (T)0;
       for (int i = 0; i < 4; ++i) t += sh.wave[16 * k + 4 * ((int)threadIdx.x & 3) + i];
-      publish(w + ((size_t)k * a.spmv_grid + slot) * kWords<T>, e, t);
+      publish(w + ((size_t)k * stride + slot) * kWords<T>, e, t);
     }
   }
 }
@@ -343,7 +344,7 @@ __device__ __forceinline__ bool gather(const ResArgs<T> &a, ResShared<T> &sh, co
   T v[NV];
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = (T)0;
-  if (SPMV ? used : tid < (int)gridDim.x) {
+  if (used) {
     for (int spins = 0;; ++spins) {
       bool all = true;
 #pragma unroll
@@ -451,7 +452,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
     q = s[0];
     T acc[3] = {(T)0, (T)0, (T)0};
     if (ok) acc[0] += p * q;
-    publish_groups<T, 3>(a, sh, a.w1, e, slot, acc);
+    publish_groups<T, 3>(a.spmv_grid, sh, a.w1, e, slot, acc);
   }
   if (!sh.st.done) for (bool first = true;; first = false) {
     T pq;
@@ -473,7 +474,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
       p = z + beta * p;
       T acc[1] = {(T)0};
       if (ok) acc[0] += p * q;
-      publish_groups<T, 1>(a, sh, a.w1, e, slot, acc);
+      publish_groups<T, 1>(a.spmv_grid, sh, a.w1, e, slot, acc);
       T tot[1];
       if (!gather<T, 1, true>(a, sh, a.w1, e, used, tot)) { lost = true; break; }
       pq = tot[0];
@@ -494,7 +495,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
     if constexpr (FAITHFUL) {
       publish_rows<T, 1>(a, sh, a.w2, e);
       T rn[1];
-      if (!gather<T, 1, false>(a, sh, a.w2, e, used, rn)) { lost = true; break; }
+      if (!gather<T, 1, false>(a, sh, a.w2, e, tid < (int)gridDim.x, rn)) { lost = true; break; }
       const T beta = rn[0] / sh.st.rho;
       p = z + beta * p;
       halo_columns<T, 2>(lo, nlow, re, nhalo, a.ez, a.ex, [&](int c, T zc, T xc) {
@@ -522,11 +523,11 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
         acc[2] += ui * ui;
       }
       ++e;
-      publish_groups<T, 3>(a, sh, a.w1, e, slot, acc);
+      publish_groups<T, 3>(a.spmv_grid, sh, a.w1, e, slot, acc);
     } else {
       publish_rows<T, 2>(a, sh, a.w2, e);
       T tot[2];
-      if (!gather<T, 2, false>(a, sh, a.w2, e, used, tot)) { lost = true; break; }
+      if (!gather<T, 2, false>(a, sh, a.w2, e, tid < (int)gridDim.x, tot)) { lost = true; break; }
       if (tid == 0) {
         sh.st.pq = pq;
         sh.st.alpha = alpha;
@@ -589,6 +590,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
   double *const hist = blockIdx.x == 0 ? a.hist : nullptr;
   const int slot = group_slot(a.ngroups);
   const bool used = tid < a.spmv_grid && slot_used(tid, a.ngroups);
+  const int g4 = (int)blockIdx.x * 4 + (tid & 3), group = g4 < a.ngroups ? g4 : -1;
   unsigned e = 0;
   bool lost = false;
   if (!sh.st.done) for (bool first = true;; first = false) {
@@ -605,14 +607,14 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
         const T ui = ti / d;
         acc[2] += ui * ui;
       }
-      publish_groups<T, 3>(a, sh, a.w1, e, slot, acc);
+      publish_groups<T, 3>(a.spmv_grid, sh, a.w1, e, slot, acc);
     } else {
       T s[1];
       row.template sums<1>(a, sl, lane, wb, win, win, s);
       v = s[0];
       T acc[3] = {(T)0, (T)0, (T)0};
       if (ok) acc[0] += rt * v;
-      publish_groups<T, 3>(a, sh, a.w1, e, slot, acc);
+      publish_groups<T, 3>(a.spmv_grid, sh, a.w1, e, slot, acc);
     }
     T rv[3];
     if (!gather<T, 3, true>(a, sh, a.w1, e, used, rv)) { lost = true; break; }
@@ -627,14 +629,15 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
     const T s = rr - alpha * v;
     const T t2 = s / dg;
     if (ok) st_agent(a.ez + r, t2);
-    sh.part[0][tid] = s;
-    sh.part[1][tid] = s;
     if (ok) win[own] = t2;
-    __syncthreads();
     ++e;
-    publish_rows<T, 1>(a, sh, a.w2, e);
+    {
+      T acc[1] = {(T)0};
+      if (ok) acc[0] += s * s;
+      publish_groups<T, 1>(a.vec_grid, sh, a.w2, e, group, acc);
+    }
     T ss[1];
-    if (!gather<T, 1, false>(a, sh, a.w2, e, used, ss)) { lost = true; break; }
+    if (!gather<T, 1, false>(a, sh, a.w2, e, tid < a.ngroups, ss)) { lost = true; break; }
     if (tid == 0) sh.st.alpha = alpha;
     FinSnorm<T>{&sh.st, nullptr, 0}.finish(ss);
     halo_columns<T, 1>(lo, nlow, re, nhalo, a.ez, a.ez, [&](int c, T tc, T) { win[c - wb] = tc; });
@@ -657,7 +660,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
         acc[1] += tv * tv;
       }
       ++e;
-      publish_groups<T, 2>(a, sh, a.w1, e, slot, acc);
+      publish_groups<T, 2>(a.spmv_grid, sh, a.w1, e, slot, acc);
     }
     T tt[2];
     if (!gather<T, 2, true>(a, sh, a.w1, e, used, tt)) { lost = true; break; }
@@ -670,13 +673,17 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
       st_agent(a.ew + r, w);
       if constexpr (FAITHFUL) st_agent(a.ex + r, x);
     }
-    sh.part[0][tid] = rr;
-    sh.part[1][tid] = rt;
-    __syncthreads();
     ++e;
-    publish_rows<T, 2>(a, sh, a.w2, e);
+    {
+      T acc[2] = {(T)0, (T)0};
+      if (ok) {
+        acc[0] += rt * rr;
+        acc[1] += rr * rr;
+      }
+      publish_groups<T, 2>(a.vec_grid, sh, a.w2, e, group, acc);
+    }
     T rn[2];
-    if (!gather<T, 2, false>(a, sh, a.w2, e, used, rn)) { lost = true; break; }
+    if (!gather<T, 2, false>(a, sh, a.w2, e, tid < a.ngroups, rn)) { lost = true; break; }
     if (tid == 0) {
       sh.st.ts = tt[0];
       sh.st.tt = tt[1];
@@ -808,7 +815,7 @@ static int resident_run(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool f
   a.nslice = s->nslice;
   a.ngroups = (s->nslice + 3) / 4;
   a.spmv_grid = sell_grid(s);
-  a.vec_grid = fused_grid(n);
+  a.vec_grid = CG ? fused_grid(n) : bi_grid(n);
   a.hist = hist;
   a.du = du;
   const int fmt = sizeof(T) == 4 ? s->fmt32 : s->fmt64;

@@ -547,10 +547,13 @@ __device__ __forceinline__ void spmv_sho_body(int n, const int *__restrict__ off
 // one array per offset, and the entry at offset -o of row r is row r - o's
 // value at offset +o.  A value is then read twice, by two rows o apart; o is
 // at most the bandwidth, and the workgroups of one XCD walk one contiguous
-// row range together, so the second read is served by that XCD's L2 and the
-// stream from the Infinity Cache or HBM halves.  What binds the SpMV here is
-// that stream (the caches deliver the second read and the x gathers several
-// times faster), so the loads are all cached, never non-temporal.
+// row range together, so the second read is mostly served by that XCD's L2
+// and the stream from the Infinity Cache or HBM halves; the loads are all
+// cached, never non-temporal.  128^3 Hex8: the fused FP32 CG step 39 -> 32 us,
+// an FP64 SpMV with its update 117 -> 90 us; 101^3 FP64 39 -> 32 us.  What
+// binds it now are the L1s' line requests to the L2 (2.35 M a launch in FP32),
+// which halving the stream does not lower: 9, 14 or 27 entries of a lane in
+// flight and 1024 to 8192 workgroups are within 15%.
 // Entries are added in ascending offset order, the CRS order: FP64 adds only
 // the row's own entries (bit `lane` of pm[slice * K + k]), so its sums are
 // those of the other layouts to the bit; FP32 adds absent entries as +0.

@@ -865,7 +865,8 @@ const float *sho_values32(ehip_system *s) {
 // Values into the half storage, one wave per slice: each row's entries at
 // offsets >= 0 (a slice's CRS range staged in LDS with coalesced loads when
 // it fits: D = 1), and zero[slice], the rows whose off-diagonal entries are
-// all zero.  Bound by reading Values once: 0.25 ms at 128^3 Hex8 (FP64).
+// all zero.  Bound by reading Values once: 0.34 ms at 128^3 Hex8 (FP64; the
+// full copy's gather 0.35).
 template <typename T, int D>
 __device__ __forceinline__ int sym_stage(int sl, int n, int lane, const int *__restrict__ rows,
                                          const T *__restrict__ in, T *buf) {
@@ -916,7 +917,9 @@ constexpr int kSymU = 7;  // stored values of a lane in flight
 // Each row's entries at offsets < 0 against the values stored for them, one
 // wave per slice as above: equal, or the row is a zero row, or the row that
 // stored the value is one and takes this row's value instead.  An entry the
-// row does not have must have a zero value stored.
+// row does not have must have a zero value stored.  0.35 ms at 128^3 Hex8
+// (FP64), reading Values again and the copy (0.49 with one stored value of a
+// lane in flight).
 template <typename T, int D>
 __global__ __launch_bounds__(256) void k_sym_check(int n, int nslice, SymTab tab, const int *__restrict__ rows,
                                                    const unsigned *__restrict__ mask,
