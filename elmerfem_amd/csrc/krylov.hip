@@ -2144,6 +2144,9 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   // the halved stream gave (63^3 Hex8: 37 us full, 42 us half; FP64 112, 84)
   s->sym_on = p->method == EHIP_CG && p->precond < EHIP_PRECOND_ILU0 &&
               (s->sho_d == 1 || p->precision == EHIP_FP64);
+  // on a lane, of systems the resident loops would take elsewhere: their
+  // copies fit the caches, and the check's wait costs more than it gives
+  if (tl_shared_device && s->n <= 262144) s->sym_on = false;
   // one launch per sequence where the rows fit the chip (not for callers
   // without runtime objects of their own, nor when launches are sampled)
   s->resident_on = events && !tl_shared_device && p->profile_every <= 0 && p->precond < EHIP_PRECOND_ILU0;
