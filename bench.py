@@ -717,11 +717,15 @@ def main():
     # the SpMV step's epilogue: folded (the previous vector step's partials summed
     # in every workgroup, two launches per iteration) unless EHIP_CG_FOLD=0
     epi = "EpiCgFast1<float>" if os.environ.get("EHIP_CG_FOLD", "1")[:1] == "0" else "EpiCgFold<float>"
+    half = False  # CG on a symmetric matrix of this layout reads half of the values
     if c32["format"] == "sell_shared":
         lay = sys_.spmv_shared_layout()
+        half = lay["node_block"] <= 1 and 8 * lay["entries"] >= (16 << 20)
         # values streamed non-temporally only when the FP32 copy exceeds the 256 MiB Infinity Cache
         nt = "true" if 4 * lay["entries"] > (256 << 20) else "false"
         kname = "k_spmv_epi_sho<float,256,%d,%d,%s,%s>" % (lay["lane_unroll"], max(1, lay["node_block"]), nt, epi)
+        if half:
+            kname = "k_spmv_epi_sym<float,256,9,1,%s>" % epi
     elif c32["format"] == "sell":
         lay = sys_.spmv_sell_layout()
         if lay["node_block"]:
@@ -739,6 +743,8 @@ def main():
     # what this layout reads for the same work (16-bit column offsets or slice-shared
     # offsets, no row pointers)
     bytes32 = fused_cg32_bytes(nnz, n, bits, c32["format"], c32["chunks"])
+    if half:  # the diagonal and one of each pair of values, a word per slice, z, q and p
+        bytes32 = 4 * (lay["entries"] + n) // 2 + 8 * ((n + 63) // 64) + 20 * n
     achieved = alg32 / (us * 1e-6) / 1e9
     traffic = measured_traffic(kname)
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
