@@ -411,12 +411,12 @@ void ilu_release(ehip_system *s);
 int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, double *hist, bool events);
 
 // Resident Krylov sequences (resident.hip): whether the system and the LDS allow
-// one; its launches (the state's ticket[3] tells a grid that gave up, with
+// one (of CG or BiCGStab, with the true residual of every iteration or not); its launches (the state's ticket[3] tells a grid that gave up, with
 // nothing changed); and the lock to hold from there until the state is read.
 template <typename T>
 struct Vecs;
 template <typename T>
-bool resident_fits(ehip_system *s, bool faithful);
+bool resident_fits(ehip_system *s, bool cg, bool faithful);
 template <typename T>
 int resident_cg(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du);
 template <typename T>

@@ -1384,9 +1384,8 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
     hipLaunchKernelGGL(k_init_state<T>, dim3(1), dim3(1), 0, s->stream, st, (T)c.tol, c.maxit, (T)c.divtol, iter0,
                        tol_u);
   }
-  bool resident = false;
+  bool resident = s->resident_on && resident_fits<T>(s, c.method == EHIP_CG, c.mode == EHIP_FAITHFUL);
   if (c.method == EHIP_CG) {
-    resident = s->resident_on && resident_fits<T>(s, c.mode == EHIP_FAITHFUL);
     if (c.mode == EHIP_FAITHFUL) {
       EHIP_HIP_TRY(hipMemcpyAsync(v.p, v.z, sizeof(T) * n, hipMemcpyDeviceToDevice, s->stream));
       if (resident) {
@@ -1433,8 +1432,6 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
       }
     }
   } else {
-    resident = s->resident_on && resident_fits<T>(s, c.mode == EHIP_FAITHFUL);
-    const int gb = bi_grid(n);
     hipLaunchKernelGGL(k_bi_start<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st, part);
     fin<T>(s, FinBiStart<T>{st, part, g}, g, st);
     for (int it_seen = iter0;; it_seen = hst->iter) {
@@ -1447,15 +1444,15 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
         launch_epi<T>(s, plan, vals, v.t1v, e3, st);
         if (c.prof) prof_end(s);
         fin<T>(s, e3, epi_grid<T>(s, plan), st);
-        hipLaunchKernelGGL(k_bi_s<T>, dim3(gb), dim3(kVecBlock), 0, s->stream, n, v, st, part);
-        fin<T>(s, FinSnorm<T>{st, part, gb}, gb, st);
+        hipLaunchKernelGGL(k_bi_s<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st, part);
+        fin<T>(s, FinSnorm<T>{st, part, g}, g, st);
         hipLaunchKernelGGL(k_bi_snorm_exit<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st);
         hipLaunchKernelGGL(k_bi_snorm_mark<T>, dim3(1), dim3(1), 0, s->stream, st);
         EpiBiT<T> e6{v, st, part, pg, &st->ticket[0], 1};
         launch_epi_fin<T>(s, plan, vals, v.t2v, e6, st);
-        hipLaunchKernelGGL(k_bi_xr<T>, dim3(gb), dim3(kVecBlock), 0, s->stream, n, v, st, part,
+        hipLaunchKernelGGL(k_bi_xr<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v, st, part,
                            c.mode == EHIP_FAST ? 1 : 0, c.hist);
-        fin<T>(s, FinBiXr<T>{st, part, gb, c.mode == EHIP_FAST ? 1 : 0, c.hist}, gb, st);
+        fin<T>(s, FinBiXr<T>{st, part, g, c.mode == EHIP_FAST ? 1 : 0, c.hist}, g, st);
         c.spmv += 2;
         if (c.mode == EHIP_FAITHFUL) {
           EpiBiResidual<T> e8{v, st, part, pg, &st->ticket[2], c.hist, (T)0, (T)0, du};
@@ -1715,7 +1712,7 @@ static int mixed_cg_ru(ehip_system *s, SolveCtx &c, double delta, int *inner_tot
   // the SELL copy of the FP32 values is refreshed here, outside any recording
   if (active_fmt<float>(s) == 1 && !sell_values32(s)) return EHIP_ENOMEM;
   if (active_fmt<float>(s) == 2 && !sym_values32(s) && !sho_values32(s)) return EHIP_ENOMEM;
-  bool resident = s->resident_on && resident_fits<float>(s, false);
+  bool resident = s->resident_on && resident_fits<float>(s, true, false);
   while (!s->h_st->done) {
     if (resident && (rc = run_resident<float>(s, c, v, st32, s->h_st32, false, nullptr, nullptr, it_prev, &resident)))
       return rc;
@@ -2150,7 +2147,8 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   // one launch per sequence where the rows fit the chip (not for callers
   // without runtime objects of their own, nor when launches are sampled)
   s->resident_on = events && !tl_shared_device && p->profile_every <= 0 && p->precond < EHIP_PRECOND_ILU0;
-  if (s->resident_on && resident_fits<double>(s, p->mode == EHIP_FAITHFUL && p->precision == EHIP_FP64))
+  if (s->sym_on && s->resident_on &&
+      resident_fits<double>(s, true, p->mode == EHIP_FAITHFUL && p->precision == EHIP_FP64))
     s->sym_on = false;  // that loop reads the full copy
   SolveClock clk(events, s->stream);
   EHIP_HIP_TRY(clk.create());

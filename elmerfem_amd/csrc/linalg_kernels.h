@@ -37,11 +37,6 @@ inline int vec_grid(int n) {
 constexpr int kFusedCap = 1024;
 inline int fused_grid(int n) { return std::min(vec_grid(n), kFusedCap); }
 
-// Grid of BiCGStab's two vector steps: one row per thread up to 262 144 rows,
-// so that a partial sum is that of 256 consecutive rows, as the resident
-// loop (resident.hip) groups them; vec_grid beyond.
-inline int bi_grid(int n) { return n <= 262144 ? std::max(8, ((n + kVecBlock - 1) / kVecBlock + 7) / 8 * 8) : vec_grid(n); }
-
 // Calls f(i, j) for every stored nonzero j (0-based) of row i, walking the
 // SpMV chunks so that loads of Values/Cols stay coalesced: each thread finds
 // the row of its nonzero by binary search over the chunk's row pointers held

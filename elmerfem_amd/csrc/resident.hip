@@ -29,9 +29,17 @@
 //
 // Bits.  Sums are grouped as the launched kernels group them -- the SpMV's
 // partials per 256 rows, CG's vector step's per 1024 rows with four rows to
-// a thread, BiCGStab's per 256 rows, the totals over 256 threads -- and the scalar updates and
+// a thread, the totals over 256 threads -- and the scalar updates and
 // stopping tests are the same functors (cg_steps.h), so a solve gives the
-// same bits either way.
+// same bits either way.  BiCGStab's launched vector steps walk the rows by
+// a grid of G = vec_grid workgroups, so a partial sum there takes the tiles
+// of 256 rows b, b + G, b + 2 G and b + 3 G, a thread one row of each: a
+// resident workgroup owns those four tiles, each with its window, instead
+// of 1024 rows in a row.  (Its solutions near the s-norm exit follow the
+// order of the sums by far more than rounding, so another grouping would be
+// another answer.)  That takes three more halos: of FP64 systems, a bandwidth
+// up to 920 fits the LDS (1 970 with one window) where CG's 1024 rows in a
+// row take 3 680 (7 880).
 //
 // Waiting.  All workgroups of the grid (at most 256, one per CU) must be on
 // the chip at once.  One such launch at a time runs on a device (a host lock),
@@ -166,10 +174,7 @@ __device__ __forceinline__ int spmv_slot(int g, int ngroups) {
 }
 // The slot of the group that this thread publishes, -1 where it has no rows;
 // found once, as it takes a division.
-__device__ __forceinline__ int group_slot(int ngroups) {
-  const int g = (int)blockIdx.x * 4 + ((int)threadIdx.x & 3);
-  return g < ngroups ? spmv_slot(g, ngroups) : -1;
-}
+__device__ __forceinline__ int group_slot(int g, int ngroups) { return g < ngroups ? spmv_slot(g, ngroups) : -1; }
 __device__ __forceinline__ bool slot_used(int b, int ngroups) {
   const int xcd = b & 7, lb = b >> 3;
   return (int)((long long)ngroups * xcd / 8) + lb < (int)((long long)ngroups * (xcd + 1) / 8);
@@ -204,9 +209,10 @@ struct ResRow {
   // Sums of one or two vectors held in LDS windows starting at column wb, in
   // the launched kernels' order (spmv_sho_body, spmv_sell2_body,
   // spmv_sell_body).
+  // `own` is the row's own place there.
   template <int NX>
-  __device__ __forceinline__ void sums(const ResArgs<T> &a, int sl, int lane, int wb, const T *w0, const T *w1,
-                                       T (&s)[NX]) const {
+  __device__ __forceinline__ void sums(const ResArgs<T> &a, int sl, int lane, int wb, int own, const T *w0,
+                                       const T *w1, T (&s)[NX]) const {
     constexpr bool kF32 = sizeof(T) == 4;
 #pragma unroll
     for (int x = 0; x < NX; ++x) s[x] = (T)0;
@@ -223,7 +229,6 @@ struct ResRow {
       // KW offsets in a few wide scalar loads: past the slice's list they are
       // the next slices' (or the padding's), inside the window all the same
       const int *__restrict__ t = a.tab + (p0 >> 6);
-      const int own = (int)threadIdx.x + a.halo;
 #pragma unroll
       for (int k = 0; k < KW; ++k) add(v[k], own + t[k], (m >> k) & 1u);
     } else if constexpr (!kF32) {
@@ -300,10 +305,12 @@ __device__ __forceinline__ void publish_groups(int stride, ResShared<T> &sh, Wor
   }
 }
 
-// Partial sums of the vector step over this workgroup's 1024 rows
-// (block_publish after CgTile::step: four rows to a thread).
+// Partial sums of the vector step over this workgroup's four tiles of 256
+// rows, a row of each to a thread (block_publish after CgTile::step, or after
+// BiCGStab's vector steps); tile k begins at row first + k * apart.
 template <typename T, int NV>
-__device__ __forceinline__ void publish_rows(const ResArgs<T> &a, ResShared<T> &sh, Word *w, unsigned e) {
+__device__ __forceinline__ void publish_rows(const ResArgs<T> &a, ResShared<T> &sh, Word *w, unsigned e, int first,
+                                             int apart) {
   const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (tid < 256) {
     T acc[NV];
@@ -312,7 +319,7 @@ __device__ __forceinline__ void publish_rows(const ResArgs<T> &a, ResShared<T> &
 #pragma unroll
     for (int k = 0; k < kVI; ++k) {
       const int i = k * kVecBlock + tid;
-      if ((int)blockIdx.x * kResRows + i < a.n) {
+      if (first + k * apart + tid < a.n) {
         const T ri = sh.part[0][i], zi = sh.part[1][i];
         acc[0] += ri * zi;
         if constexpr (NV > 1) acc[1] += ri * ri;
@@ -381,23 +388,23 @@ __device__ __forceinline__ bool gather(const ResArgs<T> &a, ResShared<T> &sh, co
   return sh.fail == 0;
 }
 
-// Calls f(c, entries of e0 (and e1) at column c) for the workgroup's halo
-// columns, kHaloU columns of a thread in flight.
+// Calls f(c, entries of e0 (and e1) at column c) for the halo columns of
+// each TH threads' rows, kHaloU columns of a thread in flight.
 constexpr int kHaloU = 6;
-template <typename T, int NE, class Fn>
+template <typename T, int TH, int NE, class Fn>
 __device__ __forceinline__ void halo_columns(int lo, int nlow, int re, int nhalo, const T *e0, const T *e1, Fn f) {
-  for (int i0 = (int)threadIdx.x; i0 < nhalo; i0 += kHaloU * kResRows) {
+  for (int i0 = (int)threadIdx.x & (TH - 1); i0 < nhalo; i0 += kHaloU * TH) {
     T v[NE][kHaloU];
 #pragma unroll
     for (int u = 0; u < kHaloU; ++u) {
-      const int i = min(i0 + u * kResRows, nhalo - 1);
+      const int i = min(i0 + u * TH, nhalo - 1);
       const int c = i < nlow ? lo + i : re + (i - nlow);
       v[0][u] = ld_agent(e0 + c);
       if constexpr (NE > 1) v[1][u] = ld_agent(e1 + c);
     }
 #pragma unroll
     for (int u = 0; u < kHaloU; ++u) {
-      const int i = i0 + u * kResRows;
+      const int i = i0 + u * TH;
       if (i < nhalo) f(i < nlow ? lo + i : re + (i - nlow), v[0][u], v[NE - 1][u]);
     }
   }
@@ -441,14 +448,14 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
   }
   __syncthreads();
   double *const hist = blockIdx.x == 0 ? a.hist : nullptr;
-  const int slot = group_slot(a.ngroups);
+  const int slot = group_slot((int)blockIdx.x * 4 + (tid & 3), a.ngroups);
   const bool used = tid < a.spmv_grid && slot_used(tid, a.ngroups);
   unsigned e = 1;
   T sx[FAITHFUL ? 2 : 1];
   bool lost = false;
   if constexpr (FAITHFUL) {
     T s[1];
-    row.template sums<1>(a, sl, lane, wb, win, win, s);
+    row.template sums<1>(a, sl, lane, wb, own, win, win, s);
     q = s[0];
     T acc[3] = {(T)0, (T)0, (T)0};
     if (ok) acc[0] += p * q;
@@ -468,7 +475,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
       }
       pq = tot[0];
     } else {
-      row.template sums<1>(a, sl, lane, wb, win, win, sx);
+      row.template sums<1>(a, sl, lane, wb, own, win, win, sx);
       const T beta = sh.st.beta;
       q = sx[0] + beta * q;
       p = z + beta * p;
@@ -493,12 +500,12 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
     if (!FAITHFUL && ok) win[own] = z;
     __syncthreads();
     if constexpr (FAITHFUL) {
-      publish_rows<T, 1>(a, sh, a.w2, e);
+      publish_rows<T, 1>(a, sh, a.w2, e, R0, kVecBlock);
       T rn[1];
       if (!gather<T, 1, false>(a, sh, a.w2, e, tid < (int)gridDim.x, rn)) { lost = true; break; }
       const T beta = rn[0] / sh.st.rho;
       p = z + beta * p;
-      halo_columns<T, 2>(lo, nlow, re, nhalo, a.ez, a.ex, [&](int c, T zc, T xc) {
+      halo_columns<T, kResRows, 2>(lo, nlow, re, nhalo, a.ez, a.ex, [&](int c, T zc, T xc) {
         win[c - wb] = zc + beta * win[c - wb];
         winx[c - wb] = xc;
       });
@@ -512,7 +519,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
         sh.st.alpha = alpha;
         sh.st.rho_new = rn[0];
       }
-      row.template sums<2>(a, sl, lane, wb, win, winx, sx);
+      row.template sums<2>(a, sl, lane, wb, own, win, winx, sx);
       q = sx[0];
       T acc[3] = {(T)0, (T)0, (T)0};
       if (ok) {
@@ -525,7 +532,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
       ++e;
       publish_groups<T, 3>(a.spmv_grid, sh, a.w1, e, slot, acc);
     } else {
-      publish_rows<T, 2>(a, sh, a.w2, e);
+      publish_rows<T, 2>(a, sh, a.w2, e, R0, kVecBlock);
       T tot[2];
       if (!gather<T, 2, false>(a, sh, a.w2, e, tid < (int)gridDim.x, tot)) { lost = true; break; }
       if (tid == 0) {
@@ -533,7 +540,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
         sh.st.alpha = alpha;
       }
       FinCgFast2<T>{&sh.st, nullptr, 0, hist}.finish(tot);
-      halo_columns<T, 1>(lo, nlow, re, nhalo, a.ez, a.ez, [&](int c, T zc, T) { win[c - wb] = zc; });
+      halo_columns<T, kResRows, 1>(lo, nlow, re, nhalo, a.ez, a.ez, [&](int c, T zc, T) { win[c - wb] = zc; });
       __syncthreads();
       if (sh.st.done) break;
       ++e;
@@ -558,20 +565,25 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
 // A x taken in one pass with the next iteration's A t1v; else FinBiXr's tests
 // on the recurrence residual.  The halo's t1v = (r + beta w) / dg needs beta,
 // so r and w = p - omega v travel with the partial sums that give it.
+// A thread's tile of 256 rows is k of the workgroup's four, a whole number of
+// grids apart; its window begins at k (256 + 2 halo).
 template <typename T, ResFmt F, int KW, bool FAITHFUL>
 __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
   extern __shared__ __align__(16) char lds[];
   __shared__ ResShared<T> sh;
   const int tid = (int)threadIdx.x, lane = tid & 63;
-  const int R0 = (int)blockIdx.x * kResRows, r = R0 + tid, rl = min(r, a.n - 1);
+  const int k = __builtin_amdgcn_readfirstlane(tid >> 8), t = tid & (kVecBlock - 1);
+  const int apart = (int)gridDim.x * kVecBlock, T0 = (int)blockIdx.x * kVecBlock;
+  const int R0 = T0 + k * apart, r = R0 + t, rl = min(r, a.n - 1);
   const bool ok = r < a.n;
-  const int sl = __builtin_amdgcn_readfirstlane(R0 / 64 + (tid >> 6));
-  const int wb = R0 - a.halo, own = tid + a.halo;
-  const int lo = max(wb, 0), re = min(R0 + kResRows, a.n);
-  const int we = min(R0 + kResRows + a.halo, a.n);
-  const int nlow = R0 - lo, nhalo = nlow + (we - re);
-  T *win = reinterpret_cast<T *>(lds);      // t1v and t2v in turn
-  T *winx = win + (kResRows + 2 * a.halo);  // x (FAITHFUL)
+  const int sl = __builtin_amdgcn_readfirstlane(R0 / 64 + (t >> 6));
+  const int width = kVecBlock + 2 * a.halo;
+  const int wb = R0 - a.halo - k * width, own = k * width + t + a.halo;
+  const int lo = max(R0 - a.halo, 0), re = min(R0 + kVecBlock, a.n);
+  const int we = min(R0 + kVecBlock + a.halo, a.n);
+  const int nlow = R0 - lo, nhalo = R0 < a.n ? nlow + (we - re) : 0;
+  T *win = reinterpret_cast<T *>(lds);  // t1v and t2v in turn
+  T *winx = win + 4 * width;            // x (FAITHFUL)
   T x = a.v.x[rl], p = a.v.p[rl], v = a.v.v[rl], rr = a.v.r[rl], t1 = a.v.t1v[rl];
   const T dg = a.v.dg[rl], rt = a.v.rtld[rl];
   const T b = FAITHFUL ? a.v.b[rl] : (T)0, d = FAITHFUL && a.du ? a.du[rl] : (T)1;
@@ -581,23 +593,22 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
     sh.st = *a.st;
     sh.fail = 0;
   }
-  for (int i = tid; i < kResRows + 2 * a.halo; i += kResRows) {
+  for (int i = k * width + t; i < (k + 1) * width; i += kVecBlock) {
     const int c = wb + i;
     win[i] = c >= 0 && c < a.n ? a.v.t1v[c] : (T)0;
     if constexpr (FAITHFUL) winx[i] = (T)0;
   }
   __syncthreads();
   double *const hist = blockIdx.x == 0 ? a.hist : nullptr;
-  const int slot = group_slot(a.ngroups);
+  const int slot = group_slot((int)blockIdx.x + (tid & 3) * (int)gridDim.x, a.ngroups);
   const bool used = tid < a.spmv_grid && slot_used(tid, a.ngroups);
-  const int g4 = (int)blockIdx.x * 4 + (tid & 3), group = g4 < a.ngroups ? g4 : -1;
   unsigned e = 0;
   bool lost = false;
   if (!sh.st.done) for (bool first = true;; first = false) {
     ++e;
     if (FAITHFUL && !first) {
       T s[2];
-      row.template sums<2>(a, sl, lane, wb, win, winx, s);
+      row.template sums<2>(a, sl, lane, wb, own, win, winx, s);
       v = s[0];
       T acc[3] = {(T)0, (T)0, (T)0};
       if (ok) {
@@ -610,7 +621,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
       publish_groups<T, 3>(a.spmv_grid, sh, a.w1, e, slot, acc);
     } else {
       T s[1];
-      row.template sums<1>(a, sl, lane, wb, win, win, s);
+      row.template sums<1>(a, sl, lane, wb, own, win, win, s);
       v = s[0];
       T acc[3] = {(T)0, (T)0, (T)0};
       if (ok) acc[0] += rt * v;
@@ -630,17 +641,16 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
     const T t2 = s / dg;
     if (ok) st_agent(a.ez + r, t2);
     if (ok) win[own] = t2;
+    sh.part[0][tid] = s;
+    sh.part[1][tid] = s;
     ++e;
-    {
-      T acc[1] = {(T)0};
-      if (ok) acc[0] += s * s;
-      publish_groups<T, 1>(a.vec_grid, sh, a.w2, e, group, acc);
-    }
+    __syncthreads();
+    publish_rows<T, 1>(a, sh, a.w2, e, T0, apart);
     T ss[1];
-    if (!gather<T, 1, false>(a, sh, a.w2, e, tid < a.ngroups, ss)) { lost = true; break; }
+    if (!gather<T, 1, false>(a, sh, a.w2, e, tid < (int)gridDim.x, ss)) { lost = true; break; }
     if (tid == 0) sh.st.alpha = alpha;
     FinSnorm<T>{&sh.st, nullptr, 0}.finish(ss);
-    halo_columns<T, 1>(lo, nlow, re, nhalo, a.ez, a.ez, [&](int c, T tc, T) { win[c - wb] = tc; });
+    halo_columns<T, kVecBlock, 1>(lo, nlow, re, nhalo, a.ez, a.ez, [&](int c, T tc, T) { win[c - wb] = tc; });
     __syncthreads();
     if (sh.st.snorm_exit) {
       x = x + alpha * t1;
@@ -650,7 +660,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
     T tv;
     {
       T q[1];
-      row.template sums<1>(a, sl, lane, wb, win, win, q);
+      row.template sums<1>(a, sl, lane, wb, own, win, win, q);
       tv = q[0];
     }
     {
@@ -673,17 +683,13 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
       st_agent(a.ew + r, w);
       if constexpr (FAITHFUL) st_agent(a.ex + r, x);
     }
+    sh.part[0][tid] = rr;
+    sh.part[1][tid] = rt;
     ++e;
-    {
-      T acc[2] = {(T)0, (T)0};
-      if (ok) {
-        acc[0] += rt * rr;
-        acc[1] += rr * rr;
-      }
-      publish_groups<T, 2>(a.vec_grid, sh, a.w2, e, group, acc);
-    }
+    __syncthreads();
+    publish_rows<T, 2>(a, sh, a.w2, e, T0, apart);
     T rn[2];
-    if (!gather<T, 2, false>(a, sh, a.w2, e, tid < a.ngroups, rn)) { lost = true; break; }
+    if (!gather<T, 2, false>(a, sh, a.w2, e, tid < (int)gridDim.x, rn)) { lost = true; break; }
     if (tid == 0) {
       sh.st.ts = tt[0];
       sh.st.tt = tt[1];
@@ -695,10 +701,10 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
     const T beta = FAITHFUL ? (sh.st.rho_new * alpha) / (sh.st.rho * omega) : sh.st.beta;
     p = rr + beta * w;
     t1 = p / dg;
-    halo_columns<T, 2>(lo, nlow, re, nhalo, a.er, a.ew,
+    halo_columns<T, kVecBlock, 2>(lo, nlow, re, nhalo, a.er, a.ew,
                        [&](int c, T rc, T wc) { win[c - wb] = (rc + beta * wc) / a.v.dg[c]; });
     if constexpr (FAITHFUL)
-      halo_columns<T, 1>(lo, nlow, re, nhalo, a.ex, a.ex, [&](int c, T xc, T) { winx[c - wb] = xc; });
+      halo_columns<T, kVecBlock, 1>(lo, nlow, re, nhalo, a.ex, a.ex, [&](int c, T xc, T) { winx[c - wb] = xc; });
     if (ok) {
       win[own] = t1;
       if constexpr (FAITHFUL) winx[own] = x;
@@ -755,10 +761,16 @@ std::mutex &resident_lock(const ehip_system *s) { return g_resident_mu[s->dev & 
 // vector values of up to 1024 tiles, two words each.
 constexpr int kW1 = 3 * 1024 * 2, kW2 = 2 * 1024 * 2;
 
-// Rows per workgroup times CUs bound n; two windows of 1024 rows and the
-// halo on both sides must fit the LDS (one in the one-SpMV order).
+// Values in a workgroup's window: its rows (BiCGStab: four tiles) and the
+// halo on both sides.
+static int64_t window(bool cg, int halo) {
+  return cg ? kResRows + 2 * (int64_t)halo : 4 * (kVecBlock + 2 * (int64_t)halo);
+}
+
+// Rows per workgroup times CUs bound n; two windows must fit the LDS (one in
+// the orders that test the recurrence residual).
 template <typename T>
-bool resident_fits(ehip_system *s, bool faithful) {
+bool resident_fits(ehip_system *s, bool cg, bool faithful) {
   const int fmt = sizeof(T) == 4 ? s->fmt32 : s->fmt64;
   const int halo = fmt == 2 ? s->sho_halo : s->sell_halo;
   if (s->n > kResRows * kResGroups || halo < 0 || s->n < 1) return false;
@@ -770,7 +782,7 @@ bool resident_fits(ehip_system *s, bool faithful) {
   } else {
     return false;
   }
-  const int64_t win = (kResRows + 2 * (int64_t)halo) * (int64_t)sizeof(T) * (faithful ? 2 : 1);
+  const int64_t win = window(cg, halo) * (int64_t)sizeof(T) * (faithful ? 2 : 1);
   return win + (int64_t)sizeof(ResShared<T>) + 64 <= kResLds;
 }
 
@@ -815,7 +827,9 @@ static int resident_run(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool f
   a.nslice = s->nslice;
   a.ngroups = (s->nslice + 3) / 4;
   a.spmv_grid = sell_grid(s);
-  a.vec_grid = CG ? fused_grid(n) : bi_grid(n);
+  // CG: 1024 rows to a workgroup; BiCGStab: the launched vector steps' grid
+  const int g = CG ? (n + kResRows - 1) / kResRows : vec_grid(n);
+  a.vec_grid = CG ? fused_grid(n) : g;
   a.hist = hist;
   a.du = du;
   const int fmt = sizeof(T) == 4 ? s->fmt32 : s->fmt64;
@@ -839,8 +853,7 @@ static int resident_run(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool f
     a.tab = s->sell_base;
   }
   if (!a.vals) return EHIP_ENOMEM;
-  const int g = (n + kResRows - 1) / kResRows;
-  const size_t lds = (size_t)(kResRows + 2 * a.halo) * sizeof(T) * (faithful ? 2 : 1);
+  const size_t lds = (size_t)window(CG, a.halo) * sizeof(T) * (faithful ? 2 : 1);
   hipLaunchKernelGGL(k_resident_clear, dim3(16), dim3(256), 0, s->stream, a.w1, kW1 + kW2, a.gave_up, &st->ticket[3]);
 #define EHIP_RES(F, KW)                                                                                            \
   if constexpr (CG) {                                                                                              \
@@ -873,8 +886,8 @@ int resident_bicgstab(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool fai
   return resident_run<T, false>(s, v, st, faithful, hist, du);
 }
 
-template bool resident_fits<double>(ehip_system *, bool);
-template bool resident_fits<float>(ehip_system *, bool);
+template bool resident_fits<double>(ehip_system *, bool, bool);
+template bool resident_fits<float>(ehip_system *, bool, bool);
 template int resident_cg<double>(ehip_system *, const Vecs<double> &, KStateT<double> *, bool, double *,
                                  const double *);
 template int resident_cg<float>(ehip_system *, const Vecs<float> &, KStateT<float> *, bool, double *, const float *);

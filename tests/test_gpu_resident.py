@@ -8,6 +8,10 @@ layout the loops read, at sizes around the 1024 rows of a workgroup and the
 256 of a partial sum, and for every exit (convergence, iteration limit, a
 tightened unscaled test).
 """
+import hashlib
+import json
+import os
+
 import numpy as np
 import pytest
 
@@ -88,7 +92,9 @@ def test_iteration_limit(ehip, precision, mode, maxit):
     s.free()
 
 
-@pytest.mark.parametrize("n", [1, 65, 257, 1025, 3100])
+# ... and the 2048, 4096 and 8192 rows of one, two and four tiles to each of
+# the first eight workgroups, and one workgroup row more
+@pytest.mark.parametrize("n", [1, 65, 257, 1025, 2048, 2049, 3100, 4097, 8192, 8193])
 @pytest.mark.parametrize("mode", [_lib.FAITHFUL, _lib.FAST])
 def test_bicgstab_row_counts(ehip, n, mode):
     rows, cols, diag, vals, b = _tridiagonal(n)
@@ -112,6 +118,35 @@ def test_bicgstab_convdiff(ehip, n, precision, mode, fmt):
         _same(s, w["kw"], precision=precision, mode=mode, true_residual_stop=stop)
     w["kw"].maxit = 3
     assert _same(s, w["kw"], precision=precision, mode=mode)["info"] == 2
+    s.free()
+
+
+with open(os.path.join(os.path.dirname(__file__), "golden", "bicgstab_convdiff.json")) as _f:
+    BICGSTAB = json.load(_f)
+
+
+@pytest.mark.parametrize("case", sorted(BICGSTAB))
+@pytest.mark.parametrize("form", ["faithful", "fast", "mixed"])
+def test_bicgstab_recorded_bits(ehip, case, form):
+    """BiCGStab's answers are those of the launched loops before there were
+    resident ones, recorded then: iterations, exit, residual and solution
+    bits.  Near the s-norm exit (info 36: the true residual stalls above the
+    tolerance) the solution follows the order of the partial sums by 1e-12
+    to 1e-7, so comparing the two loops alone cannot tell that both moved.
+    Both loops, Peclet numbers 45 and 89."""
+    _, n, index = case.split("_")
+    want = BICGSTAB[case]
+    w = W.convdiff_quad4(int(n), index=int(index))
+    s, _ = W.build_system(w)
+    vals, rhs = s.values()
+    assert hashlib.sha256(vals.tobytes()).hexdigest() == want["values"]
+    precision, mode = dict(zip(("faithful", "fast", "mixed"), FORMS))[form]
+    for every in (0, 1 << 30):
+        s.set_values(vals, rhs)
+        x, r = s.solve(w["kw"], precision=precision, mode=mode, profile_every=every)
+        got = {"iters": r["iters"], "info": r["info"], "res_true": r["res_true"].hex(),
+               "x": hashlib.sha256(x.tobytes()).hexdigest()}
+        assert got == want[form], every
     s.free()
 
 
