@@ -1611,11 +1611,23 @@ static void cg32_iterations(ehip_system *s, const Vecs<float> &v, int count, boo
   }
 }
 
-// What a recorded block bakes in: buffers, SpMV format and schedule.
-static uint64_t cg32_key(const ehip_system *s) {
+// The FP32 values that the launched steps of the solve in progress read, in
+// the layout they read them (launch_epi), brought up to date; null: no memory.
+static const float *cg32_values(ehip_system *s) {
+  const int fmt = active_fmt<float>(s);
+  if (fmt == 1) return sell_values32(s);
+  if (fmt != 2) return s->vals32;
+  const float *half = sym_values32(s);
+  return half ? half : sho_values32(s);
+}
+
+// What a recorded block bakes in: buffers, SpMV layout and schedule.  The
+// values' address tells which layout the block's kernels read: one system
+// may be solved on the half storage and, elsewhere, on the full copy, and
+// only the copy in use is up to date.
+static uint64_t cg32_key(const ehip_system *s, const float *values) {
   const uint64_t parts[] = {(uint64_t)(uintptr_t)s->work32, (uint64_t)(uintptr_t)s->vals32,
-                            (uint64_t)(uintptr_t)s->sell32, (uint64_t)(uintptr_t)s->sho32,
-                            s->sym32.good ? (uint64_t)(uintptr_t)s->sym32.v : 0,
+                            (uint64_t)(uintptr_t)values, (uint64_t)epi_grid<float>(s, s->plan32),
                             (uint64_t)(uintptr_t)s->partials32,
                             (uint64_t)(uintptr_t)s->st32, (uint64_t)(uintptr_t)s->plan32.chunk_row,
                             (uint64_t)s->fmt32, (uint64_t)s->plan32.block, (uint64_t)s->plan32.nb,
@@ -1630,11 +1642,14 @@ static uint64_t cg32_key(const ehip_system *s) {
 
 // Enqueues `count` iterations as replays of recorded blocks (one graph launch
 // per power-of-two piece instead of three kernel launches per iteration).  The
+// values copy is brought up to date first, outside any recording.  The
 // blocks are built node by node (launch_k under a recorder), not captured,
 // and hold kernels only; every iteration kernel reads its scalars from the
 // device state, so a replay is the same work as direct launches.
 static int cg32_iterations_graph(ehip_system *s, const Vecs<float> &v, int count) {
-  const uint64_t key = cg32_key(s);
+  const float *values = cg32_values(s);
+  if (!values) return EHIP_ENOMEM;
+  const uint64_t key = cg32_key(s, values);
   if (key != s->cg32_key) {
     // nothing recorded earlier may still be queued when its graph goes
     EHIP_HIP_TRY(hipStreamSynchronize(s->stream));
@@ -1709,9 +1724,6 @@ static int mixed_cg_ru(ehip_system *s, SolveCtx &c, double delta, int *inner_tot
   double lres_prev = std::log(std::max(s->h_st->res, 1e-300));
   double rate = 0.0;  // log residual change per iteration (< 0)
   int batch = std::min(cap, 8);
-  // the SELL copy of the FP32 values is refreshed here, outside any recording
-  if (active_fmt<float>(s) == 1 && !sell_values32(s)) return EHIP_ENOMEM;
-  if (active_fmt<float>(s) == 2 && !sym_values32(s) && !sho_values32(s)) return EHIP_ENOMEM;
   bool resident = s->resident_on && resident_fits<float>(s, true, false);
   while (!s->h_st->done) {
     if (resident && (rc = run_resident<float>(s, c, v, st32, s->h_st32, false, nullptr, nullptr, it_prev, &resident)))

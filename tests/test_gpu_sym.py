@@ -11,6 +11,8 @@ import numpy as np
 import pytest
 
 from elmerfem_amd import _lib, workloads as W
+from elmerfem_amd.batch import Server
+from elmerfem_amd.system import System
 
 pytestmark = pytest.mark.gpu
 
@@ -79,4 +81,70 @@ def test_unsymmetric_values_keep_the_full_copy(ehip):
     s.set_values(vals, rhs)
     b = _solves_equal(s, w["kw"], mode=_lib.FAST)
     assert not np.array_equal(a, b) and np.allclose(a, b, rtol=1e-6, atol=1e-12)
+    s.free()
+
+
+def _box27(nx, ny, nz):
+    """27-point pattern of an nx x ny x nz node grid (1-based CRS), and
+    values(seed): symmetric to the bit, diagonally dominant."""
+    n = nx * ny * nz
+    k, j, i = np.meshgrid(np.arange(nz), np.arange(ny), np.arange(nx), indexing="ij")
+    k, j, i = k.ravel(), j.ravel(), i.ravel()
+    r = np.arange(n)
+    off = [(c, b, a) for c in (-1, 0, 1) for b in (-1, 0, 1) for a in (-1, 0, 1)]
+    ok = np.stack([(k + c >= 0) & (k + c < nz) & (j + b >= 0) & (j + b < ny) & (i + a >= 0) & (i + a < nx)
+                   for c, b, a in off], 1)
+    col = np.stack([r + (c * ny + b) * nx + a for c, b, a in off], 1)
+    rows = np.concatenate([[1], 1 + np.cumsum(ok.sum(1))]).astype(np.int32)
+    diag = (rows[:-1] + ok[:, :13].sum(1)).astype(np.int32)
+
+    def values(seed):
+        g = np.random.default_rng(seed).random(n)
+        v = np.zeros(ok.shape)
+        for q in range(27):
+            if q != 13:
+                lo, hi = np.minimum(r, col[:, q]) % n, np.maximum(r, col[:, q]) % n
+                v[:, q] = np.where(ok[:, q], -(0.2 + g[lo] * g[hi]), 0.0)
+        v[:, 13] = 0.02 + np.abs(v).sum(1)
+        return v[ok]
+    return rows, (col[ok] + 1).astype(np.int32), diag, values
+
+
+@pytest.mark.parametrize("first", ["direct", "lane"])
+def test_recorded_blocks_follow_the_copy_in_use(ehip, first):
+    """A direct mixed solve reads the half storage, the same system's solve on
+    a server's lane (at most 262 144 rows) the full copy; the bandwidth is
+    beyond the resident loops', so both replay recorded blocks.  New values
+    before every solve, the two kinds in turn: each is that of a system that
+    was never solved before."""
+    rows, cols, diag, values = _box27(136, 136, 14)
+    n = len(rows) - 1
+    kw = W._kw("cg", "diagonal", 1e-10, 2000)
+    rhs = 1.0 + 0.5 * np.cos(np.arange(n))
+
+    def solve(s, seed, how):
+        s.set_values(values(seed), rhs)
+        if how == "direct":
+            x, rep = s.solve(kw, precision=_lib.MIXED_IR, mode=_lib.FAST)
+            return x, rep
+        srv = Server(kw, precision=_lib.MIXED_IR, max_slots=4)
+        srv.set_lane(100000, 1)
+        assert srv.submit(s)
+        done = []
+        while not done:
+            done = srv.step()
+        x = s.solution()
+        srv.free()
+        return x, done[0][1]
+
+    kinds = ["direct", "lane"] if first == "direct" else ["lane", "direct"]
+    s = System.from_csr(rows, cols, diag)
+    for seed in range(4):
+        x, rep = solve(s, seed, kinds[seed % 2])
+        fresh = System.from_csr(rows, cols, diag)
+        y, want = solve(fresh, seed, kinds[seed % 2])
+        fresh.free()
+        assert want["info"] == 1
+        assert (rep["info"], rep["iters"], rep["outer_iters"]) == (1, want["iters"], want["outer_iters"]), seed
+        assert np.array_equal(x, y), seed
     s.free()
