@@ -20,6 +20,7 @@ FAITHFUL, FAST = 0, 1
 PHYS_MODELPDE, PHYS_ELASTIC = 0, 1
 SPMV_CSR, SPMV_SELL, SPMV_SELL_SHARED = 0, 1, 2
 EARG, EHIP, ENOMEM, EUNSUP, ECAP, ESTATE = -1, -2, -3, -4, -5, -6
+LOOP_LAUNCHED, LOOP_RECORDED, LOOP_RESIDENT, LOOP_GAVE_UP = 1, 2, 4, 8
 NOALLOC_SCRATCH_BYTES = 96 << 20
 NOALLOC_MAX_N, NOALLOC_MAX_NNZ = 262144, 4194304
 
@@ -87,6 +88,7 @@ SIGNATURES = {
     "ehip_dirichlet": (C.c_int, [_vp, C.c_int, _vp, _vp, C.c_int, C.c_int]),
     "ehip_solve": (C.c_int, [_vp, C.POINTER(Params), _vp, C.POINTER(Report), _vp]),
     "ehip_get_solution": (C.c_int, [_vp, _vp]),
+    "ehip_solve_route": (C.c_int, [_vp, _ip, _ip, _ip]),
     "ehip_solve_csr": (C.c_int, [C.c_int, _vp, _vp, _vp, _vp, _vp, _vp, C.POINTER(Params), C.POINTER(Report)]),
     "ehip_solve_csr_noalloc": (C.c_int, [C.c_int, _vp, _vp, _vp, _vp, _vp, _vp, C.POINTER(Params),
                                          C.POINTER(Report)]),

@@ -204,6 +204,8 @@ struct ehip_system {
   bool resident_on = false;           // the solve in progress may use them
   void *res_buf = nullptr;
   size_t res_bytes = 0;
+  // what the last solve ran (ehip_solve_route)
+  int route_loops = 0, route_half = 0, route_grid32 = 0;
   uint64_t vals_ver = 1, vals32_ver = 1, sell64_ver = 0, sell32_ver = 0;
   double *vals = nullptr, *rhs = nullptr, *x = nullptr;
   float *vals32 = nullptr;

@@ -1240,6 +1240,7 @@ static void launch_epi(ehip_system *s, const SpmvPlan &p, const T *vals, const T
     if constexpr (EpiOnSym<Epi>::value) {
       if constexpr (F32) sv = sym_values32(s); else sv = sym_values64(s);
       if (sv) {
+        s->route_half |= F32 ? 2 : 1;
         if (s->sho_d == 3) launch_epi_sym<T, 3>(s, sv, xin, e, st);
         else launch_epi_sym<T, 1>(s, sv, xin, e, st);
         return;
@@ -1354,6 +1355,7 @@ static int run_resident(ehip_system *s, SolveCtx &c, const Vecs<T> &v, KStateT<T
   int rc;
   if ((rc = (c.method == EHIP_CG ? resident_cg<T> : resident_bicgstab<T>)(s, v, st, faithful, hist, du)) || (rc = read_state(s, st, hst))) return rc;
   *resident = hst->ticket[3] == 0;
+  s->route_loops |= *resident ? EHIP_LOOP_RESIDENT : EHIP_LOOP_GAVE_UP;
   if (*resident) c.spmv += std::max(0, hst->iter - it0) * ((faithful ? 2 : 1) + (c.method == EHIP_CG ? 0 : 1));
   return EHIP_OK;
 }
@@ -1392,6 +1394,7 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
         if ((rc = run_resident<T>(s, c, v, st, hst, true, c.hist, du, iter0, &resident))) return rc;
       }
       for (; !resident;) {
+        s->route_loops |= EHIP_LOOP_LAUNCHED;
         for (int k = 0; k < c.check; ++k) {
           EpiCgQ<T> e1{v, st, part, pg, &st->ticket[0]};
           if (c.prof) prof_begin(s);
@@ -1410,6 +1413,7 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
       hipLaunchKernelGGL(k_zero2<T>, dim3(g), dim3(kVecBlock), 0, s->stream, n, v.p, v.q);
       for (int it_seen = iter0;; it_seen = hst->iter) {
         if (resident && (rc = run_resident<T>(s, c, v, st, hst, false, c.hist, du, it_seen, &resident))) return rc;
+        if (!resident) s->route_loops |= EHIP_LOOP_LAUNCHED;
         for (int k = 0; !resident && k < c.check; ++k) {
           EpiCgFast1<T> e1{v, st, part, pg, &st->ticket[0], (T)0};
           if (c.prof) prof_begin(s);
@@ -1438,6 +1442,7 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
       if (resident &&
           (rc = run_resident<T>(s, c, v, st, hst, c.mode == EHIP_FAITHFUL, c.hist, du, it_seen, &resident)))
         return rc;
+      if (!resident) s->route_loops |= EHIP_LOOP_LAUNCHED;
       for (int k = 0; !resident && k < c.check; ++k) {
         EpiBiV<T> e3{v, st, part, pg, &st->ticket[0]};
         if (c.prof) prof_begin(s);
@@ -1585,6 +1590,7 @@ constexpr int kRuMaxBlock = 63;
 // carries a badly scaled beta).
 static void cg32_iterations(ehip_system *s, const Vecs<float> &v, int count, bool prof) {
   const int n = s->n, gf = fused_grid(n), pg = kEpiStride;
+  if (!tl_graph_rec) s->route_loops |= EHIP_LOOP_LAUNCHED;
   KState32 *st32 = s->st32;
   float *vpart = s->partials32 + kVecPartOff;
   if (cg_fold_enabled()) {
@@ -1598,6 +1604,7 @@ static void cg32_iterations(ehip_system *s, const Vecs<float> &v, int count, boo
                (const float *)s->partials32, epi_grid<float>(s, s->plan32), vpart);
     }
     fin<float>(s, FinCgFold<float>{st32, vpart, gf}, gf, st32);
+    s->route_grid32 = epi_grid<float>(s, s->plan32);
     return;
   }
   for (int k = 0; k < count; ++k) {
@@ -1609,6 +1616,7 @@ static void cg32_iterations(ehip_system *s, const Vecs<float> &v, int count, boo
              epi_grid<float>(s, s->plan32), vpart);
     fin<float>(s, FinCgFast2<float>{st32, vpart, gf, nullptr}, gf, st32);
   }
+  s->route_grid32 = epi_grid<float>(s, s->plan32);
 }
 
 // The FP32 values that the launched steps of the solve in progress read, in
@@ -1649,6 +1657,9 @@ static uint64_t cg32_key(const ehip_system *s, const float *values) {
 static int cg32_iterations_graph(ehip_system *s, const Vecs<float> &v, int count) {
   const float *values = cg32_values(s);
   if (!values) return EHIP_ENOMEM;
+  s->route_loops |= EHIP_LOOP_RECORDED;
+  if (values == s->sym32.v) s->route_half |= 2;
+  s->route_grid32 = epi_grid<float>(s, s->plan32);
   const uint64_t key = cg32_key(s, values);
   if (key != s->cg32_key) {
     // nothing recorded earlier may still be queued when its graph goes
@@ -2151,6 +2162,7 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   // of 3-DOF node blocks only in FP64: an entry below the diagonal takes its
   // three values from three places there, and FP32 lost by that more than
   // the halved stream gave (63^3 Hex8: 37 us full, 42 us half; FP64 112, 84)
+  s->route_loops = s->route_half = s->route_grid32 = 0;
   s->sym_on = p->method == EHIP_CG && p->precond < EHIP_PRECOND_ILU0 &&
               (s->sho_d == 1 || p->precision == EHIP_FP64);
   // on a lane, of systems the resident loops would take elsewhere: their
@@ -2257,6 +2269,7 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
     if ((rc = mixed_ir(s, c, itol, imax, &inner_total))) return rc;
     rep.outer_iters = s->h_st->pad1;
   } else if (p->precond >= EHIP_PRECOND_ILU0) {
+    s->route_loops = EHIP_LOOP_LAUNCHED;
     if ((rc = ilu_krylov(s, c, p->precond - EHIP_PRECOND_ILU0))) return rc;
   } else {
     Vecs<double> v = make_vecs<double>(s->work, n, p->method, s->x, s->rhs);
@@ -2305,6 +2318,14 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
 
 extern "C" int ehip_solve(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, double *hist) {
   return ehip::solve_impl(s, p, x, r, hist, true);
+}
+
+extern "C" int ehip_solve_route(const ehip_system *s, int *loops, int *half_storage, int *spmv_grid32) {
+  if (!s) return EHIP_EARG;
+  if (loops) *loops = s->route_loops;
+  if (half_storage) *half_storage = s->route_half;
+  if (spmv_grid32) *spmv_grid32 = s->route_grid32;
+  return EHIP_OK;
 }
 
 extern "C" int ehip_get_solution(ehip_system *s, double *x) {

@@ -200,6 +200,14 @@ class System:
         _lib.check(_lib.load().ehip_get_solution(self._h, _ptr(x)), "ehip_get_solution")
         return x
 
+    def solve_route(self):
+        """What the last solve ran: {"loops": the sum of _lib.LOOP_*, "half_storage": 1 (FP64)
+        + 2 (FP32) where half of a symmetric matrix was read, "spmv_grid32": workgroups of the
+        FP32 SpMV steps}"""
+        lo, ha, g = C.c_int(), C.c_int(), C.c_int()
+        _lib.check(_lib.load().ehip_solve_route(self._h, C.byref(lo), C.byref(ha), C.byref(g)), "ehip_solve_route")
+        return {"loops": lo.value, "half_storage": ha.value, "spmv_grid32": g.value}
+
     # ------------------------------------------------------------ ILU(k)
     def ilu_factor(self, order=0):
         """CRS_IncompleteLU of the current Values: (irows, icols, idiag, factors), 1-based."""

@@ -224,6 +224,17 @@ int ehip_dirichlet(ehip_system *s, int nbc, const int *bc_rows, const double *bc
 int ehip_solve(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, double *hist);
 /* Solution currently on the device. */
 int ehip_get_solution(ehip_system *s, double *x);
+/* Which loops and storage the system's last ehip_solve ran: loops is the sum
+ * of EHIP_LOOP_*; half_storage 1 (FP64) + 2 (FP32) where the SpMVs of a CG
+ * solve read only the values at offsets >= 0 of a symmetric stencil matrix;
+ * spmv_grid32 the workgroups of its FP32 SpMV steps (0: none launched).  The
+ * choice changes no FP64 row sum.  Any pointer may be NULL.  No counterpart in
+ * the reference. */
+#define EHIP_LOOP_LAUNCHED 1 /* kernels launched one by one */
+#define EHIP_LOOP_RECORDED 2 /* recorded blocks of them replayed */
+#define EHIP_LOOP_RESIDENT 4 /* a whole sequence in one launch */
+#define EHIP_LOOP_GAVE_UP 8  /* such a launch gave up waiting; the sequence then ran launched */
+int ehip_solve_route(const ehip_system *s, int *loops, int *half_storage, int *spmv_grid32);
 /* One-shot drop-in for a Before-Linsolve hook: host CRS + b in, x out. */
 int ehip_solve_csr(int n, const int *rows, const int *cols, const int *diag, const double *values,
                    const double *b, double *x, const ehip_params *p, ehip_report *r);

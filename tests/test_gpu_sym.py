@@ -148,3 +148,29 @@ def test_recorded_blocks_follow_the_copy_in_use(ehip, first):
         assert (rep["info"], rep["iters"], rep["outer_iters"]) == (1, want["iters"], want["outer_iters"]), seed
         assert np.array_equal(x, y), seed
     s.free()
+
+
+def test_route_names_what_ran(ehip):
+    """ehip_solve_route: 25^3 fits the resident loops (full copy); sampled
+    solves launch; 274 625 rows replay recorded blocks of the half storage,
+    or launch, in FP64, in HUTI's order; a zero right-hand side runs nothing."""
+    small, large = W.poisson_hex8(25, sigma=1.0), W.poisson_hex8(64, sigma=1.0)
+    s, _ = W.build_system(small)
+    vals, rhs = s.values()
+    for precision, mode in FORMS:
+        for every, loops in ((0, _lib.LOOP_RESIDENT), (1 << 30, _lib.LOOP_LAUNCHED)):
+            s.solve(small["kw"], precision=precision, mode=mode, profile_every=every)
+            assert s.solve_route()["loops"] == loops and s.solve_route()["half_storage"] == 0
+    s.solve(W._kw("cg", "ilu0", 1e-10, 500))
+    assert s.solve_route()["loops"] == _lib.LOOP_LAUNCHED
+    s.set_values(vals, 0.0 * rhs)
+    s.solve(small["kw"])
+    assert s.solve_route() == {"loops": 0, "half_storage": 0, "spmv_grid32": 0}
+    s.free()
+    s, _ = W.build_system(large)
+    for precision, mode in FORMS:
+        s.solve(large["kw"], precision=precision, mode=mode)
+        mixed = precision == _lib.MIXED_IR
+        assert s.solve_route()["loops"] == (_lib.LOOP_RECORDED if mixed else _lib.LOOP_LAUNCHED)
+        assert s.solve_route()["half_storage"] == (3 if mixed else 1)
+    s.free()
