@@ -1120,13 +1120,15 @@ static void launch_epi_sellb(ehip_system *s, const T *sv, const T *xin, const Ep
 // after them reduces 4x fewer partials): the fused FP32 CG step on 128^3
 // Hex8 Poisson measured 73.5 against 75.2 us.  The FP64 and node-blocked
 // kernels measured slower that way and keep sell_grid.
-// With the half storage, whose step takes its second reads from the caches
-// and gains from more waves in flight, 2048 (microbenchmark of the step at
-// 128^3, 1024 / 2048 / 4096 workgroups: 36.7 / 33.2 / 31.7 us).
+// On the half storage, whose step takes its second reads from the caches
+// and gains from more waves in flight, 2048: whole mixed solves with 1024 /
+// 2048 / 3072 / 4096 workgroups take 12.3 / 12.0 / 12.4 / 12.7 ms at 101^3 and
+// 25.5 / 24.6 / 24.4 / 24.9 ms at 128^3 (beyond 2048 the vector step, whose
+// workgroups each add up all partial sums, loses what the SpMV gains).
 template <typename T>
-static int epi_sell_grid(const ehip_system *s) {
+static int epi_sell_grid(const ehip_system *s, bool half = false) {
   if (sizeof(T) != 4 || s->sellb_d) return sell_grid(s);
-  return std::min(sell_grid(s), s->sym_ok && s->sym_on ? 2048 : 1024);
+  return std::min(sell_grid(s), half ? 2048 : 1024);
 }
 
 template <int U, class Epi>
@@ -1196,7 +1198,7 @@ __global__ __launch_bounds__(BS) void k_spmv_epi_sym(int n, SymTab tab, const un
 
 template <typename T, int D, class Epi>
 static void launch_epi_sym(ehip_system *s, const T *sv, const T *xin, const Epi &e, const KStateT<T> *st) {
-  const int g = epi_sell_grid<T>(s);
+  const int g = epi_sell_grid<T>(s, true);
   const unsigned long long *zero;
   if constexpr (sizeof(T) == 4) zero = s->sym32.zero; else zero = s->sym64.zero;
   if (s->prof_start)
@@ -1215,10 +1217,15 @@ static int active_fmt(const ehip_system *s) {
   return f == 2 ? (s->sho_ok ? 2 : 0) : (f == 1 && s->sell_ok ? 1 : 0);
 }
 
-// Workgroups (and so published partials) of an epilogue SpMV launch
+// Workgroups (and so published partials) of the epilogue SpMV launch last
+// enqueued: the half storage's when that copy holds the current values
 template <typename T>
 static int epi_grid(const ehip_system *s, const SpmvPlan &p) {
-  return active_fmt<T>(s) ? epi_sell_grid<T>(s) : p.grid;
+  const int fmt = active_fmt<T>(s);
+  if (!fmt) return p.grid;
+  if constexpr (sizeof(T) == 4)
+    return epi_sell_grid<T>(s, fmt == 2 && s->sym_on && s->sym32.good && s->sym32.ver == s->vals32_ver);
+  return epi_sell_grid<T>(s);
 }
 
 // SpMV with epilogue on the system's active format (SELL-64 or CSR stream);

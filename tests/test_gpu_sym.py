@@ -174,3 +174,31 @@ def test_route_names_what_ran(ehip):
         assert s.solve_route()["loops"] == (_lib.LOOP_RECORDED if mixed else _lib.LOOP_LAUNCHED)
         assert s.solve_route()["half_storage"] == (3 if mixed else 1)
     s.free()
+
+
+def test_fp32_workgroups_follow_the_copy_in_use(ehip):
+    """The half storage's FP32 steps run on up to 2048 workgroups; values that
+    are not symmetric and a pinned SELL-64 layout keep the 1024 those kernels
+    are fastest with, and so the sums they always had.  274 625 rows make
+    1080 workgroups."""
+    w = W.poisson_hex8(64, sigma=1.0)
+    s, _ = W.build_system(w)
+    vals, rhs = s.values()
+    unsym = vals.copy()
+    unsym[s.pattern()[1][s.n // 2] - 1] *= 1.0 + 1e-6  # its first entry is not the diagonal
+    got = []
+    for v, fmt, half, grid in ((vals, _lib.SPMV_SELL_SHARED, 3, 1080), (unsym, _lib.SPMV_SELL_SHARED, 0, 1024),
+                               (vals, _lib.SPMV_SELL, 0, 1024), (unsym, _lib.SPMV_SELL, 0, 1024),
+                               (vals, _lib.SPMV_SELL_SHARED, 3, 1080)):
+        s.spmv_set_format(fmt, 0)
+        s.spmv_set_format(fmt, 1)
+        for every in (0, 1 << 30):
+            s.set_values(v, rhs)
+            x, rep = s.solve(w["kw"], precision=_lib.MIXED_IR, mode=_lib.FAST, profile_every=every)
+            assert rep["info"] == 1
+            route = s.solve_route()
+            assert (route["half_storage"], route["spmv_grid32"]) == (half, grid)
+            got.append((x, rep["iters"]))
+    for i, j in ((0, 1), (2, 3), (2, 6), (2, 7), (4, 5), (0, 8), (0, 9)):  # SELL-64 gives the full copy's bits
+        assert got[i][1] == got[j][1] and np.array_equal(got[i][0], got[j][0]), (i, j)
+    s.free()
