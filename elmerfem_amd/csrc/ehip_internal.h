@@ -99,6 +99,7 @@ struct SymCopy {
   unsigned long long *zero = nullptr;
   uint64_t ver = 0;
   bool good = false;
+  int hint = -1;  // slice in which the last whole check failed, for k_sym_probe
 };
 
 }  // namespace ehip
@@ -186,7 +187,7 @@ struct ehip_system {
   int64_t sym_len = 0;                // values of a copy, padding included
   unsigned *sym_mask = nullptr;       // n
   unsigned long long *sym_pm = nullptr; // nslice * K
-  int *sym_flag = nullptr;            // set by a fill that met unequal values
+  int *sym_flag = nullptr;            // 2: set by a probe, a check that met unequal values
   ehip::SymCopy<double> sym64;
   ehip::SymCopy<float> sym32;
   // workspace of the multi-system engine, kept across admissions (a

@@ -2297,6 +2297,7 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
     if ((rc = backscale_system(s, s->rhs, s->x, bscale))) return rc;
   // unscaled FP64 true residual ||b - A x|| / ||b|| and ComputeNorm
   {
+    if (!(s->route_half & 1)) s->sym_on = false;  // not symmetric when scaled: not asked again
     double *out = reinterpret_cast<double *>(&s->st->ts);
     EpiResid er{b0, s->partials, kEpiStride, &s->st->ticket[0], out};
     launch_epi_fin<double>(s, s->plan64, s->vals, s->x, er, (const KState *)nullptr);

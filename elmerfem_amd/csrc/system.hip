@@ -9,8 +9,10 @@
 #include <cstring>
 #include <limits>
 #include <mutex>
+#include <type_traits>
 
 #include "ehip_internal.h"
+#include "launch.h"
 #include "pattern.h"
 #include "spmv_core.h"
 
@@ -430,7 +432,7 @@ static int build_sym(ehip_system *s, const std::vector<int> &ctab) {
   int rc;
   if ((rc = dmalloc(s, (void **)&s->sym_mask, sizeof(unsigned) * (size_t)n)) ||
       (rc = dmalloc(s, (void **)&s->sym_pm, sizeof(unsigned long long) * (size_t)s->nslice * K)) ||
-      (rc = dmalloc(s, (void **)&s->sym_flag, sizeof(int))))
+      (rc = dmalloc(s, (void **)&s->sym_flag, 2 * sizeof(int))))
     return rc;
   hipLaunchKernelGGL(k_sym_masks, dim3(std::min((s->nslice + 3) / 4, 4096)), dim3(256), 0, s->stream, n, s->nslice, D,
                      t, s->sho_off, s->sho_tab, s->sho_mask, s->sym_mask, s->sym_pm);
@@ -881,9 +883,10 @@ template <typename T, int D>
 __global__ __launch_bounds__(256) void k_sym_fill(int n, int nslice, SymTab tab, const int *__restrict__ rows,
                                                   const int *__restrict__ diag, const unsigned *__restrict__ mask,
                                                   const T *__restrict__ in, T *__restrict__ out,
-                                                  unsigned long long *__restrict__ zero, int *flag) {
+                                                  unsigned long long *__restrict__ zero,
+                                                  const int *__restrict__ flag) {
   __shared__ T buf[4][D == 1 ? 64 * kSymMax : 1];
-  if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
+  if (flag[0]) return;  // the probe met unequal values
   const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
   for (int s0 = blockIdx.x * 4; s0 < nslice; s0 += gridDim.x * 4) {
     const int sl = s0 + wv;
@@ -919,15 +922,17 @@ constexpr int kSymU = 7;  // stored values of a lane in flight
 // stored the value is one and takes this row's value instead.  An entry the
 // row does not have must have a zero value stored.  0.35 ms at 128^3 Hex8
 // (FP64), reading Values again and the copy (0.49 with one stored value of a
-// lane in flight).
+// lane in flight).  flag[0]: the probe's finding (nothing is left to do);
+// flag[1] becomes a slice with unequal values, plus one.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void k_sym_check(int n, int nslice, SymTab tab, const int *__restrict__ rows,
                                                    const unsigned *__restrict__ mask,
                                                    const unsigned long long *__restrict__ zero,
                                                    const T *__restrict__ in, T *__restrict__ out, int *flag) {
   __shared__ T buf[4][D == 1 ? 64 * kSymMax : 1];
+  if (flag[0]) return;
   const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
-  bool bad = false;
+  int bad = 0;
   for (int s0 = blockIdx.x * 4; s0 < nslice; s0 += gridDim.x * 4) {
     const int sl = s0 + wv;
     const bool live = sl < nslice;
@@ -961,7 +966,7 @@ __global__ __launch_bounds__(256) void k_sym_check(int n, int nslice, SymTab tab
             if (q0 < 0 || vv[u][d] == have) continue;
             const int q = q0 + d;
             if (on && ((zero[q >> 6] >> (q & 63)) & 1ull)) out[tab.val[tab.K - 1 - k] + D * q + own] = have;
-            else bad |= !(on && zr);
+            else if (!(on && zr)) bad = sl + 1;
           }
           j += on ? D : 0;
         }
@@ -969,39 +974,96 @@ __global__ __launch_bounds__(256) void k_sym_check(int n, int nslice, SymTab tab
     }
     __syncthreads();
   }
-  if (bad) *flag = 1;
+  if (bad) flag[1] = bad;
+}
+
+// Whether values that are not symmetric show it in a sample of the slices,
+// before the copy is filled and checked whole: a system whose values are
+// symmetric to rounding only (or not at all) would pay that at every refresh
+// (0.7 ms a precision at 128^3 Hex8) for a copy it cannot use.  Each row of
+// kSymProbe slices, and of the slice `hint` in which the last whole check
+// failed, compares its entries at offsets < 0 with their mirror images in
+// CRS.  flag[0] is set where k_sym_check would refuse; what this passes is
+// checked whole all the same, so the answer never depends on the sample.
+constexpr int kSymProbe = 256;
+template <typename T, int D>
+__global__ __launch_bounds__(256) void k_sym_probe(int n, int nslice, int hint, SymTab tab,
+                                                   const int *__restrict__ rows, const int *__restrict__ diag,
+                                                   const unsigned *__restrict__ mask, const T *__restrict__ in,
+                                                   int *flag) {
+  const int w = blockIdx.x * 4 + ((int)threadIdx.x >> 6);  // kSymProbe + 1 of them
+  if (w > kSymProbe) return;
+  const int sl = w == kSymProbe ? hint : (int)((long long)nslice * w / kSymProbe);
+  const int r = sl * 64 + ((int)threadIdx.x & 63);
+  if (sl < 0 || r >= n) return;
+  auto zero_row = [&](int q) {
+    for (int j = rows[q]; j < rows[q + 1]; ++j)
+      if (j != diag[q] && in[j] != (T)0) return false;
+    return true;
+  };
+  const unsigned m = mask[r];
+  const int node = r / D, own = r - D * node;
+  int j = rows[r];
+  bool bad = false;
+  for (int k = 0; k < tab.diag; ++k) {
+    const bool on = (m >> k) & 1u;
+    const int up = tab.K - 1 - k, q0 = D * (node + tab.col[k]);
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int q = q0 + d;
+      if (q < 0) continue;
+      const unsigned mq = mask[q];
+      const T have = on ? in[j + d] : (T)0;
+      const T other = (mq >> up) & 1u ? in[rows[q] + D * __popc(mq & ((1u << up) - 1u)) + own] : (T)0;
+      // the rules of k_sym_fill and k_sym_check
+      if (!(have == other) && !(on && (zero_row(r) || zero_row(q)))) bad = true;
+    }
+    j += on ? D : 0;
+  }
+  if (bad) flag[0] = 1;
 }
 
 template <typename T>
 static const T *sym_values(ehip_system *s, SymCopy<T> &c, const T *in, uint64_t ver) {
   if (!s->sym_ok || !s->sym_on) return nullptr;
+  auto failed = [](hipError_t e) {  // reported when the solve takes it
+    if (e != hipSuccess && tl_launch_err == hipSuccess) tl_launch_err = e;
+    return e != hipSuccess;
+  };
   if (c.ver != ver) {
-    if (!c.v) {
-      if (dmalloc(s, (void **)&c.v, sizeof(T) * (size_t)s->sym_len)) return nullptr;
-      if (!c.zero && dmalloc(s, (void **)&c.zero, sizeof(unsigned long long) * (size_t)s->nslice)) return nullptr;
-      // the padding stays zero
-      if (hipMemsetAsync(c.v, 0, sizeof(T) * (size_t)s->sym_len, s->stream) != hipSuccess) return nullptr;
-    }
-    if (!c.zero) return nullptr;
-    const dim3 g(std::min((s->nslice + 3) / 4, 8192)), bs(256);
-    const SymTab &t = s->sym_tab;
-    if (s->sho_d == 3) {
-      hipLaunchKernelGGL((k_sym_fill<T, 3>), g, bs, 0, s->stream, s->n, s->nslice, t, s->rows, s->diag, s->sym_mask, in,
-                         c.v, c.zero, s->sym_flag);
-      hipLaunchKernelGGL((k_sym_check<T, 3>), g, bs, 0, s->stream, s->n, s->nslice, t, s->rows, s->sym_mask, c.zero, in,
-                         c.v, s->sym_flag);
-    } else {
-      hipLaunchKernelGGL((k_sym_fill<T, 1>), g, bs, 0, s->stream, s->n, s->nslice, t, s->rows, s->diag, s->sym_mask, in,
-                         c.v, c.zero, s->sym_flag);
-      hipLaunchKernelGGL((k_sym_check<T, 1>), g, bs, 0, s->stream, s->n, s->nslice, t, s->rows, s->sym_mask, c.zero, in,
-                         c.v, s->sym_flag);
-    }
-    int bad = 1;
-    if (hipMemcpyAsync(&bad, s->sym_flag, sizeof(int), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-        hipStreamSynchronize(s->stream) != hipSuccess)
-      return nullptr;
     c.ver = ver;
-    c.good = bad == 0;
+    c.good = false;
+    if (!c.v) {
+      if (!c.zero && dmalloc(s, (void **)&c.zero, sizeof(unsigned long long) * (size_t)s->nslice)) return nullptr;
+      if (dmalloc(s, (void **)&c.v, sizeof(T) * (size_t)s->sym_len)) return nullptr;
+      // the padding stays zero
+      if (failed(hipMemsetAsync(c.v, 0, sizeof(T) * (size_t)s->sym_len, s->stream))) return nullptr;
+    }
+    const dim3 g(std::min((s->nslice + 3) / 4, 8192)), gp(kSymProbe / 4 + 1), bs(256);
+    const SymTab &t = s->sym_tab;
+    int *flag = s->sym_flag;
+    if (failed(hipMemsetAsync(flag, 0, 2 * sizeof(int), s->stream))) return nullptr;
+    auto run = [&](auto d) {
+      constexpr int D = decltype(d)::value;
+      hipLaunchKernelGGL((k_sym_probe<T, D>), gp, bs, 0, s->stream, s->n, s->nslice, c.hint, t, s->rows, s->diag,
+                         s->sym_mask, in, flag);
+      hipLaunchKernelGGL((k_sym_fill<T, D>), g, bs, 0, s->stream, s->n, s->nslice, t, s->rows, s->diag, s->sym_mask, in,
+                         c.v, c.zero, flag);
+      hipLaunchKernelGGL((k_sym_check<T, D>), g, bs, 0, s->stream, s->n, s->nslice, t, s->rows, s->sym_mask, c.zero, in,
+                         c.v, flag);
+    };
+    if (s->sho_d == 3) run(std::integral_constant<int, 3>{});
+    else run(std::integral_constant<int, 1>{});
+    int bad[2] = {1, 0};
+    if (failed(hipGetLastError()) ||
+        failed(hipMemcpyAsync(bad, flag, sizeof(bad), hipMemcpyDeviceToHost, s->stream)) ||
+        failed(hipStreamSynchronize(s->stream)))
+      return nullptr;
+    c.good = !bad[0] && !bad[1];
+    if (bad[1]) {
+      c.hint = bad[1] - 1;
+      s->route_half |= 4;
+    }
   }
   return c.good ? c.v : nullptr;
 }

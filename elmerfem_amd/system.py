@@ -202,7 +202,8 @@ class System:
 
     def solve_route(self):
         """What the last solve ran: {"loops": the sum of _lib.LOOP_*, "half_storage": 1 (FP64)
-        + 2 (FP32) where half of a symmetric matrix was read, "spmv_grid32": workgroups of the
+        + 2 (FP32) where half of a symmetric matrix was read + 4 where all values were
+        compared and are not symmetric, "spmv_grid32": workgroups of the
         FP32 SpMV steps}"""
         lo, ha, g = C.c_int(), C.c_int(), C.c_int()
         _lib.check(_lib.load().ehip_solve_route(self._h, C.byref(lo), C.byref(ha), C.byref(g)), "ehip_solve_route")

@@ -226,7 +226,9 @@ int ehip_solve(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
 int ehip_get_solution(ehip_system *s, double *x);
 /* Which loops and storage the system's last ehip_solve ran: loops is the sum
  * of EHIP_LOOP_*; half_storage 1 (FP64) + 2 (FP32) where the SpMVs of a CG
- * solve read only the values at offsets >= 0 of a symmetric stencil matrix;
+ * solve read only the values at offsets >= 0 of a symmetric stencil matrix,
+ * + 4 where all values were compared and found not symmetric (values that
+ * a sample of them shows not to be are not compared any further);
  * spmv_grid32 the workgroups of its FP32 SpMV steps (0: none launched).  The
  * choice changes no FP64 row sum.  Any pointer may be NULL.  No counterpart in
  * the reference. */
