@@ -204,7 +204,6 @@ struct ehip_system {
   int sho_wmax = 0;                   // entries of the longest offset list
   bool resident_on = false;           // the solve in progress may use them
   void *res_buf = nullptr;
-  size_t res_bytes = 0;
   // what the last solve ran (ehip_solve_route)
   int route_loops = 0, route_half = 0, route_grid32 = 0;
   uint64_t vals_ver = 1, vals32_ver = 1, sell64_ver = 0, sell32_ver = 0;
@@ -424,6 +423,7 @@ template <typename T>
 int resident_cg(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du);
 template <typename T>
 int resident_bicgstab(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du);
+bool resident_buffers(ehip_system *s);  // false: no memory for their buffers
 std::mutex &resident_lock(const ehip_system *s);
 
 // SpMV launch sampling (ehip_params.profile_every)

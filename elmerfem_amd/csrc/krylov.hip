@@ -1358,6 +1358,10 @@ static int nvecs(int method) { return method == EHIP_CG ? 6 : 10; }
 template <typename T>
 static int run_resident(ehip_system *s, SolveCtx &c, const Vecs<T> &v, KStateT<T> *st, KStateT<T> *hst, bool faithful,
                         double *hist, const T *du, int it0, bool *resident) {
+  if (!resident_buffers(s)) {  // no memory for them: the launched loop needs none
+    *resident = false;
+    return EHIP_OK;
+  }
   std::lock_guard<std::mutex> lk(resident_lock(s));
   int rc;
   if ((rc = (c.method == EHIP_CG ? resident_cg<T> : resident_bicgstab<T>)(s, v, st, faithful, hist, du)) || (rc = read_state(s, st, hst))) return rc;
@@ -1636,13 +1640,13 @@ static const float *cg32_values(ehip_system *s) {
   return half ? half : sho_values32(s);
 }
 
-// What a recorded block bakes in: buffers, SpMV layout and schedule.  The
-// values' address tells which layout the block's kernels read: one system
-// may be solved on the half storage and, elsewhere, on the full copy, and
-// only the copy in use is up to date.
+// What a recorded block bakes in: buffers, SpMV layout and schedule.  One
+// system may be solved on the half storage and, elsewhere, on the full copy,
+// and only the copy in use is up to date; a copy may lie where the other was.
 static uint64_t cg32_key(const ehip_system *s, const float *values) {
   const uint64_t parts[] = {(uint64_t)(uintptr_t)s->work32, (uint64_t)(uintptr_t)s->vals32,
-                            (uint64_t)(uintptr_t)values, (uint64_t)epi_grid<float>(s, s->plan32),
+                            (uint64_t)(uintptr_t)values, (uint64_t)(values == s->sym32.v),
+                            (uint64_t)epi_grid<float>(s, s->plan32),
                             (uint64_t)(uintptr_t)s->partials32,
                             (uint64_t)(uintptr_t)s->st32, (uint64_t)(uintptr_t)s->plan32.chunk_row,
                             (uint64_t)s->fmt32, (uint64_t)s->plan32.block, (uint64_t)s->plan32.nb,

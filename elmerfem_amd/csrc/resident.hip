@@ -786,22 +786,23 @@ bool resident_fits(ehip_system *s, bool cg, bool faithful) {
   return win + (int64_t)sizeof(ResShared<T>) + 64 <= kResLds;
 }
 
-// Enqueues the sequence and its commit; the caller holds resident_lock from
-// here until it has read the state back, whose ticket[3] tells that the
+static size_t vec_len(int n) { return ((size_t)n + 63) / 64 * 64; }
+
+// The exchange words and vectors, allocated at first use.
+bool resident_buffers(ehip_system *s) {
+  const size_t need =
+      (sizeof(Word) * (kW1 + kW2) + sizeof(KState) + 256) + 9 * vec_len(s->n) * sizeof(double);
+  if (!s->res_buf && dmalloc(s, &s->res_buf, need)) return false;
+  return true;
+}
+
+// Enqueues the sequence and its commit; the caller has the buffers and holds
+// resident_lock from here until it has read the state back, whose ticket[3] tells that the
 // grid gave up and nothing changed.
 template <typename T, bool CG>
 static int resident_run(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du) {
   const int n = s->n;
-  int rc;
-  const size_t vec = ((size_t)n + 63) / 64 * 64;
-  const size_t need = (sizeof(Word) * (kW1 + kW2) + sizeof(KState) + 256) + 9 * vec * sizeof(double);
-  if (s->res_bytes < need) {
-    if (s->res_buf) dfree(s, s->res_buf, s->res_bytes);
-    s->res_buf = nullptr;
-    s->res_bytes = 0;
-    if ((rc = dmalloc(s, &s->res_buf, need))) return rc;
-    s->res_bytes = need;
-  }
+  const size_t vec = vec_len(n);
   char *p = (char *)s->res_buf;
   ResArgs<T> a{};
   a.w1 = (Word *)p;

@@ -29,11 +29,24 @@ void set_error(const char *fmt, ...) {
 
 int max_grid() { return 2048; }
 
+// Tests of what runs without memory: this thread's next `count` device
+// allocations of lo to hi bytes ask for more than there is.
+static thread_local struct {
+  size_t lo, hi;
+  int count;
+} tl_fail = {0, 0, 0};
+
 int dmalloc(ehip_system *s, void **p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) return EHIP_OK;
-  hipError_t e = hipMalloc(p, bytes);
+  size_t ask = bytes;
+  if (tl_fail.count > 0 && bytes >= tl_fail.lo && bytes <= tl_fail.hi) {
+    --tl_fail.count;
+    ask = (size_t)1 << 60;
+  }
+  hipError_t e = hipMalloc(p, ask);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // reported here; a caller that can do without goes on
     set_error("hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
     *p = nullptr;
     return EHIP_ENOMEM;
@@ -429,11 +442,16 @@ static int build_sym(ehip_system *s, const std::vector<int> &ctab) {
     t.val[k] = (int)(ld * std::abs(k - K / 2) + pad + (o < 0 ? (int64_t)o * D * D : 0));
   }
   s->sym_len = len;
-  int rc;
-  if ((rc = dmalloc(s, (void **)&s->sym_mask, sizeof(unsigned) * (size_t)n)) ||
-      (rc = dmalloc(s, (void **)&s->sym_pm, sizeof(unsigned long long) * (size_t)s->nslice * K)) ||
-      (rc = dmalloc(s, (void **)&s->sym_flag, 2 * sizeof(int))))
-    return rc;
+  if (dmalloc(s, (void **)&s->sym_mask, sizeof(unsigned) * (size_t)n) ||
+      dmalloc(s, (void **)&s->sym_pm, sizeof(unsigned long long) * (size_t)s->nslice * K) ||
+      dmalloc(s, (void **)&s->sym_flag, 2 * sizeof(int))) {
+    // no memory for it: the full copy serves
+    dfree(s, s->sym_mask, sizeof(unsigned) * (size_t)n);
+    dfree(s, s->sym_pm, sizeof(unsigned long long) * (size_t)s->nslice * K);
+    s->sym_mask = nullptr;
+    s->sym_pm = nullptr;
+    return EHIP_OK;
+  }
   hipLaunchKernelGGL(k_sym_masks, dim3(std::min((s->nslice + 3) / 4, 4096)), dim3(256), 0, s->stream, n, s->nslice, D,
                      t, s->sho_off, s->sho_tab, s->sho_mask, s->sym_mask, s->sym_pm);
   EHIP_HIP_TRY(hipGetLastError());
@@ -840,9 +858,28 @@ static void sho_gather(ehip_system *s, const T *in, T *out) {
                        s->sho_mask, s->sho_off, in, out);
 }
 
+// A full copy's memory; a half copy that the solve in progress does not read
+// gives way to it.
+static int alloc_full(ehip_system *s, void **p, size_t bytes) {
+  int rc = dmalloc(s, p, bytes);
+  auto release = [&](auto &c) {
+    if (!c.v || (s->sym_on && c.good)) return;
+    dfree(s, c.v, sizeof(*c.v) * (size_t)s->sym_len);
+    c.v = nullptr;
+    c.good = false;
+    c.ver = 0;
+  };
+  if (rc && (s->sym64.v || s->sym32.v)) {
+    release(s->sym64);
+    release(s->sym32);
+    rc = dmalloc(s, p, bytes);
+  }
+  return rc;
+}
+
 const double *sho_values64(ehip_system *s) {
   if (!s->sho64) {
-    if (dmalloc(s, (void **)&s->sho64, sizeof(double) * s->sho_nnz)) return nullptr;
+    if (alloc_full(s, (void **)&s->sho64, sizeof(double) * s->sho_nnz)) return nullptr;
     s->sho64_ver = 0;
   }
   if (s->sho64_ver != s->vals_ver) {
@@ -854,7 +891,7 @@ const double *sho_values64(ehip_system *s) {
 
 const float *sho_values32(ehip_system *s) {
   if (!s->sho32) {
-    if (dmalloc(s, (void **)&s->sho32, sizeof(float) * s->sho_nnz)) return nullptr;
+    if (alloc_full(s, (void **)&s->sho32, sizeof(float) * s->sho_nnz)) return nullptr;
     s->sho32_ver = 0;
   }
   if (s->sho32_ver != s->vals32_ver) {
@@ -1327,6 +1364,13 @@ int ehip_system_get_values(ehip_system *s, double *values, double *rhs) {
   EHIP_HIP_TRY(hipStreamSynchronize(s->stream));
   if (values) EHIP_HIP_TRY(hipMemcpy(values, s->vals, sizeof(double) * s->nnz, hipMemcpyDeviceToHost));
   if (rhs) EHIP_HIP_TRY(hipMemcpy(rhs, s->rhs, sizeof(double) * s->n, hipMemcpyDeviceToHost));
+  return EHIP_OK;
+}
+
+int ehip_internal_fail_allocs(int64_t lo, int64_t hi, int count) {
+  tl_fail.lo = (size_t)lo;
+  tl_fail.hi = (size_t)hi;
+  tl_fail.count = count;
   return EHIP_OK;
 }
 

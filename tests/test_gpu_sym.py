@@ -7,6 +7,8 @@ SELL-64 layout: for assembled matrices with Dirichlet rows (zero rows whose
 columns stay), for symmetric Dirichlet elimination, for 3-DOF node blocks,
 and for values that are not symmetric, which keep the full copy.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -242,3 +244,61 @@ def test_unsymmetric_values_are_told_from_a_sample(ehip, kind, precision, mode):
         assert halves(one) == 0
         assert halves(vals) == half
     s.free()
+
+
+def _fail_allocs(lo, hi, count):
+    assert _lib.load().ehip_internal_fail_allocs(C.c_int64(lo), C.c_int64(hi), count) == 0
+
+
+def test_solves_do_without_the_memory_of_a_faster_path(ehip):
+    """Where there is no memory for the resident loops' buffers, the half
+    storage's masks (system creation) or values, a solve runs as it would
+    without them, to the same FP64 bits; and a half copy that the solve does
+    not read gives way to the full copy it needs."""
+    w = W.poisson_hex8(25, sigma=1.0)
+    s, _ = W.build_system(w)
+    vals, rhs = s.values()
+    how = dict(precision=_lib.FP64, mode=_lib.FAST)
+    x, _ = s.solve(w["kw"], profile_every=1 << 30, **how)  # all buffers but the resident loops'
+    try:
+        for expect in (_lib.LOOP_LAUNCHED, _lib.LOOP_RESIDENT):
+            if expect == _lib.LOOP_LAUNCHED:
+                _fail_allocs(72 * s.n, 1 << 40, 1)
+            s.set_values(vals, rhs)
+            y, rep = s.solve(w["kw"], **how)
+            assert rep["info"] == 1 and s.solve_route()["loops"] == expect
+            assert np.array_equal(x, y)
+        s.free()
+
+        w = W.poisson_hex8(64, sigma=1.0)
+        masks = 8 * 27 * ((65 ** 3 + 63) // 64)
+        _fail_allocs(masks, masks, 1)
+        got = []
+        for half in (0, 1):
+            s, _ = W.build_system(w)
+            _fail_allocs(0, 0, 0)
+            vals, rhs = s.values()
+            got.append(s.solve(w["kw"], **how)[0])
+            assert s.solve_route()["half_storage"] == half
+            if not half:
+                s.free()
+        assert np.array_equal(*got)
+        # the full FP64 copy, wanted by BiCGStab, takes the place of the half one
+        full = 8 * s.spmv_shared_layout()["entries"]
+        before = s.device_bytes()
+        _fail_allocs(full, full, 1)
+        s.set_values(vals, rhs)
+        _, rep = s.solve(W._kw("bicgstab", "diagonal", 1e-10, 3000), **how)
+        assert rep["info"] == 1
+        assert s.device_bytes() < before + full
+        # and CG goes on with the full copy when the half one finds no memory
+        _fail_allocs(full // 4, full, 1)
+        s.set_values(vals, rhs)
+        y, _ = s.solve(w["kw"], **how)
+        assert s.solve_route()["half_storage"] == 0 and np.array_equal(y, got[0])
+        s.set_values(vals, rhs)
+        y, _ = s.solve(w["kw"], **how)
+        assert s.solve_route()["half_storage"] == 1 and np.array_equal(y, got[0])
+        s.free()
+    finally:
+        _fail_allocs(0, 0, 0)
