@@ -2174,6 +2174,10 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   // three values from three places there, and FP32 lost by that more than
   // the halved stream gave (63^3 Hex8: 37 us full, 42 us half; FP64 112, 84)
   s->route_loops = s->route_half = s->route_grid32 = 0;
+  struct Leave {  // other callers of the SpMVs here (the engine's reports) have full copies
+    ehip_system *s;
+    ~Leave() { s->sym_on = s->resident_on = false; }
+  } leave{s};
   s->sym_on = p->method == EHIP_CG && p->precond < EHIP_PRECOND_ILU0 &&
               (s->sho_d == 1 || p->precision == EHIP_FP64);
   // on a lane, of systems the resident loops would take elsewhere: their

@@ -302,3 +302,23 @@ def test_solves_do_without_the_memory_of_a_faster_path(ehip):
         s.free()
     finally:
         _fail_allocs(0, 0, 0)
+
+
+def test_half_storage_ends_with_the_solve(ehip):
+    """The engine reports on its full copies, whatever a direct solve before
+    allowed: after one that left early (zero right-hand side) a batched solve
+    of a system over the size limit allocates no half copy."""
+    from elmerfem_amd.batch import solve_batch
+    w = W.poisson_hex8(64, sigma=1.0)
+    held = []
+    for before in (False, True):
+        s, _ = W.build_system(w)
+        vals, rhs = s.values()
+        s.set_values(vals, 0.0 * rhs)
+        s.solve(w["kw"] if before else W._kw("bicgstab"))
+        s.set_values(vals, rhs)
+        _, reps, _ = solve_batch([s], w["kw"], mode=_lib.FAST)
+        assert reps[0]["info"] == 1
+        held.append(s.device_bytes())
+        s.free()
+    assert held[0] == held[1]
