@@ -4,7 +4,6 @@
 
 #include <cstdint>
 #include <cstdlib>
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -206,6 +205,7 @@ struct ehip_system {
   void *res_buf = nullptr;
   // what the last solve ran (ehip_solve_route)
   int route_loops = 0, route_half = 0, route_grid32 = 0;
+  int resident_test = 0;              // ehip_internal_resident
   uint64_t vals_ver = 1, vals32_ver = 1, sell64_ver = 0, sell32_ver = 0;
   double *vals = nullptr, *rhs = nullptr, *x = nullptr;
   float *vals32 = nullptr;
@@ -424,7 +424,11 @@ int resident_cg(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful,
 template <typename T>
 int resident_bicgstab(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du);
 bool resident_buffers(ehip_system *s);  // false: no memory for their buffers
-std::mutex &resident_lock(const ehip_system *s);
+// Room on the device for a resident loop of g workgroups, held from before
+// its launch until its state is read.
+bool resident_admit(const ehip_system *s, int g);
+void resident_release(const ehip_system *s, int g, bool gave_up);
+int resident_groups(int n, bool cg);
 
 // SpMV launch sampling (ehip_params.profile_every)
 void prof_begin(ehip_system *s);

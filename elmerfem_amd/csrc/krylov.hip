@@ -1352,9 +1352,10 @@ static Vecs<T> make_vecs(T *w, int n, int method, T *x, T *b) {
 static int nvecs(int method) { return method == EHIP_CG ? 6 : 10; }
 
 // A Krylov sequence in one launch (resident.hip), until it stops; its state in
-// hst.  *resident = false: the grid gave up waiting (the device is shared
-// with something that kept part of it off the chip) and the vectors and the
-// state are as before, for the launched loop to go on from.
+// hst.  *resident = false: there was no room for it, or the grid gave up
+// waiting (the device is shared with something that kept part of it off the
+// chip), and the vectors and the state are as before, for the launched loop
+// to go on from.
 template <typename T>
 static int run_resident(ehip_system *s, SolveCtx &c, const Vecs<T> &v, KStateT<T> *st, KStateT<T> *hst, bool faithful,
                         double *hist, const T *du, int it0, bool *resident) {
@@ -1362,9 +1363,15 @@ static int run_resident(ehip_system *s, SolveCtx &c, const Vecs<T> &v, KStateT<T
     *resident = false;
     return EHIP_OK;
   }
-  std::lock_guard<std::mutex> lk(resident_lock(s));
-  int rc;
-  if ((rc = (c.method == EHIP_CG ? resident_cg<T> : resident_bicgstab<T>)(s, v, st, faithful, hist, du)) || (rc = read_state(s, st, hst))) return rc;
+  const int g = resident_groups(s->n, c.method == EHIP_CG);
+  if (!resident_admit(s, g)) {  // others hold the chip, or use it
+    *resident = false;
+    return EHIP_OK;
+  }
+  int rc = (c.method == EHIP_CG ? resident_cg<T> : resident_bicgstab<T>)(s, v, st, faithful, hist, du);
+  if (!rc) rc = read_state(s, st, hst);
+  resident_release(s, g, !rc && hst->ticket[3] != 0);
+  if (rc) return rc;
   *resident = hst->ticket[3] == 0;
   s->route_loops |= *resident ? EHIP_LOOP_RESIDENT : EHIP_LOOP_GAVE_UP;
   if (*resident) c.spmv += std::max(0, hst->iter - it0) * ((faithful ? 2 : 1) + (c.method == EHIP_CG ? 0 : 1));
@@ -2185,7 +2192,8 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   if (tl_shared_device && s->n <= 262144) s->sym_on = false;
   // one launch per sequence where the rows fit the chip (not for callers
   // without runtime objects of their own, nor when launches are sampled)
-  s->resident_on = events && !tl_shared_device && p->profile_every <= 0 && p->precond < EHIP_PRECOND_ILU0;
+  s->resident_on = events && !tl_shared_device && p->profile_every <= 0 && p->precond < EHIP_PRECOND_ILU0 &&
+                   s->resident_test != 1;
   if (s->sym_on && s->resident_on &&
       resident_fits<double>(s, true, p->mode == EHIP_FAITHFUL && p->precision == EHIP_FP64))
     s->sym_on = false;  // that loop reads the full copy

@@ -41,14 +41,20 @@
 // up to 920 fits the LDS (1 970 with one window) where CG's 1024 rows in a
 // row take 3 680 (7 880).
 //
-// Waiting.  All workgroups of the grid (at most 256, one per CU) must be on
-// the chip at once.  One such launch at a time runs on a device (a host lock),
-// other kernels end by themselves, and every wait is bounded: a thread that
-// polls past kSpins gives up for the whole grid.  Results go to separate
+// Waiting.  All workgroups of the grid must be on the chip at once.  A
+// workgroup (1024 threads of at most 128 registers, at most 156 of 160 KB of
+// LDS) fits any CU that no other one holds, so the process counts CUs: loops
+// run side by side while every XCD has a CU for each workgroup of theirs that
+// it can be given (resident_admit); one that finds no room runs launched.
+// Other kernels end by themselves, and every wait is bounded: a thread that
+// polls past kSpins (a quarter of a second or so) gives up for the whole
+// grid.  That is for what the count does not see, other processes and CU
+// masks; it does not happen again for kRest.  Results go to separate
 // buffers, which a commit launch copies only if nobody gave up, so the
 // launched loop then takes over from the unchanged vectors.
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <mutex>
 
 #include "cg_steps.h"
@@ -60,9 +66,10 @@ namespace ehip {
 namespace {
 
 constexpr int kResRows = 1024;    // rows (and threads) of a workgroup
-constexpr int kResGroups = 256;   // one per CU
+constexpr int kResGroups = 256;   // at most, one per CU
 constexpr int kResLds = 156 * 1024;
-constexpr int kSpins = 1 << 20;
+constexpr int kSpins = 1 << 18;
+constexpr int kCusPerXcd = 32;
 typedef unsigned long long Word;
 
 __device__ __forceinline__ Word ld_word(const Word *p) {
@@ -745,17 +752,62 @@ __global__ __launch_bounds__(256) void k_resident_commit(int n, Vecs<T> v, Vecs<
   if (blockIdx.x == 0 && threadIdx.x == 0) *st = *st_out;
 }
 
-__global__ void k_resident_clear(Word *w, int nw, int *gave_up, unsigned *mark) {
+__global__ void k_resident_clear(Word *w, int nw, int *gave_up, unsigned *mark, int give_up) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nw; i += gridDim.x * blockDim.x) w[i] = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *gave_up = 0;
+    *gave_up = give_up;
     *mark = 0;
   }
 }
 
-static std::mutex g_resident_mu[16];
+// One device, as this process's solves use it.
+struct Device {
+  std::mutex mu;
+  int cus = 0;     // of the device; 0: not asked yet
+  int held = 0;    // CUs of an XCD that resident loops may hold
+  std::chrono::steady_clock::time_point rest{};  // no resident loop before
+};
+static Device g_device[64];
+static Device &device(const ehip_system *s) { return g_device[s->dev & 63]; }
 
-std::mutex &resident_lock(const ehip_system *s) { return g_resident_mu[s->dev & 15]; }
+// After a grid gave up, how long solves on the device stay launched.
+constexpr std::chrono::seconds kRest(10);
+
+// Workgroups go to the XCDs in turn, so a grid of g takes at most ceil(g / 8)
+// CUs of any one of them.
+static int cus_of_xcd(const Device &d, int g) {
+  const int xcds = std::max(1, d.cus / kCusPerXcd);
+  return (g + xcds - 1) / xcds;
+}
+
+// Room for a resident loop of g workgroups.  Four host threads that solve
+// together, resident loops one at a time / as many as there is room for, the
+// rest launched / all launched, a round of four solves: 17^3 Hex8 in HUTI's
+// order 2.9 / 2.0 / 3.8 ms, 47^3 12.2 / 7.6 / 10.7 ms, 60^3 mixed 12.1 / 9.1 /
+// 9.3 ms, 301^2 Quad4 BiCGStab 84 / 25 / 43 ms (keeping large loops off beside
+// other solves was never better).
+bool resident_admit(const ehip_system *s, int g) {
+  Device &d = device(s);
+  std::lock_guard<std::mutex> lk(d.mu);
+  if (!d.cus && hipDeviceGetAttribute(&d.cus, hipDeviceAttributeMultiprocessorCount, s->dev) != hipSuccess) {
+    d.cus = 0;
+    return false;
+  }
+  const int xcds = std::max(1, d.cus / kCusPerXcd), need = cus_of_xcd(d, g);
+  if (d.held + need > d.cus / xcds) return false;
+  if (std::chrono::steady_clock::now() < d.rest) return false;
+  d.held += need;
+  return true;
+}
+void resident_release(const ehip_system *s, int g, bool gave_up) {
+  Device &d = device(s);
+  std::lock_guard<std::mutex> lk(d.mu);
+  d.held -= cus_of_xcd(d, g);
+  if (gave_up) d.rest = std::chrono::steady_clock::now() + kRest;
+}
+
+// CG: 1024 rows to a workgroup; BiCGStab: the launched vector steps' grid
+int resident_groups(int n, bool cg) { return cg ? (n + kResRows - 1) / kResRows : vec_grid(n); }
 
 // Words of the exchanges: three SpMV values of up to 1024 groups, two
 // vector values of up to 1024 tiles, two words each.
@@ -796,9 +848,9 @@ bool resident_buffers(ehip_system *s) {
   return true;
 }
 
-// Enqueues the sequence and its commit; the caller has the buffers and holds
-// resident_lock from here until it has read the state back, whose ticket[3] tells that the
-// grid gave up and nothing changed.
+// Enqueues the sequence and its commit; the caller has the buffers and is
+// admitted from here until it has read the state back, whose ticket[3] tells
+// that the grid gave up and nothing changed.
 template <typename T, bool CG>
 static int resident_run(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du) {
   const int n = s->n;
@@ -828,8 +880,7 @@ static int resident_run(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool f
   a.nslice = s->nslice;
   a.ngroups = (s->nslice + 3) / 4;
   a.spmv_grid = sell_grid(s);
-  // CG: 1024 rows to a workgroup; BiCGStab: the launched vector steps' grid
-  const int g = CG ? (n + kResRows - 1) / kResRows : vec_grid(n);
+  const int g = resident_groups(n, CG);
   a.vec_grid = CG ? fused_grid(n) : g;
   a.hist = hist;
   a.du = du;
@@ -855,7 +906,8 @@ static int resident_run(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool f
   }
   if (!a.vals) return EHIP_ENOMEM;
   const size_t lds = (size_t)window(CG, a.halo) * sizeof(T) * (faithful ? 2 : 1);
-  hipLaunchKernelGGL(k_resident_clear, dim3(16), dim3(256), 0, s->stream, a.w1, kW1 + kW2, a.gave_up, &st->ticket[3]);
+  hipLaunchKernelGGL(k_resident_clear, dim3(16), dim3(256), 0, s->stream, a.w1, kW1 + kW2, a.gave_up, &st->ticket[3],
+                     s->resident_test == 2 ? 1 : 0);
 #define EHIP_RES(F, KW)                                                                                            \
   if constexpr (CG) {                                                                                              \
     if (faithful) hipLaunchKernelGGL((k_resident_cg<T, F, KW, true>), dim3(g), dim3(kResRows), lds, s->stream, a); \
@@ -885,6 +937,18 @@ int resident_cg(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful,
 template <typename T>
 int resident_bicgstab(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du) {
   return resident_run<T, false>(s, v, st, faithful, hist, du);
+}
+
+// Tests: mode 0 as usual, 1 launched loops only, 2 every grid is told that a
+// thread of its gave up (it ends as ever and commits nothing).  Ends the
+// device's rest.
+extern "C" int ehip_internal_resident(ehip_system *s, int mode) {
+  if (!s) return EHIP_EARG;
+  s->resident_test = mode;
+  Device &d = device(s);
+  std::lock_guard<std::mutex> lk(d.mu);
+  d.rest = {};
+  return EHIP_OK;
 }
 
 template bool resident_fits<double>(ehip_system *, bool, bool);
