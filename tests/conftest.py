@@ -12,6 +12,14 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs through libehip's C ABI)")
 
 
+def launched_only(system):
+    """Keeps a system's solves off the resident loops, which take most systems
+    of at most 262 144 rows, for tests of the launched and recorded ones."""
+    import ctypes as C
+    from elmerfem_amd import _lib
+    assert _lib.load().ehip_internal_resident(system._h, C.c_int(1)) == 0
+
+
 @pytest.fixture(scope="session")
 def ehip():
     """libehip initialised on device 0.  GPU tests fail (not skip) when the

@@ -14,6 +14,7 @@ import pytest
 import oracle_lib as O
 from elmerfem_amd import _lib, workloads as W
 from elmerfem_amd.system import System, solve_csr
+from conftest import launched_only
 from golden.golden_cases import CASES, assembled_case
 
 pytestmark = pytest.mark.gpu
@@ -649,11 +650,13 @@ def test_mixed_graph_replay_equals_direct_launches(ehip, case):
     solves (graphs replayed from the cache)."""
     w, pat, vals, rhs, rows = assembled_case(CASES[case])
     s = System.from_csr(pat.rows, pat.cols, pat.diag)
+    launched_only(s)
     out = []
     for prof in (1, 0, 0, 1):
         s.set_values(vals, rhs)
         x, rep = s.solve(w["kw"], precision=_lib.MIXED_IR, mode=_lib.FAST, profile_every=prof)
         assert rep["info"] == 1
+        assert s.solve_route()["loops"] == (_lib.LOOP_LAUNCHED if prof else _lib.LOOP_RECORDED)
         out.append((x, rep["iters"]))
     for x, it in out[1:]:
         assert it == out[0][1] and np.array_equal(x, out[0][0])
@@ -671,11 +674,13 @@ def test_mixed_folded_steps_equal_unfolded(ehip, case, fmt, monkeypatch):
     s = System.from_csr(pat.rows, pat.cols, pat.diag)
     s.set_values(vals, rhs)
     set_format(s, fmt)
+    launched_only(s)
     out = []
     for fold in ("1", "0", "1"):
         monkeypatch.setenv("EHIP_CG_FOLD", fold)
         s.set_values(vals, rhs)
         x, rep = s.solve(w["kw"], precision=_lib.MIXED_IR, mode=_lib.FAST, true_residual_stop=True)
+        assert s.solve_route()["loops"] == _lib.LOOP_RECORDED
         assert rep["info"] == 1 and rep["res_true"] <= RES_BAR
         out.append((x, rep["iters"], rep["outer_iters"]))
     for x, it, up in out[1:]:

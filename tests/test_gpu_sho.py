@@ -15,6 +15,7 @@ import pytest
 import oracle_lib as O
 from elmerfem_amd import _lib, mesh as M, workloads as W
 from elmerfem_amd.system import System
+from conftest import launched_only
 
 pytestmark = pytest.mark.gpu
 
@@ -313,7 +314,14 @@ def test_cached_and_streamed_value_loads_same_bits(ehip, monkeypatch, precision,
         vals, rhs = s.values()
         y64 = s.spmv(u)
         assert np.array_equal(y64, oracle_spmv(rows, cols, vals, u[:s.n]))
+        # one value made unequal to its mirror image keeps the full copy, and
+        # only launched loops read it with this kind of load
+        vals[rows[s.n // 2] - 1] *= 1.0 + 1e-6
+        s.set_values(vals, rhs)
+        launched_only(s)
         x, rep = s.solve(w["kw"], precision=precision, mode=mode, true_residual_stop=True)
+        route = s.solve_route()
+        assert route["half_storage"] & 3 == 0 and not route["loops"] & _lib.LOOP_RESIDENT
         assert rep["info"] == 1 and rep["res_true"] <= 1e-10, rep
         y32 = s.spmv(u, precision=1) if precision == _lib.MIXED_IR else None
         got.append((y64, y32, x, rep["iters"], rep["outer_iters"]))

@@ -1,9 +1,9 @@
 """Half storage of symmetric stencil matrices in CG solves.
 
-A CG solve of a system over 16 MB of FP64 values on a slice-shared-offset
-pattern reads only the values at offsets >= 0.  Row sums keep the CRS order
-and the launches their workgroups, so whole solves give the bits of the
-SELL-64 layout: for assembled matrices with Dirichlet rows (zero rows whose
+A launched CG solve of a system over 16 MB of FP64 values on a slice-shared-
+offset pattern reads only the values at offsets >= 0.  Row sums keep the CRS
+order and the launches (of FP32 steps up to 1024 workgroups) their grid, so
+whole solves give the bits of the SELL-64 layout: for assembled matrices with Dirichlet rows (zero rows whose
 columns stay), for symmetric Dirichlet elimination, for 3-DOF node blocks,
 and for values that are not symmetric, which keep the full copy.
 """
@@ -15,20 +15,27 @@ import pytest
 from elmerfem_amd import _lib, workloads as W
 from elmerfem_amd.batch import Server
 from elmerfem_amd.system import System
+from conftest import launched_only
 
 pytestmark = pytest.mark.gpu
 
 FORMS = [(_lib.FP64, _lib.FAITHFUL), (_lib.FP64, _lib.FAST), (_lib.MIXED_IR, _lib.FAST)]
 
 
-def _solves_equal(s, kw, **how):
+def _solves_equal(s, kw, half, **how):
+    """half: which copies the solve on the shared-offset layout halves."""
     out = []
     vals, rhs = s.values()
+    launched_only(s)  # resident loops read the full copy
+    mixed = how.get("precision") == _lib.MIXED_IR
     for fmt in (_lib.SPMV_SELL_SHARED, _lib.SPMV_SELL):
         s.set_values(vals, rhs)  # scaling and back leaves them an ulp off
         s.spmv_set_format(fmt, 0)
         s.spmv_set_format(fmt, 1)
         out.append(s.solve(kw, **how))
+        route = s.solve_route()
+        assert route["half_storage"] & 3 == (half if fmt == _lib.SPMV_SELL_SHARED else 0)
+        assert route["loops"] == (_lib.LOOP_RECORDED if mixed else _lib.LOOP_LAUNCHED)
     (x0, r0), (x1, r1) = out
     assert r0["info"] == r1["info"] == 1 and r0["iters"] == r1["iters"]
     assert r0["res_true"] == r1["res_true"]
@@ -36,14 +43,16 @@ def _solves_equal(s, kw, **how):
     return x0
 
 
-# 45: just over the size limit and a ragged last slice; 48: a multiple of 16
-@pytest.mark.parametrize("n", [45, 48])
-@pytest.mark.parametrize("precision,mode", FORMS)
+# 45: just over the size limit and a ragged last slice; 48: a multiple of 16;
+# 64: more rows than the resident loops take, another ragged slice (not in
+# mixed precision: more than 1024 workgroups group FP32 sums otherwise there)
+@pytest.mark.parametrize("n,precision,mode", [(n, *f) for n in (45, 48, 64) for f in FORMS
+                                              if n < 64 or f[0] == _lib.FP64])
 def test_poisson_equals_sell(ehip, n, precision, mode):
     w = W.poisson_hex8(n, sigma=1.0)
     s, _ = W.build_system(w)
     assert 8 * s.spmv_shared_layout()["entries"] >= 16 << 20
-    _solves_equal(s, w["kw"], precision=precision, mode=mode)
+    _solves_equal(s, w["kw"], 3 if precision == _lib.MIXED_IR else 1, precision=precision, mode=mode)
     s.free()
 
 
@@ -52,7 +61,7 @@ def test_tet4_symmetric_dirichlet_equals_sell(ehip, precision, mode):
     w = W.heat_tet4(53)
     w["kw"].symmetric = True
     s, _ = W.build_system(w)
-    _solves_equal(s, w["kw"], precision=precision, mode=mode)
+    _solves_equal(s, w["kw"], 3 if precision == _lib.MIXED_IR else 1, precision=precision, mode=mode)
     s.free()
 
 
@@ -61,7 +70,7 @@ def test_elasticity_equals_sell(ehip, precision, mode):
     w = W.elasticity_hex(22)
     s, _ = W.build_system(w)
     assert s.spmv_shared_layout()["node_block"] == 3
-    _solves_equal(s, w["kw"], precision=precision, mode=mode, inner_tol=0.1)
+    _solves_equal(s, w["kw"], 0 if precision == _lib.MIXED_IR else 1, precision=precision, mode=mode, inner_tol=0.1)
     s.free()
 
 
@@ -79,9 +88,9 @@ def test_unsymmetric_values_keep_the_full_copy(ehip):
     changed[j] *= 1.0 + 1e-9
     assert changed[j] != vals[j]
     s.set_values(changed, rhs)
-    a = _solves_equal(s, w["kw"], mode=_lib.FAST)
+    a = _solves_equal(s, w["kw"], 0, mode=_lib.FAST)
     s.set_values(vals, rhs)
-    b = _solves_equal(s, w["kw"], mode=_lib.FAST)
+    b = _solves_equal(s, w["kw"], 1, mode=_lib.FAST)
     assert not np.array_equal(a, b) and np.allclose(a, b, rtol=1e-6, atol=1e-12)
     s.free()
 
