@@ -1022,6 +1022,11 @@ __global__ __launch_bounds__(256) void k_sym_check(int n, int nslice, SymTab tab
 // failed, compares its entries at offsets < 0 with their mirror images in
 // CRS.  flag[0] is set where k_sym_check would refuse; what this passes is
 // checked whole all the same, so the answer never depends on the sample.
+// Two unequal values that are not zero are a refusal (a zero row has none);
+// where one is zero, only the hint's rows look whether a zero row explains
+// it.  Few waves, so what counts is the chain of memory trips: kSymU entries
+// of a lane in flight, 16 us (73 with one entry at a time and zero rows
+// looked up everywhere).
 constexpr int kSymProbe = 256;
 template <typename T, int D>
 __global__ __launch_bounds__(256) void k_sym_probe(int n, int nslice, int hint, SymTab tab,
@@ -1034,28 +1039,43 @@ __global__ __launch_bounds__(256) void k_sym_probe(int n, int nslice, int hint, 
   const int r = sl * 64 + ((int)threadIdx.x & 63);
   if (sl < 0 || r >= n) return;
   auto zero_row = [&](int q) {
-    for (int j = rows[q]; j < rows[q + 1]; ++j)
-      if (j != diag[q] && in[j] != (T)0) return false;
-    return true;
+    bool some = false;
+    for (int j = rows[q]; j < rows[q + 1]; ++j) some |= j != diag[q] && !(in[j] == (T)0);
+    return !some;
   };
   const unsigned m = mask[r];
-  const int node = r / D, own = r - D * node;
-  int j = rows[r];
+  const int node = r / D, own = r - D * node, j0 = rows[r];
   bool bad = false;
-  for (int k = 0; k < tab.diag; ++k) {
-    const bool on = (m >> k) & 1u;
-    const int up = tab.K - 1 - k, q0 = D * (node + tab.col[k]);
+  for (int k0 = 0; k0 < tab.diag; k0 += kSymU) {
+    T have[kSymU][D], other[kSymU][D];
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int q = q0 + d;
-      if (q < 0) continue;
-      const unsigned mq = mask[q];
-      const T have = on ? in[j + d] : (T)0;
-      const T other = (mq >> up) & 1u ? in[rows[q] + D * __popc(mq & ((1u << up) - 1u)) + own] : (T)0;
-      // the rules of k_sym_fill and k_sym_check
-      if (!(have == other) && !(on && (zero_row(r) || zero_row(q)))) bad = true;
+    for (int u = 0; u < kSymU; ++u) {
+      const int k = min(k0 + u, tab.diag - 1), up = tab.K - 1 - k, q0 = D * (node + tab.col[k]);
+      const bool on = (m >> k) & 1u;
+      const int j = j0 + D * __popc(m & ((1u << k) - 1u));
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const int q = max(q0, 0) + d;
+        const unsigned mq = mask[q];
+        const bool there = q0 >= 0 && ((mq >> up) & 1u);
+        // clamped to the row's first entry where there is none
+        const T a = in[on ? j + d : j0], b = in[rows[q] + (there ? D * __popc(mq & ((1u << up) - 1u)) + own : 0)];
+        have[u][d] = on && q0 >= 0 ? a : (T)0;
+        other[u][d] = there ? b : (T)0;
+      }
     }
-    j += on ? D : 0;
+#pragma unroll
+    for (int u = 0; u < kSymU; ++u)
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        if (have[u][d] == other[u][d]) continue;
+        if (have[u][d] != (T)0 && other[u][d] != (T)0) {
+          bad = true;
+        } else if (w == kSymProbe) {  // the rules of k_sym_fill and k_sym_check
+          const int k = min(k0 + u, tab.diag - 1);
+          bad |= !(((m >> k) & 1u) && (zero_row(r) || zero_row(D * (node + tab.col[k]) + d)));
+        }
+      }
   }
   if (bad) flag[0] = 1;
 }

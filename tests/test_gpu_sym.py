@@ -235,10 +235,10 @@ def test_unsymmetric_values_are_told_from_a_sample(ehip, kind, precision, mode):
     inner = np.bincount(row, off, s.n) > 0  # not a Dirichlet row
     pairs = np.nonzero(off & inner[row] & inner[cols - 1])[0]
 
-    def halves(v):
+    def halves(v, info=1):
         s.set_values(v, rhs)
         _, rep = s.solve(w["kw"], return_x=False, **how)
-        assert rep["info"] == 1
+        assert rep["info"] == info
         return s.solve_route()["half_storage"]
 
     rounding = vals * (1.0 + 1e-7 * np.random.default_rng(4).random(len(vals)))
@@ -252,6 +252,15 @@ def test_unsymmetric_values_are_told_from_a_sample(ehip, kind, precision, mode):
         assert halves(one) in ((0, 4) if half else (0,))
         assert halves(one) == 0
         assert halves(vals) == half
+    # an entry without its mirror image (a zero there) shows only to the whole
+    # comparison, or in the slice where that failed
+    w["kw"].maxit = 2
+    for at in (0.25, 0.6):
+        one = vals.copy()
+        one[pairs[int(at * len(pairs))]] = 0.0
+        assert halves(one, 2) == (4 if half else 0)
+        assert halves(one, 2) == 0
+    assert halves(vals, 2) == half
     s.free()
 
 
