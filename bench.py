@@ -675,6 +675,8 @@ def main():
     # more solve samples every 4th fused SpMV launch with kernel-bound events
     steps = run("mixed_ir", _lib.MIXED_IR, _lib.FAST, args.steps, keep_x=True)
     sampled = run("mixed_ir(sampled)", _lib.MIXED_IR, _lib.FAST, 1, profile_every=4)
+    # CG on a symmetric matrix of the shared-offset layout reads half of the values
+    half = bool(sys_.solve_route()["half_storage"] & 2)
     wall = np.array([r["wall_ms"] for r in steps])
     iters = np.array([r["iters"] for r in steps])
     ms_per_step = float(wall.mean())
@@ -717,10 +719,8 @@ def main():
     # the SpMV step's epilogue: folded (the previous vector step's partials summed
     # in every workgroup, two launches per iteration) unless EHIP_CG_FOLD=0
     epi = "EpiCgFast1<float>" if os.environ.get("EHIP_CG_FOLD", "1")[:1] == "0" else "EpiCgFold<float>"
-    half = False  # CG on a symmetric matrix of this layout reads half of the values
     if c32["format"] == "sell_shared":
         lay = sys_.spmv_shared_layout()
-        half = lay["node_block"] <= 1 and 8 * lay["entries"] >= (16 << 20)
         # values streamed non-temporally only when the FP32 copy exceeds the 256 MiB Infinity Cache
         nt = "true" if 4 * lay["entries"] > (256 << 20) else "false"
         kname = "k_spmv_epi_sho<float,256,%d,%d,%s,%s>" % (lay["lane_unroll"], max(1, lay["node_block"]), nt, epi)
@@ -737,22 +737,23 @@ def main():
         kname = "k_spmv_epi<float,%d,%d,%s,%s>" % (c32["block"], c32["nnz_per_block"],
                                                   "ColsU16" if bits == 16 else "ColsI32", epi)
     us = float(np.mean([r["spmv_us"] for r in sampled if r["spmv_samples"] > 0]))
-    # algorithmic bytes of one fused FP32 CG step: FP32 values, int32 column
-    # indices, row pointers, z read, q and p read and written
-    alg32 = 8 * nnz + 4 * (n + 1) + 20 * n
-    # what this layout reads for the same work (16-bit column offsets or slice-shared
-    # offsets, no row pointers)
+    # one fused FP32 CG step on plain CSR: FP32 values, int32 column indices,
+    # row pointers, z read, q and p read and written.  No kernel here moves
+    # that much, so it says nothing about the memory
+    csr32 = 8 * nnz + 4 * (n + 1) + 20 * n
+    # what the layout in use has to move for the same work (16-bit column offsets or
+    # slice-shared offsets, no row pointers): what the roofline counts
     bytes32 = fused_cg32_bytes(nnz, n, bits, c32["format"], c32["chunks"])
     if half:  # the diagonal and one of each pair of values, a word per slice, z, q and p
         bytes32 = 4 * (lay["entries"] + n) // 2 + 8 * ((n + 63) // 64) + 20 * n
-    achieved = alg32 / (us * 1e-6) / 1e9
+    achieved = bytes32 / (us * 1e-6) / 1e9
     traffic = measured_traffic(kname)
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                 "kernel": kname + " (fused FP32 SpMV + CG update)",
-                "bytes_per_launch": alg32, "mean_us": us,
+                "bytes_per_launch": bytes32, "mean_us": us,
                 "samples": int(sum(r["spmv_samples"] for r in sampled)),
-                "layout_bytes_per_launch": bytes32, "layout_gbs": bytes32 / (us * 1e-6) / 1e9,
+                "csr_bytes_per_launch": csr32, "csr_gbs": csr32 / (us * 1e-6) / 1e9,
                 "physical_gbs": traffic / (us * 1e-6) / 1e9 if traffic else None,
                 "physical_frac": traffic / (us * 1e-6) / 1e9 / HBM_PEAK_GBS if traffic else None,
                 "traffic_source": "profiles/hbm_traffic_poisson_hex8_128.json" if traffic else None}

@@ -13,7 +13,7 @@
 // workgroups (four in BiCGStab): partial sums, and the halo's new entries with
 // the second one.  Per iteration, launched and resident: 17^3 Hex8 in HUTI's
 // order 27 and 10 us, 55^3 Tet4 (SELL-64) one-SpMV order 20 and 17 us, 301^2
-// Quad4 BiCGStab in HUTI's order 50 and 23 us.  Of the 10 us, measured by the
+// Quad4 BiCGStab in HUTI's order 52 and 25 us.  Of the 10 us, measured by the
 // kernel's own clock, some 5 are the exchanges' trips to the memory the XCDs
 // share, the rest the row sums and the reductions inside the workgroup.
 //
@@ -784,8 +784,8 @@ static int cus_of_xcd(const Device &d, int g) {
 // together, resident loops one at a time / as many as there is room for, the
 // rest launched / all launched, a round of four solves: 17^3 Hex8 in HUTI's
 // order 2.9 / 2.0 / 3.8 ms, 47^3 12.2 / 7.6 / 10.7 ms, 60^3 mixed 12.1 / 9.1 /
-// 9.3 ms, 301^2 Quad4 BiCGStab 84 / 25 / 43 ms (keeping large loops off beside
-// other solves was never better).
+// 9.3 ms, 200^2 Quad4 BiCGStab 19.5 / 11.5 / 26.8 ms (keeping large loops off
+// beside other solves was never better).
 bool resident_admit(const ehip_system *s, int g) {
   Device &d = device(s);
   std::lock_guard<std::mutex> lk(d.mu);

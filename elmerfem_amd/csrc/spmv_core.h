@@ -548,12 +548,17 @@ __device__ __forceinline__ void spmv_sho_body(int n, const int *__restrict__ off
 // value at offset +o.  A value is then read twice, by two rows o apart; o is
 // at most the bandwidth, and the workgroups of one XCD walk one contiguous
 // row range together, so the second read is mostly served by that XCD's L2
-// and the stream from the Infinity Cache or HBM halves; the loads are all
-// cached, never non-temporal.  128^3 Hex8: the fused FP32 CG step 39 -> 32 us,
-// an FP64 SpMV with its update 117 -> 90 us; 101^3 FP64 39 -> 32 us.  What
-// binds it now are the L1s' line requests to the L2 (2.35 M a launch in FP32),
-// which halving the stream does not lower: 9, 14 or 27 entries of a lane in
-// flight and 1024 to 8192 workgroups are within 15%.
+// and the stream from the Infinity Cache or HBM shrinks; the loads are all
+// cached, never non-temporal.  128^3 Hex8, kernel traces of whole solves, full
+// copy and half: the fused FP32 CG step 44.8 and 36.2 us, the FP64 SpMVs of
+// HUTI's order 101 + 110 and 81 + 102 us, of the one-SpMV order 99 and 92 us;
+// 101^3 FP64 39 + 50 and 33 + 42 us.  What binds the FP32 step is still the
+// stream between the L2s and the fabric: 210 MB at 5.8 TB/s (the full copy:
+// 278 MB at 6.2), where each value read once and the vectors would be 163 MB;
+// the rest are second reads that the L2 no longer held.  The L1s' requests
+// to the L2 did not shrink (2.47 M lines a launch, 2.26 M for a plain product
+// of the full copy).  9, 14 or 27 entries of a lane in flight are within 10%;
+// the workgroups are chosen with the launch (krylov.hip).
 // Entries are added in ascending offset order, the CRS order: FP64 adds only
 // the row's own entries (bit `lane` of pm[slice * K + k]), so its sums are
 // those of the other layouts to the bit; FP32 adds absent entries as +0.
