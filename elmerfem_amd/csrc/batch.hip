@@ -37,6 +37,7 @@
 #include <deque>
 #include <condition_variable>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <type_traits>
@@ -1083,6 +1084,7 @@ struct ehip_batch {
   int dev = 0;
   hipStream_t stream = nullptr;
   ehip_params p{};
+  std::unique_ptr<DeviceUse> use;  // while systems are in the engine
   int capacity = 0;              // slots
   int64_t chunk_cap = 0;         // work items
   // device
@@ -1516,6 +1518,7 @@ static int engine_admit(ehip_batch *b, ehip_system *s) {
   // the active counter counts this slot
   hipLaunchKernelGGL(k_inc, dim3(1), dim3(1), 0, b->stream, b->active);
   EHIP_HIP_TRY(hipGetLastError());
+  if (!b->use) b->use.reset(new DeviceUse(s->dev, true));
   return slot;
 }
 
@@ -2056,6 +2059,7 @@ extern "C" int ehip_server_step(ehip_batch *b, int *ndone, ehip_system **done_sy
     if ((rc = upload_worklist(b))) return rc;
     b->dirty = false;
   }
+  if (!live) b->use.reset();
   if (live) {
     if ((rc = engine_launch(b))) return rc;
     b->in_flight = true;

@@ -424,6 +424,16 @@ int resident_cg(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful,
 template <typename T>
 int resident_bicgstab(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool faithful, double *hist, const T *du);
 bool resident_buffers(ehip_system *s);  // false: no memory for their buffers
+// A solve, batch or server with work in progress on a device; launched: by
+// kernels of its own, which resident loops are not started beside.
+struct DeviceUse {
+  int dev;
+  bool launched;
+  DeviceUse(int device, bool launched);
+  ~DeviceUse();
+  DeviceUse(const DeviceUse &) = delete;
+  void launch();  // launched from now on
+};
 // Room on the device for a resident loop of g workgroups, held from before
 // its launch until its state is read.
 bool resident_admit(const ehip_system *s, int g);

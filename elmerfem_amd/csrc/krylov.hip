@@ -1333,6 +1333,7 @@ struct SolveCtx {
   double *hist;  // device, may be null
   int spmv;
   bool prof;     // sample the SpMV launches of this loop
+  DeviceUse *use;
 };
 
 template <typename T>
@@ -1351,8 +1352,8 @@ static Vecs<T> make_vecs(T *w, int n, int method, T *x, T *b) {
 }
 static int nvecs(int method) { return method == EHIP_CG ? 6 : 10; }
 
-// A Krylov sequence in one launch (resident.hip), until it stops; its state in
-// hst.  *resident = false: there was no room for it, or the grid gave up
+// A Krylov sequence in one launch (resident.hip), until it stops or the launch
+// has run its number of iterations (hst->done tells); its state in hst.  *resident = false: there was no room for it, or the grid gave up
 // waiting (the device is shared with something that kept part of it off the
 // chip), and the vectors and the state are as before, for the launched loop
 // to go on from.
@@ -1366,6 +1367,7 @@ static int run_resident(ehip_system *s, SolveCtx &c, const Vecs<T> &v, KStateT<T
   const int g = resident_groups(s->n, c.method == EHIP_CG);
   if (!resident_admit(s, g)) {  // others hold the chip, or use it
     *resident = false;
+    c.use->launch();
     return EHIP_OK;
   }
   int rc = (c.method == EHIP_CG ? resident_cg<T> : resident_bicgstab<T>)(s, v, st, faithful, hist, du);
@@ -1374,6 +1376,7 @@ static int run_resident(ehip_system *s, SolveCtx &c, const Vecs<T> &v, KStateT<T
   if (rc) return rc;
   *resident = hst->ticket[3] == 0;
   s->route_loops |= *resident ? EHIP_LOOP_RESIDENT : EHIP_LOOP_GAVE_UP;
+  if (!*resident) c.use->launch();
   if (*resident) c.spmv += std::max(0, hst->iter - it0) * ((faithful ? 2 : 1) + (c.method == EHIP_CG ? 0 : 1));
   return EHIP_OK;
 }
@@ -1408,8 +1411,9 @@ static int krylov(ehip_system *s, SolveCtx &c, const SpmvPlan &plan, const T *va
   if (c.method == EHIP_CG) {
     if (c.mode == EHIP_FAITHFUL) {
       EHIP_HIP_TRY(hipMemcpyAsync(v.p, v.z, sizeof(T) * n, hipMemcpyDeviceToDevice, s->stream));
-      if (resident) {
-        if ((rc = run_resident<T>(s, c, v, st, hst, true, c.hist, du, iter0, &resident))) return rc;
+      for (int it_seen = iter0; resident; it_seen = hst->iter) {
+        if ((rc = run_resident<T>(s, c, v, st, hst, true, c.hist, du, it_seen, &resident))) return rc;
+        if (hst->done) break;
       }
       for (; !resident;) {
         s->route_loops |= EHIP_LOOP_LAUNCHED;
@@ -2197,6 +2201,9 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   if (s->sym_on && s->resident_on &&
       resident_fits<double>(s, true, p->mode == EHIP_FAITHFUL && p->precision == EHIP_FP64))
     s->sym_on = false;  // that loop reads the full copy
+  const bool cg = p->method == EHIP_CG, fp64 = p->precision == EHIP_FP64;
+  DeviceUse use(s->dev, !(s->resident_on && (fp64 ? resident_fits<double>(s, cg, p->mode == EHIP_FAITHFUL)
+                                                  : resident_fits<float>(s, cg, false))));
   SolveClock clk(events, s->stream);
   EHIP_HIP_TRY(clk.create());
   ehip_report rep{};
@@ -2257,6 +2264,7 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
     dhist = s->hist;
   }
   SolveCtx c{};
+  c.use = &use;
   c.method = p->method;
   c.precond = p->precond;
   c.maxit = p->maxit;

@@ -46,6 +46,11 @@
 // LDS) fits any CU that no other one holds, so the process counts CUs: loops
 // run side by side while every XCD has a CU for each workgroup of theirs that
 // it can be given (resident_admit); one that finds no room runs launched.
+// Beside launched kernels none is started: a loop keeps the CUs, and a
+// hardware queue that streams may share, from them until it stops, where
+// launched loops take turns kernel by kernel.  For the same reason a launch
+// stops after kSlice iterations (kSliceShared when other solves are in
+// progress), so whoever comes then waits for no more than those.
 // Other kernels end by themselves, and every wait is bounded: a thread that
 // polls past kSpins (a quarter of a second or so) gives up for the whole
 // grid.  That is for what the count does not see, other processes and CU
@@ -70,6 +75,9 @@ constexpr int kResGroups = 256;   // at most, one per CU
 constexpr int kResLds = 156 * 1024;
 constexpr int kSpins = 1 << 18;
 constexpr int kCusPerXcd = 32;
+// Iterations of a launch: 2 to 12 ms, against some 40 us to go on with the
+// next, and 0.3 to 1.5 ms.
+constexpr int kSlice = 256, kSliceShared = 32;
 typedef unsigned long long Word;
 
 __device__ __forceinline__ Word ld_word(const Word *p) {
@@ -154,6 +162,7 @@ struct ResArgs {
   int n, nslice, halo;
   int ngroups;                  // 256-row groups with rows
   int spmv_grid, vec_grid;      // workgroups of the launched kernels
+  int cap;                      // iterations after which the launch stops
   const int *off, *tab;         // SHO: slice offsets and offset lists; SELL: slice offsets, slice bases
   const unsigned *mask;         // SHO
   const unsigned short *c16;    // SELL
@@ -419,7 +428,9 @@ __device__ __forceinline__ void halo_columns(int lo, int nlow, int re, int nhalo
 
 }  // namespace
 
-// One CG sequence.  FAITHFUL: HUTI's order with the true residual of every
+// One CG sequence, or `cap` iterations of it: it then stops between two, in
+// the state of the launched loop there, and the next launch goes on.
+// FAITHFUL: HUTI's order with the true residual of every
 // iteration; its product A x and the next iteration's A p are taken in one
 // pass over the matrix.  Else the one-SpMV order (FinCgFast2's tests).
 template <typename T, ResFmt F, int KW, bool FAITHFUL>
@@ -458,6 +469,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
   const int slot = group_slot((int)blockIdx.x * 4 + (tid & 3), a.ngroups);
   const bool used = tid < a.spmv_grid && slot_used(tid, a.ngroups);
   unsigned e = 1;
+  int left = a.cap;
   T sx[FAITHFUL ? 2 : 1];
   bool lost = false;
   if constexpr (FAITHFUL) {
@@ -478,7 +490,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
         EpiCgResidual<T> f{a.v, &sh.st, nullptr, 0, nullptr, hist, nullptr, 0, (T)0, a.du};
         f.finish(two);
         __syncthreads();
-        if (sh.st.done) break;
+        if (sh.st.done || --left == 0) break;
       }
       pq = tot[0];
     } else {
@@ -549,7 +561,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
       FinCgFast2<T>{&sh.st, nullptr, 0, hist}.finish(tot);
       halo_columns<T, kResRows, 1>(lo, nlow, re, nhalo, a.ez, a.ez, [&](int c, T zc, T) { win[c - wb] = zc; });
       __syncthreads();
-      if (sh.st.done) break;
+      if (sh.st.done || --left == 0) break;
       ++e;
     }
   }
@@ -567,8 +579,8 @@ __global__ __launch_bounds__(kResRows) void k_resident_cg(ResArgs<T> a) {
   }
 }
 
-// One BiCGStab sequence in huti_bicgstab.src order, four exchanges an
-// iteration.  FAITHFUL: the true residual of every iteration, its product
+// One BiCGStab sequence (or `cap` iterations) in huti_bicgstab.src order, four
+// exchanges an iteration.  FAITHFUL: the true residual of every iteration, its product
 // A x taken in one pass with the next iteration's A t1v; else FinBiXr's tests
 // on the recurrence residual.  The halo's t1v = (r + beta w) / dg needs beta,
 // so r and w = p - omega v travel with the partial sums that give it.
@@ -610,6 +622,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
   const int slot = group_slot((int)blockIdx.x + (tid & 3) * (int)gridDim.x, a.ngroups);
   const bool used = tid < a.spmv_grid && slot_used(tid, a.ngroups);
   unsigned e = 0;
+  int left = a.cap;
   bool lost = false;
   if (!sh.st.done) for (bool first = true;; first = false) {
     ++e;
@@ -641,7 +654,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
       EpiBiResidual<T> f{a.v, &sh.st, nullptr, 0, nullptr, hist, (T)0, (T)0, a.du};
       f.finish(two);
       __syncthreads();
-      if (sh.st.done) break;
+      if (sh.st.done || --left == 0) break;
     }
     const T alpha = sh.st.rho / rv[0];
     const T s = rr - alpha * v;
@@ -717,6 +730,7 @@ __global__ __launch_bounds__(kResRows) void k_resident_bi(ResArgs<T> a) {
       if constexpr (FAITHFUL) winx[own] = x;
     }
     __syncthreads();
+    if (!FAITHFUL && --left == 0) break;
   }
   if (lost) return;  // nothing is committed
   if (ok) {
@@ -764,6 +778,8 @@ __global__ void k_resident_clear(Word *w, int nw, int *gave_up, unsigned *mark, 
 struct Device {
   std::mutex mu;
   int cus = 0;     // of the device; 0: not asked yet
+  int solves = 0;  // solves, batches and servers with work in progress
+  int launched = 0;  // those of them that launch their kernels
   int held = 0;    // CUs of an XCD that resident loops may hold
   std::chrono::steady_clock::time_point rest{};  // no resident loop before
 };
@@ -780,12 +796,31 @@ static int cus_of_xcd(const Device &d, int g) {
   return (g + xcds - 1) / xcds;
 }
 
+DeviceUse::DeviceUse(int device, bool launched) : dev(device & 63), launched(launched) {
+  std::lock_guard<std::mutex> lk(g_device[dev].mu);
+  ++g_device[dev].solves;
+  g_device[dev].launched += launched;
+}
+DeviceUse::~DeviceUse() {
+  std::lock_guard<std::mutex> lk(g_device[dev].mu);
+  --g_device[dev].solves;
+  g_device[dev].launched -= launched;
+}
+void DeviceUse::launch() {
+  std::lock_guard<std::mutex> lk(g_device[dev].mu);
+  g_device[dev].launched += !launched;
+  launched = true;
+}
+
 // Room for a resident loop of g workgroups.  Four host threads that solve
-// together, resident loops one at a time / as many as there is room for, the
-// rest launched / all launched, a round of four solves: 17^3 Hex8 in HUTI's
-// order 2.9 / 2.0 / 3.8 ms, 47^3 12.2 / 7.6 / 10.7 ms, 60^3 mixed 12.1 / 9.1 /
-// 9.3 ms, 200^2 Quad4 BiCGStab 19.5 / 11.5 / 26.8 ms (keeping large loops off
-// beside other solves was never better).
+// together, resident loops one at a time / so / all launched, a round of four
+// solves: 17^3 Hex8 in HUTI's order 2.9 / 2.7 / 3.8 ms, 47^3 12.2 / 9.9 / 10.7
+// ms, 60^3 mixed 12.1 / 9.3 / 9.3 ms, 200^2 Quad4 BiCGStab 19.5 / 12.0 / 26.8 ms.
+// One thread's launched work beside another's solves, resident / so / launched:
+// an 80^3 mixed CG beside 301^2 BiCGStab 42 / 11.2 / 10.6 ms, a batch of five
+// Quad4 systems beside 500^2 BiCGStab 260 / 11.5 / 12.1 ms.  A 17^3 solve beside
+// 301^2 ones whose stream shares its hardware queue, in whole sequences / so /
+// launched: 20 / 5.4 / 4.0 ms (1.0 on another queue, 1.9 launched).
 bool resident_admit(const ehip_system *s, int g) {
   Device &d = device(s);
   std::lock_guard<std::mutex> lk(d.mu);
@@ -794,7 +829,7 @@ bool resident_admit(const ehip_system *s, int g) {
     return false;
   }
   const int xcds = std::max(1, d.cus / kCusPerXcd), need = cus_of_xcd(d, g);
-  if (d.held + need > d.cus / xcds) return false;
+  if (d.launched > 0 || d.held + need > d.cus / xcds) return false;
   if (std::chrono::steady_clock::now() < d.rest) return false;
   d.held += need;
   return true;
@@ -804,6 +839,13 @@ void resident_release(const ehip_system *s, int g, bool gave_up) {
   std::lock_guard<std::mutex> lk(d.mu);
   d.held -= cus_of_xcd(d, g);
   if (gave_up) d.rest = std::chrono::steady_clock::now() + kRest;
+}
+
+static int slice(const ehip_system *s) {
+  if (s->resident_test == 3) return 1;
+  Device &d = device(s);
+  std::lock_guard<std::mutex> lk(d.mu);
+  return d.solves > 1 ? kSliceShared : kSlice;
 }
 
 // CG: 1024 rows to a workgroup; BiCGStab: the launched vector steps' grid
@@ -880,6 +922,7 @@ static int resident_run(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool f
   a.nslice = s->nslice;
   a.ngroups = (s->nslice + 3) / 4;
   a.spmv_grid = sell_grid(s);
+  a.cap = slice(s);
   const int g = resident_groups(n, CG);
   a.vec_grid = CG ? fused_grid(n) : g;
   a.hist = hist;
@@ -940,8 +983,8 @@ int resident_bicgstab(ehip_system *s, const Vecs<T> &v, KStateT<T> *st, bool fai
 }
 
 // Tests: mode 0 as usual, 1 launched loops only, 2 every grid is told that a
-// thread of its gave up (it ends as ever and commits nothing).  Ends the
-// device's rest.
+// thread of its gave up (it ends as ever and commits nothing), 3 launches of
+// one iteration each.  Ends the device's rest.
 extern "C" int ehip_internal_resident(ehip_system *s, int mode) {
   if (!s) return EHIP_EARG;
   s->resident_test = mode;

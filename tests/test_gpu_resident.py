@@ -19,6 +19,7 @@ import numpy as np
 import pytest
 
 from elmerfem_amd import _lib, workloads as W
+from elmerfem_amd.batch import Server
 from elmerfem_amd.system import System
 
 pytestmark = pytest.mark.gpu
@@ -228,6 +229,56 @@ def test_a_grid_that_gave_up(ehip, method, precision, mode):
         assert (r["info"], r["iters"], r["outer_iters"]) == tuple(out[0][1][k] for k in ("info", "iters", "outer_iters"))
         assert np.array_equal(r["history"], out[0][1]["history"]) and np.array_equal(x, out[0][0])
     s.free()
+
+
+@pytest.mark.parametrize("precision,mode", FORMS)
+@pytest.mark.parametrize("method", ["cg", "bicgstab"])
+def test_launches_that_stop_between_iterations(ehip, method, precision, mode):
+    """A launch runs a number of iterations at most and the next goes on from
+    the state it left: with launches of one iteration each a solve gives the
+    same history and bits, whether it converges or meets its limit."""
+    w = W.poisson_hex8(14, sigma=1.0) if method == "cg" else W.convdiff_quad4(60, index=3)
+    s, _ = W.build_system(w)
+    vals, rhs = s.values()
+    for maxit in (10000, 5):
+        w["kw"].maxit = maxit
+        out = []
+        for test in (0, 3):
+            _resident(s, test)
+            s.set_values(vals, rhs)
+            out.append(s.solve(w["kw"], precision=precision, mode=mode, history=True, true_residual_stop=True))
+            assert s.solve_route()["loops"] == _lib.LOOP_RESIDENT
+        (x0, r0), (x1, r1) = out
+        for k in ("info", "iters", "outer_iters", "res_scaled", "res_true"):
+            assert r0[k] == r1[k], (k, r0[k], r1[k])
+        assert np.array_equal(r0["history"], r1["history"]) and np.array_equal(x0, x1)
+    s.free()
+
+
+def test_none_beside_launched_work(ehip):
+    """While a server holds a request, a direct solve takes turns with it launch
+    by launch, to the same bits; before and after, it runs resident."""
+    w = W.poisson_hex8(14, sigma=1.0)
+    s, _ = W.build_system(w)
+    vals, rhs = s.values()
+    t, _ = W.build_system(W.heat_tet4(9))
+    srv = Server(w["kw"], precision=_lib.MIXED_IR, max_slots=4)
+    got = []
+    for loops in (_lib.LOOP_RESIDENT, _lib.LOOP_LAUNCHED, _lib.LOOP_RESIDENT):
+        if loops == _lib.LOOP_LAUNCHED:
+            assert srv.submit(t)
+        s.set_values(vals, rhs)
+        got.append(s.solve(w["kw"], mode=_lib.FAST)[0])
+        assert s.solve_route()["loops"] == loops
+        if loops == _lib.LOOP_LAUNCHED:
+            done = []
+            while not done:
+                done = srv.step()
+            assert done[0][1]["info"] == 1
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    srv.free()
+    s.free()
+    t.free()
 
 
 def test_several_threads(ehip):
