@@ -1353,19 +1353,18 @@ static Vecs<T> make_vecs(T *w, int n, int method, T *x, T *b) {
 static int nvecs(int method) { return method == EHIP_CG ? 6 : 10; }
 
 // A Krylov sequence in one launch (resident.hip), until it stops or the launch
-// has run its number of iterations (hst->done tells); its state in hst.  *resident = false: there was no room for it, or the grid gave up
-// waiting (the device is shared with something that kept part of it off the
-// chip), and the vectors and the state are as before, for the launched loop
-// to go on from.
+// has run its number of iterations (hst->done tells); its state in hst.
+// *resident = false: there was no room for it, or the grid gave up waiting
+// (the device is shared with something that kept part of it off the chip),
+// and the vectors and the state are as before, for the launched loop to go
+// on from.
 template <typename T>
 static int run_resident(ehip_system *s, SolveCtx &c, const Vecs<T> &v, KStateT<T> *st, KStateT<T> *hst, bool faithful,
                         double *hist, const T *du, int it0, bool *resident) {
-  if (!resident_buffers(s)) {  // no memory for them: the launched loop needs none
-    *resident = false;
-    return EHIP_OK;
-  }
   const int g = resident_groups(s->n, c.method == EHIP_CG);
-  if (!resident_admit(s, g)) {  // others hold the chip, or use it
+  // no memory for the buffers, which the launched loop does without; or others
+  // hold the chip, or use it
+  if (!resident_buffers(s) || !resident_admit(s, g)) {
     *resident = false;
     c.use->launch();
     return EHIP_OK;
