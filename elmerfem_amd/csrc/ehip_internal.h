@@ -178,10 +178,10 @@ struct ehip_system {
   float *sho32 = nullptr;
   uint64_t sho64_ver = 0, sho32_ver = 0;
   // half storage for symmetric values of such a pattern (CG solves of
-  // systems over kSymMinBytes): the offsets, every row's present entries as
+  // systems that sym_pays names): the offsets, every row's present entries as
   // a 32-bit mask, and the same as one 64-bit lane mask per (slice, entry)
   bool sym_ok = false;
-  bool sym_on = false;                // the solve in progress may use it
+  int sym_on = 0;                     // precisions (sym_pays) that the solve in progress may use it in
   ehip::SymTab sym_tab{};
   int64_t sym_len = 0;                // values of a copy, padding included
   unsigned *sym_mask = nullptr;       // n
@@ -350,10 +350,36 @@ inline int sho_nt_from(int nslice, int64_t bytes, int64_t n, int elem) {
   return (int)((double)nslice * (double)c / (double)bytes);
 }
 
-// Smallest FP64 values copy (bytes) that takes the half storage: below it
-// the copy fits the L2s (8 x 4 MB with the vectors), so halving its stream
-// gains nothing, and the system is small enough for the resident loops.
-constexpr int64_t kSymMinBytes = 16ll << 20;
+// Smallest full values copy (bytes) of a precision in place of which CG reads
+// the half storage.  It halves the stream from the memory, so it pays where
+// that binds: once copy and vectors outgrow the 256 MB Infinity Cache, while
+// below that its second reads and the check at every refresh cost more than
+// they save.  Whole solves, full / half (ms): FP64 in HUTI's order Hex8 65^3
+// (61 MB) 9.05 / 9.40, 80^3 (114 MB) 15.9 / 16.1, 92^3 (172 MB) 24.1 / 23.8,
+// 101^3 (227 MB) 35.5 / 30.7; Tet4 80^3 (63 MB) 21.5 / 22.5, 110^3 (163 MB) 53.3
+// / 53.1.  Mixed, by the FP32 copy: Tet4 70^3 (21 MB) 7.87 / 8.14, Hex8 72^3 (42
+// MB) 6.44 / 6.51, 80^3 (57 MB) 8.45 / 8.31, 128^3 (230 MB) 30.8 / 27.1.  FP64
+// elasticity Hex8 22^3 (23 MB) 7.0 / 8.3, 40^3 (131 MB) 31.4 / 33.4, 46^3 (197 MB)
+// 44.5 / 45.2, 50^3 (253 MB) 63.2 / 60.2.
+// EHIP_HALF_MIN_MB=m (read when a system is created and at every solve) sets
+// it to m MB for all.
+inline int64_t sym_min_bytes(int elem, int node_block) {
+  const char *v = std::getenv("EHIP_HALF_MIN_MB");
+  if (v && *v) return (int64_t)std::atoll(v) << 20;
+  if (node_block > 1) return 224ll << 20;
+  return (elem == 8 ? 150ll : 48ll) << 20;
+}
+// precisions (1 FP64 + 2 FP32) in which the pattern's copies are large enough;
+// of 3-DOF node blocks only FP64: an entry below the diagonal takes its three
+// values from three places there, and FP32 lost by that more than the halved
+// stream gave (63^3 Hex8: 37 us full, 42 us half; FP64 112, 84)
+inline int sym_pays(const ehip_system *s) {
+  const int64_t nz = s->sho_nnz;
+  if (!s->sho_ok || s->sho_d == 2) return 0;
+  const bool b64 = 8 * nz >= sym_min_bytes(8, s->sho_d);
+  const bool b32 = s->sho_d == 1 && 4 * nz >= sym_min_bytes(4, s->sho_d);
+  return (b64 ? 1 : 0) + (b32 ? 2 : 0);
+}
 
 inline int sell_grid(const ehip_system *s) {
   int g = (s->nslice + 3) / 4;

@@ -1224,7 +1224,7 @@ static int epi_grid(const ehip_system *s, const SpmvPlan &p) {
   const int fmt = active_fmt<T>(s);
   if (!fmt) return p.grid;
   if constexpr (sizeof(T) == 4)
-    return epi_sell_grid<T>(s, fmt == 2 && s->sym_on && s->sym32.good && s->sym32.ver == s->vals32_ver);
+    return epi_sell_grid<T>(s, fmt == 2 && (s->sym_on & 2) && s->sym32.good && s->sym32.ver == s->vals32_ver);
   return epi_sell_grid<T>(s);
 }
 
@@ -2179,27 +2179,30 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
   const int n = s->n;
   int rc;
   if ((rc = ensure_state(s))) return rc;
-  // half storage only where the method needs a symmetric matrix anyway, and
-  // of 3-DOF node blocks only in FP64: an entry below the diagonal takes its
-  // three values from three places there, and FP32 lost by that more than
-  // the halved stream gave (63^3 Hex8: 37 us full, 42 us half; FP64 112, 84)
   s->route_loops = s->route_half = s->route_grid32 = 0;
   struct Leave {  // other callers of the SpMVs here (the engine's reports) have full copies
     ehip_system *s;
-    ~Leave() { s->sym_on = s->resident_on = false; }
+    ~Leave() {
+      s->sym_on = 0;
+      s->resident_on = false;
+    }
   } leave{s};
-  s->sym_on = p->method == EHIP_CG && p->precond < EHIP_PRECOND_ILU0 &&
-              (s->sho_d == 1 || p->precision == EHIP_FP64);
+  // half storage only where the method needs a symmetric matrix anyway; the
+  // mixed form of 3-DOF node blocks reads no halved FP32 copy, and its FP64
+  // products are too few for the check
+  s->sym_on = 0;
+  if (p->method == EHIP_CG && p->precond < EHIP_PRECOND_ILU0)
+    s->sym_on = p->precision == EHIP_FP64 ? sym_pays(s) & 1 : (s->sho_d == 1 ? sym_pays(s) : 0);
   // on a lane, of systems the resident loops would take elsewhere: their
   // copies fit the caches, and the check's wait costs more than it gives
-  if (tl_shared_device && s->n <= 262144) s->sym_on = false;
+  if (tl_shared_device && s->n <= 262144) s->sym_on = 0;
   // one launch per sequence where the rows fit the chip (not for callers
   // without runtime objects of their own, nor when launches are sampled)
   s->resident_on = events && !tl_shared_device && p->profile_every <= 0 && p->precond < EHIP_PRECOND_ILU0 &&
                    s->resident_test != 1;
   if (s->sym_on && s->resident_on &&
       resident_fits<double>(s, true, p->mode == EHIP_FAITHFUL && p->precision == EHIP_FP64))
-    s->sym_on = false;  // that loop reads the full copy
+    s->sym_on = 0;  // that loop reads the full copy
   const bool cg = p->method == EHIP_CG, fp64 = p->precision == EHIP_FP64;
   DeviceUse use(s->dev, !(s->resident_on && (fp64 ? resident_fits<double>(s, cg, p->mode == EHIP_FAITHFUL)
                                                   : resident_fits<float>(s, cg, false))));
@@ -2320,7 +2323,7 @@ int solve_impl(ehip_system *s, const ehip_params *p, double *x, ehip_report *r, 
     if ((rc = backscale_system(s, s->rhs, s->x, bscale))) return rc;
   // unscaled FP64 true residual ||b - A x|| / ||b|| and ComputeNorm
   {
-    if (!(s->route_half & 1)) s->sym_on = false;  // not symmetric when scaled: not asked again
+    if (!(s->route_half & 1)) s->sym_on = 0;  // not symmetric when scaled: not asked again
     double *out = reinterpret_cast<double *>(&s->st->ts);
     EpiResid er{b0, s->partials, kEpiStride, &s->st->ticket[0], out};
     launch_epi_fin<double>(s, s->plan64, s->vals, s->x, er, (const KState *)nullptr);

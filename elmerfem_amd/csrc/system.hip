@@ -414,7 +414,7 @@ __global__ __launch_bounds__(256) void k_sym_masks(int n, int nslice, int D, Sym
 // the offsets of all slices together are one symmetric list of at most 31.
 static int build_sym(ehip_system *s, const std::vector<int> &ctab) {
   const int D = s->sho_d, n = s->n;
-  if (D == 2 || 8 * s->sho_nnz < kSymMinBytes) return EHIP_OK;
+  if (!sym_pays(s)) return EHIP_OK;
   int list[kSymMax + 1], K = 0;
   for (int v : ctab) {
     int *e = std::lower_bound(list, list + K, v);
@@ -858,12 +858,15 @@ static void sho_gather(ehip_system *s, const T *in, T *out) {
                        s->sho_mask, s->sho_off, in, out);
 }
 
+static int sym_bit(double) { return 1; }
+static int sym_bit(float) { return 2; }
+
 // A full copy's memory; a half copy that the solve in progress does not read
 // gives way to it.
 static int alloc_full(ehip_system *s, void **p, size_t bytes) {
   int rc = dmalloc(s, p, bytes);
   auto release = [&](auto &c) {
-    if (!c.v || (s->sym_on && c.good)) return;
+    if (!c.v || ((s->sym_on & sym_bit(*c.v)) && c.good)) return;
     dfree(s, c.v, sizeof(*c.v) * (size_t)s->sym_len);
     c.v = nullptr;
     c.good = false;
@@ -1082,7 +1085,7 @@ __global__ __launch_bounds__(256) void k_sym_probe(int n, int nslice, int hint, 
 
 template <typename T>
 static const T *sym_values(ehip_system *s, SymCopy<T> &c, const T *in, uint64_t ver) {
-  if (!s->sym_ok || !s->sym_on) return nullptr;
+  if (!s->sym_ok || !(s->sym_on & sym_bit(T()))) return nullptr;
   auto failed = [](hipError_t e) {  // reported when the solve takes it
     if (e != hipSuccess && tl_launch_err == hipSuccess) tl_launch_err = e;
     return e != hipSuccess;

@@ -1,7 +1,7 @@
 """Half storage of symmetric stencil matrices in CG solves.
 
-A launched CG solve of a system over 16 MB of FP64 values on a slice-shared-
-offset pattern reads only the values at offsets >= 0.  Row sums keep the CRS
+A launched CG solve of a large system on a slice-shared-offset pattern reads
+only the values at offsets >= 0.  Row sums keep the CRS
 order and the launches (of FP32 steps up to 1024 workgroups) their grid, so
 whole solves give the bits of the SELL-64 layout: for assembled matrices with Dirichlet rows (zero rows whose
 columns stay), for symmetric Dirichlet elimination, for 3-DOF node blocks,
@@ -18,6 +18,14 @@ from elmerfem_amd.system import System
 from conftest import launched_only
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _from_8_mb(monkeypatch):
+    """By default the half storage takes the place of large copies only, which
+    these tests need not have."""
+    monkeypatch.setenv("EHIP_HALF_MIN_MB", "8")
+
 
 FORMS = [(_lib.FP64, _lib.FAITHFUL), (_lib.FP64, _lib.FAST), (_lib.MIXED_IR, _lib.FAST)]
 
@@ -43,7 +51,7 @@ def _solves_equal(s, kw, half, **how):
     return x0
 
 
-# 45: just over the size limit and a ragged last slice; 48: a multiple of 16;
+# 45: a ragged last slice; 48: a multiple of 16;
 # 64: more rows than the resident loops take, another ragged slice (not in
 # mixed precision: more than 1024 workgroups group FP32 sums otherwise there)
 @pytest.mark.parametrize("n,precision,mode", [(n, *f) for n in (45, 48, 64) for f in FORMS
@@ -51,7 +59,6 @@ def _solves_equal(s, kw, half, **how):
 def test_poisson_equals_sell(ehip, n, precision, mode):
     w = W.poisson_hex8(n, sigma=1.0)
     s, _ = W.build_system(w)
-    assert 8 * s.spmv_shared_layout()["entries"] >= 16 << 20
     _solves_equal(s, w["kw"], 3 if precision == _lib.MIXED_IR else 1, precision=precision, mode=mode)
     s.free()
 
@@ -340,3 +347,19 @@ def test_half_storage_ends_with_the_solve(ehip):
         held.append(s.device_bytes())
         s.free()
     assert held[0] == held[1]
+
+
+@pytest.mark.parametrize("kind,n,half64,half_mixed", [("hex8", 64, 0, 0), ("hex8", 80, 0, 2), ("hex8", 92, 1, 3),
+                                                      ("elastic", 40, 0, 0), ("elastic", 50, 1, 0)])
+def test_sizes_that_take_the_half_storage(ehip, monkeypatch, kind, n, half64, half_mixed):
+    """FP64 copies from 150 MB on (224 MB with node blocks), FP32 copies from
+    48 MB on: 64^3 Hex8 has 59 and 30 MB, 80^3 114 and 57, 92^3 172 and 86;
+    40^3 elasticity 131 MB in FP64, 50^3 253."""
+    monkeypatch.delenv("EHIP_HALF_MIN_MB")
+    w = W.poisson_hex8(n) if kind == "hex8" else W.elasticity_hex(n)
+    w["kw"].maxit = 2
+    s, _ = W.build_system(w)
+    for precision, half in ((_lib.FP64, half64), (_lib.MIXED_IR, half_mixed)):
+        s.solve(w["kw"], precision=precision, mode=_lib.FAST, return_x=False)
+        assert s.solve_route()["half_storage"] == half
+    s.free()
